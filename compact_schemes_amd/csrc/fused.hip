@@ -14,16 +14,16 @@
 // and every S2 sweep applies the non-reflective characteristic update of its
 // two faces from the boundary values of its own solve (the reference's drva).
 //
-// Line solve: chunked LU recurrences as in line_solver.hip, chunks balanced
-// (lengths differ by at most one, every chunk >= 4 rows).  Kernel variants,
-// chosen per axis (cs_solver_tune):
+// Line solve: chunked LU recurrences as in line_solver.hip; lines of any
+// length from 16 to 512 rows, chunks of K rows or one less (chunk_start).
+// Kernel variants, chosen per axis (cs_solver_tune):
 //   direct: a thread evaluates the pointwise inputs of its own chunk rows and
-//     gets the two halo rows on each side from the neighbouring chunks (wave
-//     shuffles for x lines, LDS for y/z lines); carries by wave scans (x) or
-//     LDS folds (y/z).  Needs equal chunks (N = P*K); other lengths run the
-//   ragged kernel, where every chunk also evaluates its halo rows;
+//     gets the halo and seam rows from the other chunks through LDS; carries
+//     by wave scans (x lines, xt_kernel) or LDS folds (y/z lines,
+//     direct_kernel);
 //   tile: the inputs of TL lines pass through an LDS tile one row block at a
-//     time with coalesced loads (x lines load along the line).
+//     time with coalesced loads (x lines load along the line); also what the
+//     shortest uneven lines run, whose chunks are more than one row short.
 // Pointwise arithmetic (primitives, fluxes, closure and seam rows, stress,
 // characteristic BCs, stage update) is not contracted, so it rounds as the
 // CPU oracle does; the recurrences of the solve use FMA.
@@ -132,19 +132,19 @@ int dt_fold_pos(const cs_solver* sv) {
     if (sv->curv) {
         // the closing x sweep on the transposing kernel (8-point chunks)
         const AxisDesc& r = sv->rax[kS1Axes[1][2]];
-        return r.variant != 1 && r.K == 8 && r.N == r.P * 8 ? 2 : -1;
+        return r.variant != 1 && chunks_fit(r.N, r.P, r.K) ? 2 : -1;
     }
     // the first (y) sweep on the direct kernel with whole waves
     const AxisDesc& r = sv->rax[kS1Axes[1][0]];
     const int TL = r.tl == 8 ? 8 : 16;
-    return r.variant != 1 && r.N == r.P * r.K && (TL * r.P) % 64 == 0 ? 0 : -1;
+    return r.variant != 1 && chunks_fit(r.N, r.P, r.K) && (TL * r.P) % 64 == 0 ? 0 : -1;
 }
 
 // workgroups of the sweep at position pos (0: the direct y/z kernel, 2: the
 // transposing x kernel), one pair of maxima each
 static int fold_blocks(const cs_solver* sv, int pos) {
     const AxisDesc& r = sv->rax[kS1Axes[sv->order][pos]];
-    const int lines = pos == 2 ? 64 / r.GS : (r.tl == 8 ? 8 : 16);
+    const int lines = pos == 2 ? 64 / r.P : (r.tl == 8 ? 8 : 16);
     return (int)((r.nlines + lines - 1) / lines);
 }
 
@@ -185,8 +185,8 @@ int one_sweep(cs_solver* sv, int which, const double* q, const double* sbcc, dou
     if (which < 0 || which > 10) return fail(CS_ERR_ARG, "sweep index out of 0..10");
     if (which >= 7) {
         for (int a = 0; a < 3; a++)
-            if ((which == 7 || which - 8 == a) && !filter_axis_fused(sv, a))
-                return fail(CS_ERR_UNSUPPORTED, "the filter of this axis has no fused sweep");
+            if ((which == 7 || which - 8 == a) && !filter_axis_tunable(sv, a))
+                return fail(CS_ERR_UNSUPPORTED, "this axis does not split into equal chunks");
         if (out != q) CS_HIP(hipMemcpyAsync(out, q, sizeof(double) * 5 * sv->g.lmx, hipMemcpyDeviceToDevice, s));
         return filter_sweeps(sv, out, s, which == 7 ? -1 : which - 8);
     }
@@ -203,6 +203,10 @@ bool filter_fusable(const cs_solver* sv) {
 }
 
 bool filter_axis_fused(const cs_solver* sv, int a) { return sv->fax[a].ftab != nullptr; }
+
+bool filter_axis_tunable(const cs_solver* sv, int a) {
+    return filter_axis_fused(sv, a) && sv->ax[a].N == sv->ax[a].P * sv->ax[a].K;
+}
 
 template <int AX>
 static int filter_axis(cs_solver* sv, double* q, const SweepCommon& cm, hipStream_t s) {

@@ -11,11 +11,21 @@ namespace fused {
 constexpr int kYLines = 16;   // lines per workgroup of a y/z sweep
 constexpr int kMaxP = 32;     // chunks per line
 
-// one axis: derivative operator with balanced chunks
+// First row of chunk c (N for c = P) of a line of N rows in P = ceil(N/K)
+// chunks: K rows a chunk, K-1 in the D = P*K - N chunks after the first; lines
+// too short for that (chunks_fit) are balanced, at least 4 rows a chunk.
+__host__ __device__ inline bool chunks_fit(int N, int P, int K) { return P * K - N <= (P > 2 ? P - 2 : 0); }
+__host__ __device__ inline int chunk_start(int N, int P, int K, int c) {
+    if (!chunks_fit(N, P, K)) return (int)(((long)c * N) / P);
+    const int D = P * K - N, d = c < 1 ? 0 : c - 1;
+    return c * K - (d < D ? d : D);
+}
+
+// one axis: derivative and filter operators on one chunk length
 struct AxisDesc {
-    const double* tab;   // [5][N]: nu, mu, rho, Mf, Rb
-    const double* ftab;  // filter operator (build_line_table layout, 8-point chunks), or null
-    int N, P, K, GS;     // GS: lanes per line in the x layout (pow2 >= P)
+    const double* tab;   // derivative operator, chunk_table layout: [5][P*K] nu, mu, rho, Mf, Rb, ...
+    const double* ftab;  // filter operator in the same layout, or null
+    int N, P, K;
     long nlines;
     long st;
     int seam;            // both faces seam (periodic wrap on one subdomain)
@@ -121,11 +131,13 @@ int time_step(cs_solver* sv, const double* q, double dt_fixed, hipStream_t s);
 // transposing kernel, per-point metrics), -1 = none (a pass of its own)
 int dt_fold_pos(const cs_solver* sv);
 int one_sweep(cs_solver* sv, int which, const double* q, const double* sbcc, double* out, hipStream_t s);
-int build_axis_table(int n, int seam, int K, int P, std::vector<double>& h);
+void chunk_table(const std::vector<double>& h, int n, int K, int P, std::vector<double>& out);
 // every axis filters with the 8-point fused sweep of ax (the adjoint's assumption)
 bool filter_fusable(const cs_solver* sv);
 // the filter along axis a runs a fused sweep (fax), else the line solver
 bool filter_axis_fused(const cs_solver* sv, int a);
+// that sweep runs equal chunks and takes the shapes of cs_solver_tune_filter
+bool filter_axis_tunable(const cs_solver* sv, int a);
 int filter_sweeps(cs_solver* sv, double* q, hipStream_t s, int axis = -1);
 int step_filter(cs_solver* sv, double* qa, hipStream_t s);
 // adjoint (vjp.hip: per-operator products; tape.hip: fused transposed sweeps)

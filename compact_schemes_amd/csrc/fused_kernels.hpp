@@ -13,14 +13,40 @@ namespace fused {
 
 // loads and stores of a field of storage type TS at the byte offset of the
 // point in an FP64 field (an FP32 field holds the same points at half the offset)
-__device__ __forceinline__ double ldv(const double* p, uoff bo) { return ldg(p, bo); }
-__device__ __forceinline__ double ldv(const float* p, uoff bo) {
-    return (double)*reinterpret_cast<const float*>(reinterpret_cast<const char*>(p) + (bo >> 1));
+template <bool NT>
+__device__ __forceinline__ double ldr(const double* p, uoff bo) { return ldg<NT>(p, bo); }
+template <bool NT>
+__device__ __forceinline__ float ldr(const float* p, uoff bo) {
+    const float* a = reinterpret_cast<const float*>(reinterpret_cast<const char*>(p) + (bo >> 1));
+    if constexpr (NT) return __builtin_nontemporal_load(a);
+    else return *a;
 }
-__device__ __forceinline__ void stv(double* p, uoff bo, double v) { stg(p, bo, v); }
+template <bool NT>
+__device__ __forceinline__ void stv(double* p, uoff bo, double v) { stg<NT>(p, bo, v); }
+template <bool NT>
 __device__ __forceinline__ void stv(float* p, uoff bo, double v) {
-    *reinterpret_cast<float*>(reinterpret_cast<char*>(p) + (bo >> 1)) = (float)v;
+    float* a = reinterpret_cast<float*>(reinterpret_cast<char*>(p) + (bo >> 1));
+    if constexpr (NT) __builtin_nontemporal_store((float)v, a);
+    else *a = (float)v;
 }
+
+// a sweep's values at one point
+template <bool NT, class SW>
+__device__ __forceinline__ void point(const SW& sw, uoff bo, double* v) {
+    typename SW::Raw w;
+    sw.template load<NT>(bo, w);
+    sw.eval(w, v);
+}
+
+template <bool NT, class SW>
+__device__ __forceinline__ void add_out(const SW& sw, uoff bo, double* d) {
+    if constexpr (SW::kAdds) {
+        typename SW::Out e;
+        sw.template load_out<NT>(bo, e);
+        sw.add_out(e, d);
+    }
+}
+
 
 
 // ---------------------------------------------------------------------------
@@ -35,7 +61,9 @@ struct S1T {
     static constexpr bool kCurv = CURV;    // per-point metrics (curvilinear solvers)
     static constexpr int NF = 4;
     static constexpr bool kGcbc = false;   // gradients only; BC updates act on the flux sweeps
-    static constexpr bool kPv = false;     // kernels without an LDS stash re-derive u, v, w from q at the store
+    static constexpr bool kBlocks = false;
+    // bytes per point the sweep passes over (streaming rule of the launch)
+    static constexpr int kBytes = 40 + (int)sizeof(TS) * (CLOSE ? 17 : 4) + (CURV && CLOSE ? 80 : 0);
     // the transposing x kernel keeps u, v, w of its points in LDS for the
     // closure (store_pv) instead of reading q again
     static constexpr int kStash = CLOSE ? 3 : 0;
@@ -58,55 +86,65 @@ struct S1T {
     Metric mt;                // CURV: the point's metric rows and Jacobian
     double* dtpart;           // kDt: the workgroup's two time-step maxima [2*blockIdx.x]
 
-    __device__ __forceinline__ void point(uoff bo, double* v) const {
-        double qq[5];
-        Prim p = prim_at(q, bo, qq);
+    // a point's inputs, and its values from them (two steps, so that a kernel
+    // can have the loads of several points in flight)
+    struct Raw { double q[5]; };
+    template <bool NT>
+    __device__ __forceinline__ void load(uoff bo, Raw& w) const {
+#pragma unroll
+        for (int v = 0; v < 5; v++) w.q[v] = ldg<NT>(q[v], bo);
+    }
+    __device__ __forceinline__ void eval(const Raw& w, double* v) const {
+        const Prim p = primitive(w.q);
         v[0] = p.u;
         v[1] = p.v;
         v[2] = p.w;
         v[3] = p.c2;
     }
-    // point() and the largest 1/rho so far (kDt)
-    __device__ __forceinline__ void point_dt(uoff bo, double* v, double& rhoi_max) const {
-        double qq[5];
-        Prim p = prim_at(q, bo, qq);
+    // eval() and the largest 1/rho so far (kDt)
+    __device__ __forceinline__ void eval_dt(const Raw& w, double* v, double& rhoi_max) const {
+        const Prim p = primitive(w.q);
         v[0] = p.u;
         v[1] = p.v;
         v[2] = p.w;
         v[3] = p.c2;
         rhoi_max = fmax(rhoi_max, p.rhoi);
     }
-    __device__ __forceinline__ void fetch(uoff, double*) const {}
-    __device__ __forceinline__ void store(uoff bo, const double* d, const double* pv) const {
+    static constexpr bool kAdds = false;
+    template <bool NT>
+    __device__ __forceinline__ void store(uoff bo, const double* d) const {
         if constexpr (!CLOSE) {
 #pragma unroll
-            for (int f = 0; f < 4; f++) stv(gout[f], bo, d[f]);
+            for (int f = 0; f < 4; f++) stv<NT>(gout[f], bo, d[f]);
         } else {
             double qq[5];
             const Prim p = prim_at(q, bo, qq);      // q of this point: just read by this sweep
             const double uvw[3] = {p.u, p.v, p.w};
-            close(bo, d, uvw);
+            close<NT>(bo, d, uvw);
         }
     }
     // the store of the closing sweep with u, v, w of the point supplied
+    template <bool NT>
     __device__ __forceinline__ void store_pv(uoff bo, const double* d, const double* uvw) const {
-        if constexpr (CLOSE) close(bo, d, uvw);
-        else store(bo, d, nullptr);
+        if constexpr (CLOSE) close<NT>(bo, d, uvw);
+        else store<NT>(bo, d);
     }
     // the same, updating the time step's maxima mm[0..1] at the point (kDt, CURV)
+    template <bool NT>
     __device__ __forceinline__ void store_pv_dt(uoff bo, const double* d, const double* uvw, double* mm) const {
-        close_dt<true>(bo, d, uvw, mm);
+        close_dt<NT, true>(bo, d, uvw, mm);
     }
+    template <bool NT>
     __device__ __forceinline__ void close(uoff bo, const double* d, const double* uvw) const {
-        close_dt<false>(bo, d, uvw, nullptr);
+        close_dt<NT, false>(bo, d, uvw, nullptr);
     }
-    template <bool WITH_DT>
+    template <bool NT, bool WITH_DT>
     __device__ __forceinline__ void close_dt(uoff bo, const double* d, const double* uvw, double* mm) const {
         double gr[3][4];
 #pragma unroll
         for (int a = 0; a < 3; a++)
 #pragma unroll
-            for (int f = 0; f < 4; f++) gr[a][f] = (a == AX) ? d[f] : ldv(gin[a][f], bo);
+            for (int f = 0; f < 4; f++) gr[a][f] = (a == AX) ? d[f] : (double)ldr<NT>(gin[a][f], bo);
         // chain rule of calc_viscous_shear_stress_post_compute_kernel
         // (src/cuda/kernels/physics.hpp:267-281): d/dx_k = sum_a m_a[k] d/dxi_a
         double g[9], c2g[3], J = ph.J;
@@ -115,14 +153,14 @@ struct S1T {
 #pragma unroll
             for (int a = 0; a < 3; a++)
 #pragma unroll
-                for (int k = 0; k < 3; k++) M[a][k] = ldg(mt.m[a][k], bo);
+                for (int k = 0; k < 3; k++) M[a][k] = ldg<NT>(mt.m[a][k], bo);
 #pragma unroll
             for (int f = 0; f < 3; f++)
 #pragma unroll
                 for (int k = 0; k < 3; k++) g[3 * f + k] = M[0][k] * gr[0][f] + M[1][k] * gr[1][f] + M[2][k] * gr[2][f];
 #pragma unroll
             for (int k = 0; k < 3; k++) c2g[k] = M[0][k] * gr[0][3] + M[1][k] * gr[1][3] + M[2][k] * gr[2][3];
-            J = ldg(mt.J, bo);
+            J = ldg<NT>(mt.J, bo);
         } else {
             // diagonal metrics: m_a[k] = m[a] for k = a
 #pragma unroll
@@ -135,16 +173,15 @@ struct S1T {
         double t6[6], h3[3], d4;
         viscous_closure(ph.mu, J, g, c2g, uvw, t6, h3, &d4);
 #pragma unroll
-        for (int k = 0; k < 6; k++) stv(tau[k], bo, t6[k]);
+        for (int k = 0; k < 6; k++) stv<NT>(tau[k], bo, t6[k]);
 #pragma unroll
-        for (int k = 0; k < 3; k++) stv(hf[k], bo, h3[k]);
+        for (int k = 0; k < 3; k++) stv<NT>(hf[k], bo, h3[k]);
         if constexpr (WITH_DT && CURV) {
             // the point's q again (this sweep read it for the gradients)
             double qq[5];
             dt_curv_point(M, J, ph, prim_at(q, bo, qq), mm[0], mm[1]);
         }
     }
-    __device__ __forceinline__ void gcbc(uoff, int, const double*, double*) const {}
 };
 
 // the gradient sweeps with FP64 intermediates, and with FP32 ones
@@ -178,7 +215,9 @@ struct S2T {
     static constexpr bool kCurv = CURV;    // per-point metrics (curvilinear solvers)
     static constexpr int NF = 5;
     static constexpr bool kGcbc = true;
-    static constexpr bool kPv = false;
+    static constexpr bool kBlocks = CURV;
+    static constexpr int kBytes = 80 + (VISC ? (int)sizeof(TS) * (CURV ? 9 : 4) : 0) + (CURV ? 24 : 0) +
+                                  (MODE == 2 ? 40 : MODE == 3 ? 80 : 0);
     static constexpr int kStash = 0;
     static constexpr int kH = 2;
     static constexpr int kWpe = 3;
@@ -200,100 +239,154 @@ struct S2T {
     int lxi;
     long plane;
 
+    // the inputs of the flux at a point: the state; with VISC the stress row
+    // and heat flux component of the sweep (CURV: all of them), the point's
+    // metric row.  The sweep with the stage update keeps q in the caches: in
+    // the first stage its q0 is the same array.
+    struct Raw {
+        double q[5];
+        TS t[VISC ? (CURV ? 9 : 4) : 1];
+        double m[CURV ? 3 : 1];
+    };
+    template <bool NT>
+    __device__ __forceinline__ void load(uoff bo, Raw& w) const {
+#pragma unroll
+        for (int v = 0; v < 5; v++) w.q[v] = ldg<NT && MODE != 3>(q[v], bo);
+        if constexpr (CURV) {
+#pragma unroll
+            for (int k = 0; k < 3; k++) w.m[k] = ldg<NT>(mt.m[AX][k], bo);
+        }
+        if constexpr (VISC && CURV) {
+#pragma unroll
+            for (int k = 0; k < 6; k++) w.t[k] = ldr<NT>(tau6[k], bo);
+#pragma unroll
+            for (int k = 0; k < 3; k++) w.t[6 + k] = ldr<NT>(h3[k], bo);
+        } else if constexpr (VISC) {
+#pragma unroll
+            for (int k = 0; k < 3; k++) w.t[k] = ldr<NT>(tr[k], bo);
+            w.t[3] = ldr<NT>(hx, bo);
+        }
+    }
     // the AX row of calc_fluxes_pre_compute_kernel with metric row m*e_AX
     // (src/cuda/kernels/physics.hpp:98-191); zero metric terms dropped
-    __device__ __forceinline__ void point(uoff bo, double* F) const {
-        double qq[5];
-        Prim p = prim_at(q, bo, qq);
+    __device__ __forceinline__ void eval(const Raw& w, double* F) const {
+        const double* qq = w.q;
+        const Prim p = primitive(qq);
         if constexpr (CURV) {
             // the AX row with the point's metric row (m0, m1, m2)
-            const double m0 = ldg(mt.m[AX][0], bo), m1 = ldg(mt.m[AX][1], bo), m2 = ldg(mt.m[AX][2], bo);
+            const double m0 = w.m[0], m1 = w.m[1], m2 = w.m[2];
             const double ss = m0 * (p.u + ph.umf.x) + m1 * (p.v + ph.umf.y) + m2 * (p.w + ph.umf.z);
             F[0] = qq[0] * ss;
             F[1] = qq[1] * ss + m0 * p.p;
             F[2] = qq[2] * ss + m1 * p.p;
             F[3] = qq[3] * ss + m2 * p.p;
             F[4] = (qq[4] + p.p) * ss - p.p * (ph.umf.x * m0 + ph.umf.y * m1 + ph.umf.z * m2);
-            if (VISC) {
-                const double txx = ldv(tau6[0], bo), tyy = ldv(tau6[1], bo), tzz = ldv(tau6[2], bo);
-                const double txy = ldv(tau6[3], bo), tyz = ldv(tau6[4], bo), tzx = ldv(tau6[5], bo);
+            if constexpr (VISC) {
+                const double txx = w.t[0], tyy = w.t[1], tzz = w.t[2], txy = w.t[3], tyz = w.t[4], tzx = w.t[5];
                 F[1] -= m0 * txx + m1 * txy + m2 * tzx;
                 F[2] -= m0 * txy + m1 * tyy + m2 * tyz;
                 F[3] -= m0 * tzx + m1 * tyz + m2 * tzz;
-                F[4] -= m0 * ldv(h3[0], bo) + m1 * ldv(h3[1], bo) + m2 * ldv(h3[2], bo);
+                F[4] -= m0 * (double)w.t[6] + m1 * (double)w.t[7] + m2 * (double)w.t[8];
             }
-            return;
-        }
-        const double m = ph.m[AX];
-        const double vel = (AX == 0) ? p.u : (AX == 1 ? p.v : p.w);
-        const double uf = (AX == 0) ? ph.umf.x : (AX == 1 ? ph.umf.y : ph.umf.z);
-        const double ss = m * (vel + uf);
-        F[0] = qq[0] * ss;
-        F[1] = qq[1] * ss;
-        F[2] = qq[2] * ss;
-        F[3] = qq[3] * ss;
-        F[1 + AX] += m * p.p;
-        F[4] = (qq[4] + p.p) * ss - p.p * (uf * m);
-        if (VISC) {
-            F[1] -= m * ldv(tr[0], bo);
-            F[2] -= m * ldv(tr[1], bo);
-            F[3] -= m * ldv(tr[2], bo);
-            F[4] -= m * ldv(hx, bo);
+        } else {
+            const double m = ph.m[AX];
+            const double vel = (AX == 0) ? p.u : (AX == 1 ? p.v : p.w);
+            const double uf = (AX == 0) ? ph.umf.x : (AX == 1 ? ph.umf.y : ph.umf.z);
+            const double ss = m * (vel + uf);
+            F[0] = qq[0] * ss;
+            F[1] = qq[1] * ss;
+            F[2] = qq[2] * ss;
+            F[3] = qq[3] * ss;
+            F[1 + AX] += m * p.p;
+            F[4] = (qq[4] + p.p) * ss - p.p * (uf * m);
+            if constexpr (VISC) {
+                F[1] -= m * (double)w.t[0];
+                F[2] -= m * (double)w.t[1];
+                F[3] -= m * (double)w.t[2];
+                F[4] -= m * (double)w.t[3];
+            }
         }
     }
-    // the epilogue inputs of one row folded into d (loads only); store() then
-    // only writes.  The kernels fetch all their rows before their first store:
-    // dout may alias din or q0 for all the compiler knows, so a load placed
-    // after a store waits for it, and interleaved they would run one memory
-    // round trip per field and row.
-    __device__ __forceinline__ void fetch(uoff bo, double* d) const {
-        if (MODE == 1 || MODE == 2) {
+    // the epilogue: what the sweep adds to at a point (the partial sum; with
+    // the stage update also q0 and the Jacobian), and its result from that.
+    // The kernels load before their first store: dout may alias din or q0 for
+    // all the compiler knows, so a load placed after a store waits for it, and
+    // interleaved they would run one memory round trip per field and row.
+    static constexpr bool kAdds = MODE != 0;
+    struct Out {
+        double din[5], q0[MODE == 3 ? 5 : 1], J;
+    };
+    template <bool NT>
+    __device__ __forceinline__ void load_out(uoff bo, Out& e) const {
 #pragma unroll
-            for (int f = 0; f < 5; f++) d[f] = ldg(din[f], bo) + d[f];
-        } else if (MODE == 3) {
-            const double dtk = dtp[0] / (double)div;
-            const double fj = dtk * (CURV ? ldg(mt.J, bo) : ph.J);
+        for (int f = 0; f < 5; f++) e.din[f] = ldg<NT>(din[f], bo);
+        if constexpr (MODE == 3) {
+#pragma unroll
+            for (int f = 0; f < 5; f++) e.q0[f] = ldg(q0[f], bo);
+            e.J = CURV ? ldg<NT>(mt.J, bo) : ph.J;
+        }
+    }
+    __device__ __forceinline__ void add_out(const Out& e, double* d) const {
+        if constexpr (MODE == 3) {
+            const double fj = dtp[0] / (double)div * e.J;
 #pragma unroll
             for (int f = 0; f < 5; f++) {
-                const double de = ldg(din[f], bo) + d[f];
-                d[f] = ldg(q0[f], bo) - fj * de;
+                const double de = e.din[f] + d[f];
+                d[f] = e.q0[f] - fj * de;
             }
+        } else {
+#pragma unroll
+            for (int f = 0; f < 5; f++) d[f] = e.din[f] + d[f];
         }
     }
-    __device__ __forceinline__ void store(uoff bo, const double* d, const double*) const {
+    template <bool NT>
+    __device__ __forceinline__ void store(uoff bo, const double* d) const {
 #pragma unroll
-        for (int f = 0; f < 5; f++) stg(dout[f], bo, d[f]);
+        for (int f = 0; f < 5; f++) stg<NT>(dout[f], bo, d[f]);
+    }
+    // what the characteristic BC reads at a face point: the state, the weight
+    // and (curvilinear solvers) the caller's face normal and the Jacobian
+    struct FaceIn {
+        double q[5], w, cm[3], J;
+        long fi;          // face index (x: k*let+j, y: k*lxi+i, z: j*lxi+i)
+    };
+    __device__ __forceinline__ FaceIn face_in(uoff bo, int face, const double* sbcc) const {
+        FaceIn in;
+        const long o = bo / 8u;
+        in.fi = AX == 0 ? o / lxi : (AX == 1 ? (o / plane) * lxi + o % lxi : o % plane);
+#pragma unroll
+        for (int v = 0; v < 5; v++) in.q[v] = ldg(q[v], bo);
+        in.w = ldg(sbcc, bo);
+        if constexpr (CURV) {
+            // [2 face][3][face], as gcbc_go takes them
+            const double* c = mt.cm[AX] + (long)face * 3 * nface + in.fi;
+            in.cm[0] = c[0];
+            in.cm[1] = c[nface];
+            in.cm[2] = c[2 * nface];
+            in.J = ldg(mt.J, bo);
+        } else {
+            // unit normal of the face: grad(xi_AX) / |grad(xi_AX)|, grad(xi_AX) = J * metric * e_AX
+            const double sg = ph.m[AX] * ph.J < 0.0 ? -1.0 : 1.0;
+            in.cm[0] = AX == 0 ? sg : 0.0;
+            in.cm[1] = AX == 1 ? sg : 0.0;
+            in.cm[2] = AX == 2 ? sg : 0.0;
+            in.J = ph.J;
+        }
+        return in;
     }
     // non-reflective characteristic correction at a face point from the
     // boundary derivatives of this sweep (gcbc_setup_kernel +
     // gcbc_update_non_reflective_kernel, src/cuda/kernels/gcbc.hpp:251-454)
-    __device__ __forceinline__ void gcbc(uoff bo, int face, const double* drv, double* corr) const {
-        // face index of the face point (x: k*let+j, y: k*lxi+i, z: j*lxi+i)
-        const long o = bo / 8u;
-        const long fi = AX == 0 ? o / lxi : (AX == 1 ? (o / plane) * lxi + o % lxi : o % plane);
+    __device__ __forceinline__ void gcbc(const FaceIn& in, int face, const double* drv, double* corr) const {
         if (rec) {
 #pragma unroll
-            for (int v = 0; v < 5; v++) rec[(face * 5 + v) * nface + fi] = drv[v];
+            for (int v = 0; v < 5; v++) rec[(face * 5 + v) * nface + in.fi] = drv[v];
         }
-        double qq[5];
-        Prim p = prim_at(q, bo, qq);
-        double cm[3], J = ph.J;
-        if constexpr (CURV) {
-            // the caller's face normals ([2 face][3][face], as gcbc_go takes them)
-            const double* c = mt.cm[AX] + (long)face * 3 * nface + fi;
-            cm[0] = c[0];
-            cm[1] = c[nface];
-            cm[2] = c[2 * nface];
-            J = ldg(mt.J, bo);
-        } else {
-            // unit normal of the face: grad(xi_AX) / |grad(xi_AX)|, grad(xi_AX) = J * metric * e_AX
-            const double sg = ph.m[AX] * ph.J < 0.0 ? -1.0 : 1.0;
-            cm[0] = AX == 0 ? sg : 0.0;
-            cm[1] = AX == 1 ? sg : 0.0;
-            cm[2] = AX == 2 ? sg : 0.0;
-        }
+        const Prim p = primitive(in.q);
+        const double J = in.J;
+        const double* cm = in.cm;
         Eig e;
-        e.eleme(cm, qq[0], qq + 1, p.p, ph.umf);
+        e.eleme(cm, in.q[0], in.q + 1, p.p, ph.umf);
         double cha[5], ch[5];
 #pragma unroll
         for (int v = 0; v < 5; v++) cha[v] = J * drv[v];
@@ -325,23 +418,30 @@ struct S2CF : S2T<AX, MODE, VISC, float, true> {};
 template <int AX>
 struct SF {
     static constexpr int NF = 5;
+    static constexpr bool kBlocks = false;
+    static constexpr int kBytes = 40;
     static constexpr bool kGcbc = false;
-    static constexpr bool kPv = false;
     static constexpr int kStash = 0;
     static constexpr int kH = 5;
     static constexpr int kWpe = 3;
     static constexpr bool kFilter = true;
     double* q[5];
-    __device__ __forceinline__ void point(uoff bo, double* v) const {
+    struct Raw { double q[5]; };
+    template <bool NT>
+    __device__ __forceinline__ void load(uoff bo, Raw& w) const {
 #pragma unroll
-        for (int f = 0; f < 5; f++) v[f] = ldg(q[f], bo);
+        for (int f = 0; f < 5; f++) w.q[f] = ldg<NT>(q[f], bo);
     }
-    __device__ __forceinline__ void fetch(uoff, double*) const {}
-    __device__ __forceinline__ void store(uoff bo, const double* d, const double*) const {
+    __device__ __forceinline__ void eval(const Raw& w, double* v) const {
 #pragma unroll
-        for (int f = 0; f < 5; f++) stg(q[f], bo, d[f]);
+        for (int f = 0; f < 5; f++) v[f] = w.q[f];
     }
-    __device__ __forceinline__ void gcbc(uoff, int, const double*, double*) const {}
+    static constexpr bool kAdds = false;
+    template <bool NT>
+    __device__ __forceinline__ void store(uoff bo, const double* d) const {
+#pragma unroll
+        for (int f = 0; f < 5; f++) stg<NT>(q[f], bo, d[f]);
+    }
 };
 
 // SF1: the same filter, one conserved variable per workgroup (blockIdx.y picks
@@ -349,8 +449,9 @@ struct SF {
 template <int AX>
 struct SF1 {
     static constexpr int NF = 1;
+    static constexpr bool kBlocks = false;
+    static constexpr int kBytes = 40;
     static constexpr bool kGcbc = false;
-    static constexpr bool kPv = false;
     static constexpr int kStash = 0;
     static constexpr int kH = 5;
     static constexpr int kWpe = 3;
@@ -358,85 +459,88 @@ struct SF1 {
     double* q;
     long lmx;
     __device__ __forceinline__ double* field() const { return q + (long)blockIdx.y * lmx; }
-    __device__ __forceinline__ void point(uoff bo, double* v) const { v[0] = ldg(field(), bo); }
-    __device__ __forceinline__ void fetch(uoff, double*) const {}
-    __device__ __forceinline__ void store(uoff bo, const double* d, const double*) const { stg(field(), bo, d[0]); }
-    __device__ __forceinline__ void gcbc(uoff, int, const double*, double*) const {}
+    struct Raw { double q; };
+    template <bool NT>
+    __device__ __forceinline__ void load(uoff bo, Raw& w) const { w.q = ldg<NT>(field(), bo); }
+    __device__ __forceinline__ void eval(const Raw& w, double* v) const { v[0] = w.q; }
+    static constexpr bool kAdds = false;
+    template <bool NT>
+    __device__ __forceinline__ void store(uoff bo, const double* d) const { stg<NT>(field(), bo, d[0]); }
 };
 
 // ---------------------------------------------------------------------------
 // pieces shared by the sweep kernels
+//
+// A line of N rows is cut into P = ceil(N/K) chunks of K rows.  Where N is
+// not P*K, the D = P*K - N chunks after the first hold K-1 rows (Chunks), so
+// that the first and the last chunk, with the closure, seam and face rows,
+// are always whole and only the halo exchange has to look at a chunk's
+// length.  The missing row is a padding row at the chunk's end whose table
+// entries pass the recurrences through (chunk_table).
 // ---------------------------------------------------------------------------
-// interior rows and closure rows from a window w[f][u] holding rows s-2+u
+template <int K, bool EX>
+struct Chunks {
+    int D;
+    __device__ __forceinline__ Chunks(int N, int P) : D(EX ? 0 : P * K - N) {}
+    __device__ __forceinline__ int start(int c) const { return EX ? c * K : c * K - min(max(c - 1, 0), D); }
+    __device__ __forceinline__ bool whole(int c) const { return EX || c == 0 || c > D; }
+};
+
+// rows K-H..K-1 of the window's own part and the H halo rows after it: a
+// chunk of K-1 rows has its halo one row earlier
+template <int K, int H, int W>
+__device__ __forceinline__ void close_window(double (&w)[W], const double (&right)[H], bool whole) {
+#pragma unroll
+    for (int k = 0; k < H; k++) w[K + H + k] = whole ? right[k] : (k + 1 < H ? right[k + 1 < H ? k + 1 : 0] : 0.0);
+    w[K + H - 1] = whole ? w[K + H - 1] : right[0];
+}
+
+// interior rows and closure rows from a window w[u] holding rows s-2+u
 // (build_system, numerics_device_pc.hpp:176-293)
-template <int K, int NF, int W>
-__device__ __forceinline__ void window_rhs(const double (&w)[NF][W], double (&r)[NF][K], int L, bool first,
-                                           bool last) {
+template <int K, int W>
+__device__ __forceinline__ void window_rhs(const double (&w)[W], double (&r)[K], bool first, bool last) {
 #pragma unroll
-    for (int f = 0; f < NF; f++)
-#pragma unroll
-        for (int t = 0; t < K; t++)
-            r[f][t] = kAa * (w[f][t + 3] - w[f][t + 1]) + kBb * (w[f][t + 4] - w[f][t]);
+    for (int t = 0; t < K; t++) r[t] = kAa * (w[t + 3] - w[t + 1]) + kBb * (w[t + 4] - w[t]);
     if (first) {
-#pragma unroll
-        for (int f = 0; f < NF; f++) {
-            r[f][0] = kAb00 * w[f][2] + kAb01 * w[f][3] + kAb02 * w[f][4];
-            r[f][1] = kAb10 * (w[f][4] - w[f][2]);
-        }
+        r[0] = kAb00 * w[2] + kAb01 * w[3] + kAb02 * w[4];
+        r[1] = kAb10 * (w[4] - w[2]);
     }
     if (last) {
-#pragma unroll
-        for (int f = 0; f < NF; f++) {
-            double fN1 = 0.0, fN2 = 0.0, fN3 = 0.0;
-#pragma unroll
-            for (int u = 0; u < W; u++) {
-                if (u == L + 1) fN1 = w[f][u];
-                if (u == L) fN2 = w[f][u];
-                if (u == L - 1) fN3 = w[f][u];
-            }
-            const double r1 = -(kAb00 * fN1 + kAb01 * fN2 + kAb02 * fN3);
-            const double r2 = -kAb10 * (fN3 - fN1);
-#pragma unroll
-            for (int t = 0; t < K; t++) {
-                if (t == L - 1) r[f][t] = r1;
-                if (t == L - 2) r[f][t] = r2;
-            }
-        }
+        r[K - 1] = -(kAb00 * w[K + 1] + kAb01 * w[K] + kAb02 * w[K - 1]);
+        r[K - 2] = -kAb10 * (w[K - 1] - w[K + 1]);
     }
 }
 
-// filter rows from a window w[f][u] holding rows s-5+u: 10th order inside,
+// filter rows from a window w[u] holding rows s-5+u: 10th order inside,
 // order 2*dist at distance dist < 5 from a closure end, identity at the end
 // (an = the order-2M coefficient sets, an[6M..6M+M], each for its row's
 // alpha; the alphas enter through the LU tables); cyclic lines are all
 // inside rows
-template <int K, int NF, int W>
-__device__ __forceinline__ void filter_rhs(const double (&w)[NF][W], double (&r)[NF][K], int s, int N, bool cyclic,
+template <int K, int W>
+__device__ __forceinline__ void filter_rhs(const double (&w)[W], double (&r)[K], bool first, bool last,
                                            const double* an) {
     constexpr int H = 5;
 #pragma unroll
     for (int t = 0; t < K; t++) {
-        const int j = s + t;
-        const int dist = cyclic ? H : min(j, N - 1 - j);
+        double v = an[30] * w[t + H];
 #pragma unroll
-        for (int f = 0; f < NF; f++) {
-            double v = an[30] * w[f][t + H];
+        for (int m = 1; m <= 5; m++) v = __builtin_fma(0.5 * an[30 + m], w[t + H + m] + w[t + H - m], v);
+        r[t] = v;
+    }
 #pragma unroll
-            for (int m = 1; m <= 5; m++) v += 0.5 * an[30 + m] * (w[f][t + H + m] + w[f][t + H - m]);
-            r[f][t] = v;
-        }
-        if (dist < H) {
+    for (int end = 0; end < 2; end++) {
+        if (end == 0 ? first : last) {
 #pragma unroll
-            for (int f = 0; f < NF; f++) {
-                double v = w[f][t + H];
+            for (int dist = 0; dist < H; dist++) {
+                const int t = end == 0 ? dist : K - 1 - dist;
+                double v = w[t + H];
                 if (dist > 0) {
-                    const double* cf = an + 6 * dist;
-                    v = cf[0] * w[f][t + H];
+                    v = an[6 * dist] * w[t + H];
 #pragma unroll
-                    for (int m = 1; m < H; m++)
-                        if (m <= dist) v += 0.5 * cf[m] * (w[f][t + H + m] + w[f][t + H - m]);
+                    for (int m = 1; m <= dist; m++)
+                        v = __builtin_fma(0.5 * an[6 * dist + m], w[t + H + m] + w[t + H - m], v);
                 }
-                r[f][t] = v;
+                r[t] = v;
             }
         }
     }
@@ -444,12 +548,12 @@ __device__ __forceinline__ void filter_rhs(const double (&w)[NF][W], double (&r)
 
 // Sherman-Morrison correction of a cyclic filter solve: y0 and yN1 are the
 // solution of the modified system at rows 0 and N-1 (tab layout of
-// build_line_table: z at 5N, 1/(1 + z0 + kappa zN1) at 6N, kappa at 6N+1)
+// chunk_table: z at 5NP, 1/(1 + z0 + kappa zN1) at 6NP, kappa at 6NP+1)
 template <int K, int NF>
-__device__ __forceinline__ void cyclic_correction(const double* tab, int N, int s, const double (&y0)[NF],
+__device__ __forceinline__ void cyclic_correction(const double* tab, int NP, int s, const double (&y0)[NF],
                                                   const double (&yN1)[NF], double (&r)[NF][K]) {
-    const double* z = tab + 5 * N;
-    const double inv = tab[6 * N], kappa = tab[6 * N + 1];
+    const double* z = tab + 5 * NP;
+    const double inv = tab[6 * NP], kappa = tab[6 * NP + 1];
 #pragma unroll
     for (int f = 0; f < NF; f++) {
         const double beta = (y0[f] + kappa * yN1[f]) * inv;
@@ -458,18 +562,15 @@ __device__ __forceinline__ void cyclic_correction(const double* tab, int N, int 
     }
 }
 
-// the same rows as window_rhs, streamed through a 5-row register window so
-// that only the rows a right-hand side needs are live (rows from an LDS tile)
+// the same rows as window_rhs for rows s..s+L-1 of a chunk, streamed through
+// a 5-row register window so that only the rows a right-hand side needs are
+// live (rows from an LDS tile); zero in the padding rows
 template <int K, int NF, class ROW>
-__device__ __forceinline__ void stream_rhs(ROW&& row_of, double (&r)[NF][K], int L, bool first, bool last) {
+__device__ __forceinline__ void stream_rhs(ROW&& row_of, double (&r)[NF][K], int s, int L, int N, bool seam) {
     constexpr int W = K + 4;
     double w0[NF], w1[NF], w2[NF], w3[NF], w4[NF];
-    double f0[NF], f1[NF], f2[NF], fN1[NF], fN2[NF], fN3[NF];
 #pragma unroll
-    for (int f = 0; f < NF; f++) {
-        w0[f] = w1[f] = w2[f] = w3[f] = w4[f] = 0.0;
-        f0[f] = f1[f] = f2[f] = fN1[f] = fN2[f] = fN3[f] = 0.0;
-    }
+    for (int f = 0; f < NF; f++) w0[f] = w1[f] = w2[f] = w3[f] = w4[f] = 0.0;
 #pragma unroll
     for (int u = 0; u < W; u++) {
         double v[NF];
@@ -477,81 +578,62 @@ __device__ __forceinline__ void stream_rhs(ROW&& row_of, double (&r)[NF][K], int
 #pragma unroll
         for (int f = 0; f < NF; f++) { w0[f] = w1[f]; w1[f] = w2[f]; w2[f] = w3[f]; w3[f] = w4[f]; w4[f] = v[f]; }
         if (u >= 4) {
-            const int t = u - 4;
+            const int t = u - 4, j = s + t;
 #pragma unroll
-            for (int f = 0; f < NF; f++) r[f][t] = kAa * (w3[f] - w1[f]) + kBb * (w4[f] - w0[f]);
-        }
-        if (u == 4) {
-#pragma unroll
-            for (int f = 0; f < NF; f++) { f0[f] = w2[f]; f1[f] = w3[f]; f2[f] = w4[f]; }
-        }
-#pragma unroll
-        for (int f = 0; f < NF; f++) {
-            if (u == L + 1) fN1[f] = w4[f];
-            if (u == L) fN2[f] = w4[f];
-            if (u == L - 1) fN3[f] = w4[f];
-        }
-    }
-    if (first) {
-#pragma unroll
-        for (int f = 0; f < NF; f++) {
-            r[f][0] = kAb00 * f0[f] + kAb01 * f1[f] + kAb02 * f2[f];
-            r[f][1] = kAb10 * (f2[f] - f0[f]);
-        }
-    }
-    if (last) {
-#pragma unroll
-        for (int f = 0; f < NF; f++) {
-            const double r1 = -(kAb00 * fN1[f] + kAb01 * fN2[f] + kAb02 * fN3[f]);
-            const double r2 = -kAb10 * (fN3[f] - fN1[f]);
-#pragma unroll
-            for (int t = 0; t < K; t++) {
-                if (t == L - 1) r[f][t] = r1;
-                if (t == L - 2) r[f][t] = r2;
+            for (int f = 0; f < NF; f++) {
+                double x = kAa * (w3[f] - w1[f]) + kBb * (w4[f] - w0[f]);
+                if (!seam) {
+                    if (t == 0 && j == 0) x = kAb00 * w2[f] + kAb01 * w3[f] + kAb02 * w4[f];
+                    if (t == 1 && j == 1) x = kAb10 * (w3[f] - w1[f]);
+                    if (j == N - 2) x = -kAb10 * (w1[f] - w3[f]);
+                    if (j == N - 1) x = -(kAb00 * w2[f] + kAb01 * w1[f] + kAb02 * w0[f]);
+                }
+                r[f][t] = t < L ? x : 0.0;
             }
         }
     }
 }
 
+// zero in the padding row of a chunk of K-1 rows, before the backward recurrence
+template <int K, int NF>
+__device__ __forceinline__ void zero_padding(double (&r)[NF][K], bool whole) {
+#pragma unroll
+    for (int f = 0; f < NF; f++) r[f][K - 1] = whole ? r[f][K - 1] : 0.0;
+}
+
 // quasi-disjoint seam rows, wrapped onto the opposite end of the line
 // (build_system seam branch, numerics_device_pc.hpp:199-282, with the
-// neighbour sums formed as fill_gpu_buffer_kernel does, kernels/numerics_pc.hpp:86-121)
-template <int K, int NF, class SW>
-__device__ __forceinline__ void seam_rows(const SW& sw, uoff base, uoff st, int N, int L, bool first, bool last,
-                                          const double* pb, double (&r)[NF][K]) {
+// neighbour sums formed as fill_gpu_buffer_kernel does, kernels/numerics_pc.hpp:86-121).
+// For the chunk at the line's start (end = 0) or end (end = 1; L rows):
+// row(e, i, v) gives the values at distance i from end e.
+template <int K, int NF, class ROW>
+__device__ __forceinline__ void seam_rows(ROW&& row, int end, int L, const double* pb, double (&r)[NF][K]) {
     const double* pbco = pb;
     const double* pbci = pb + 16;
+    double s0[NF], s1[NF], o0[NF], o1[NF];
 #pragma unroll
-    for (int end = 0; end < 2; end++) {
-        if ((end == 0 && !first) || (end == 1 && !last)) continue;
-        double s0[NF], s1[NF], o0[NF], o1[NF];
+    for (int f = 0; f < NF; f++) { s0[f] = 0.0; s1[f] = 0.0; o0[f] = 0.0; o1[f] = 0.0; }
+#pragma unroll 1
+    for (int i = 0; i < kLmd; i++) {
+        double v[NF];
+        row(end, i, v);
 #pragma unroll
-        for (int f = 0; f < NF; f++) { s0[f] = 0.0; s1[f] = 0.0; o0[f] = 0.0; o1[f] = 0.0; }
-        for (int i = 0; i < kLmd; i++) {
-            double v[NF];
-            sw.point(base + (uoff)(end == 0 ? i : N - 1 - i) * st, v);
+        for (int f = 0; f < NF; f++) { s0[f] += pbci[i] * v[f]; s1[f] += pbci[kLmd + i] * v[f]; }
+        row(1 - end, i, v);
 #pragma unroll
-            for (int f = 0; f < NF; f++) { s0[f] += pbci[i] * v[f]; s1[f] += pbci[kLmd + i] * v[f]; }
-        }
-        for (int i = 0; i < kLmd; i++) {
-            double v[NF];
-            sw.point(base + (uoff)(end == 0 ? N - 1 - i : i) * st, v);
+        for (int f = 0; f < NF; f++) { o0[f] += pbco[i] * v[f]; o1[f] += pbco[kLmd + i] * v[f]; }
+    }
 #pragma unroll
-            for (int f = 0; f < NF; f++) { o0[f] += pbco[i] * v[f]; o1[f] += pbco[kLmd + i] * v[f]; }
-        }
+    for (int f = 0; f < NF; f++) {
+        const double a = s0[f] + o0[f], b = s1[f] + o1[f];
+        if (end == 0) {
+            r[f][0] = a;
+            r[f][1] = b;
+        } else {
 #pragma unroll
-        for (int f = 0; f < NF; f++) {
-            if (end == 0) {
-                r[f][0] = s0[f] + o0[f];
-                r[f][1] = s1[f] + o1[f];
-            } else {
-                const double r1 = -(s0[f] + o0[f]);
-                const double r2 = -(s1[f] + o1[f]);
-#pragma unroll
-                for (int t = 0; t < K; t++) {
-                    if (t == L - 1) r[f][t] = r1;
-                    if (t == L - 2) r[f][t] = r2;
-                }
+            for (int t = 0; t < K; t++) {
+                if (t == L - 1) r[f][t] = -a;
+                if (t == L - 2) r[f][t] = -b;
             }
         }
     }
@@ -559,43 +641,28 @@ __device__ __forceinline__ void seam_rows(const SW& sw, uoff base, uoff st, int 
 
 // characteristic correction of a face (first or last chunk of a line, never
 // both: lines have at least two chunks), weighted by sbcc on the kMbci rows
-// next to the face; the face derivative is the uncorrected solve result
-template <int K, int NF, class SW, bool GCBC, bool EX>
-__device__ __forceinline__ void face_corrections(const SW& sw, uoff base, uoff st, int N, int s, int L, bool first,
-                                                 bool last, double (&r)[NF][K], const double* sbcc) {
-    if constexpr (GCBC) {
-        if (first || last) {
-            const int face = last ? 1 : 0;
-            double drv[NF], corr[NF];
+// next to the face; the face derivative is the uncorrected solve result.  L =
+// rows of the chunk.
+template <int K, int NF, class SW, class FACE>
+__device__ __forceinline__ void face_correction(const SW& sw, const FACE& fc, int face, int L, double (&r)[NF][K]) {
+    static_assert(kMbci == 1, "the face row only");
+    double drv[NF], corr[NF];
 #pragma unroll
-            for (int f = 0; f < NF; f++) {
-                double d = r[f][0];
+    for (int f = 0; f < NF; f++) {
+        drv[f] = r[f][0];
 #pragma unroll
-                for (int t = 1; t < K; t++)
-                    if (last && ((EX && t == K - 1) || (!EX && t == L - 1))) d = r[f][t];
-                drv[f] = d;
-            }
-            sw.gcbc(base + (uoff)(face ? N - 1 : 0) * st, face, drv, corr);
-#pragma unroll
-            for (int t = 0; t < K; t++) {
-                const int row = s + t;
-                const bool in = (EX || t < L) && (face ? row >= N - kMbci : row < kMbci);
-                if (in) {
-                    const double wgt = ldg(sbcc, base + (uoff)row * st);
-#pragma unroll
-                    for (int f = 0; f < NF; f++) r[f][t] += wgt * corr[f];
-                }
-            }
-        }
+        for (int t = 1; t < K; t++)
+            if (face && t == L - 1) drv[f] = r[f][t];
     }
+    sw.gcbc(fc, face, drv, corr);
+#pragma unroll
+    for (int t = 0; t < K; t++)
+        if (face ? t == L - 1 : t == 0) {
+#pragma unroll
+            for (int f = 0; f < NF; f++) r[f][t] += fc.w * corr[f];
+        }
 }
 
-// ---------------------------------------------------------------------------
-// variant "direct" (equal chunks, N = P*K): each thread evaluates the
-// pointwise inputs of its own K rows once; the two halo rows on each side come
-// from the neighbouring chunks (shuffles within a wave segment for x lines,
-// LDS for y/z lines)
-// ---------------------------------------------------------------------------
 // functors that reduce the time step's maxima: value = in the point
 // evaluation of a y/z sweep (constant metrics), close = in the closing x
 // sweep's stores (per-point metrics)
@@ -610,184 +677,182 @@ struct DtFold<SW, std::void_t<decltype(SW::kDt)>> {
     static constexpr bool close = SW::kDt && SW::kCurv;
 };
 
-template <int K, int AX, int TL, class SW, bool GCBC>
-__global__ void __launch_bounds__(AX == 0 ? 256 : TL * kMaxP)
-__attribute__((amdgpu_waves_per_eu(AX == 0 ? 1 : (K == 16 ? 2 : SW::kWpe))))
+// ---------------------------------------------------------------------------
+// variant "direct", y/z lines: TL consecutive lines x P chunks per workgroup;
+// each thread evaluates the pointwise inputs of its own K rows once, the halo
+// rows on each side and the 8 + 8 rows of a periodic seam come from the other
+// chunks through LDS.
+//
+// Bound by memory latency at the occupancy its registers allow (K = 16: 256
+// VGPRs, two 4-wave workgroups a CU): the K x NF values stay in registers from
+// the loads to the stores.  So nothing but them is live: the loads run
+// kRowsAhead rows ahead of the evaluation (all rows at once spill 500-700 B a
+// lane), a field's window exists only while its right-hand side is formed, and
+// the epilogue's loads run kRowsOut rows ahead of the additions.  16 lines are
+// 128-byte rows.  Measured at 256^3 (start -> now, us; a copy of 2.1 GB runs at
+// 4.8 TB/s, the same row pattern without arithmetic at 5.3 along y and 4.7
+// along z): S1y 284 -> 216 (5.6 TB/s), S2y 550 -> 482 (5.3), S1z 309 -> 275
+// (4.4), S2z 514 -> 431 (4.4).
+// ---------------------------------------------------------------------------
+constexpr int kRowsAhead = 2;   // rows whose loads are in flight while a row is evaluated
+constexpr int kRowsOut = 4;     // rows whose epilogue loads are in flight
+
+template <int K, int AX, int TL, class SW, bool GCBC, bool EX, bool NT>
+__global__ void __launch_bounds__(TL * kMaxP) __attribute__((amdgpu_waves_per_eu(K == 16 ? 2 : SW::kWpe)))
 direct_kernel(AxisDesc ax, SweepCommon cm, SW sw) {
     constexpr int NF = SW::NF;
     constexpr int H = SW::kH;
     constexpr int W = K + 2 * H;
+    static_assert(AX != 0, "x lines run xt_kernel");
     static_assert(H <= K, "halo rows come from the neighbouring chunks only");
     extern __shared__ double lds[];
 
-    const int N = ax.N, P = ax.P;
-    int c, lloc = 0, GS = 1;
-    long line;
-    if (AX == 0) {
-        GS = ax.GS;
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-        const int lpw = 64 / GS;
-        c = lane % GS;
-        line = (long)blockIdx.x * (4 * lpw) + wave * lpw + lane / GS;
-    } else {
-        lloc = threadIdx.x % TL;
-        c = threadIdx.x / TL;
-        line = group_of(ax.xcd) * TL + lloc;
-    }
+    const int N = ax.N, P = ax.P, NP = P * K;
+    const Chunks<K, EX> ch(N, P);
+    const int lloc = threadIdx.x % TL;
+    const int c = threadIdx.x / TL;
+    const long line = group_of(ax.xcd) * TL + lloc;
     const bool act = line < ax.nlines;
-    const bool cv = c < P;
-    const bool work = act && cv;
-    const int s = c * K;
+    const int s = c * K, row0 = ch.start(c);      // table and line position of the chunk
+    const bool whole = ch.whole(c);
     const uoff st = (uoff)ax.st * 8u;
-    const uoff base = line_off(AX, act ? (uoff)line : 0u, (uoff)cm.lxi, (uoff)cm.plane);
+    // threads past the last line repeat it, padding rows repeat the chunk's last
+    // row: no branches around the loads, and nothing of theirs is stored
+    const uoff base = line_off(AX, (uoff)(act ? line : ax.nlines - 1), (uoff)cm.lxi, (uoff)cm.plane);
+    const uoff cbase = base + (uoff)row0 * st;
+    auto off = [&](int t) { return cbase + (uoff)(EX || t < K - 1 || whole ? t : K - 2) * st; };
     const double* tab = SW::kFilter ? ax.ftab : ax.tab;
     const bool cyc = SW::kFilter && ax.seam;
+    const bool first = c == 0, last = c == P - 1;
 
     // time-step maxima (DtFold functors; every lane of the workgroup's waves
     // is a thread, the launcher checks)
     constexpr bool kDt = DtFold<SW>::value;
     double dm0 = 0.0, dm1 = 0.0;
-    double w[NF][W];
+    double x[NF][K];
+    // the loads of kRowsAhead rows are in flight while a row is evaluated
+    constexpr int RA = NF > 1 && kRowsAhead < K ? kRowsAhead : K;
+    typename SW::Raw raw[RA];
+#pragma unroll
+    for (int t = 0; t < RA; t++) sw.template load<NT>(off(t), raw[t]);
+    if (RA < K) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int t = 0; t < K; t++) {
-        double x[NF];
-        if (work) {
-            if constexpr (kDt) sw.point_dt(base + (uoff)(s + t) * st, x, dm1);
-            else sw.point(base + (uoff)(s + t) * st, x);
-        } else {
+        double v[NF];
+        if constexpr (kDt) sw.eval_dt(raw[t % RA], v, dm1);
+        else sw.eval(raw[t % RA], v);
 #pragma unroll
-            for (int f = 0; f < NF; f++) x[f] = 0.0;
+        for (int f = 0; f < NF; f++) x[f][t] = v[f];
+        if (t + RA < K) {
+            sw.template load<NT>(off(t + RA), raw[t % RA]);
+            __builtin_amdgcn_sched_barrier(0);
         }
-#pragma unroll
-        for (int f = 0; f < NF; f++) w[f][t + H] = x[f];
     }
     if constexpr (kDt) {
         // the convective maximum from u, v, w, c^2 of the rows; the viscous one
         // at the largest 1/rho
-        if (work) {
 #pragma unroll
-            for (int t = 0; t < K; t++)
-                dm0 = fmax(dm0, dt_conv(sw.ph, w[0][t + H], w[1][t + H], w[2][t + H], w[3][t + H]));
-            dm1 = dt_visc(sw.ph, dm1);
-        }
+        for (int t = 0; t < K; t++) dm0 = fmax(dm0, dt_conv(sw.ph, x[0][t], x[1][t], x[2][t], x[3][t]));
+        dm1 = dt_visc(sw.ph, dm1);
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) {
             dm0 = fmax(dm0, __shfl_xor(dm0, o));
             dm1 = fmax(dm1, __shfl_xor(dm1, o));
         }
     }
-    if (AX == 0) {
+    // halo rows through LDS, hb[(f*2H + k)*P + c][TL], k = the first H then the
+    // last H rows of chunk c, FX fields at a time (neighbours wrap on cyclic
+    // lines); on a seam axis also the 8 rows next to each end, [2 end][8][NF][TL]
+    constexpr int FX = SW::kFilter ? 1 : NF;
+    const int cl = c > 0 ? c - 1 : (cyc ? P - 1 : 0), cr = c + 1 < P ? c + 1 : (cyc ? 0 : P - 1);
+    double* ends = lds + 2 * H * NF * P * TL;
+    double r[NF][K];
 #pragma unroll
-        for (int f = 0; f < NF; f++) {
-            w[f][0] = __shfl_up(w[f][K], 1, GS);
-            w[f][1] = __shfl_up(w[f][K + 1], 1, GS);
-            w[f][K + 2] = __shfl_down(w[f][2], 1, GS);
-            w[f][K + 3] = __shfl_down(w[f][3], 1, GS);
-        }
-    } else if constexpr (H != 2) {
-        // halo rows through LDS one field at a time: hb[k*P + c][TL], k = the
-        // first H then the last H rows of chunk c (neighbours wrap on cyclic lines)
-        const int cl = c > 0 ? c - 1 : (cyc ? P - 1 : 0), cr = c + 1 < P ? c + 1 : (cyc ? 0 : P - 1);
+    for (int f0 = 0; f0 < NF; f0 += FX) {
+        if (f0 > 0) __syncthreads();
 #pragma unroll
-        for (int f = 0; f < NF; f++) {
-            if (f > 0) __syncthreads();
+        for (int e = 0; e < FX; e++) {
+            const int f = f0 + e;
 #pragma unroll
             for (int k = 0; k < H; k++) {
-                lds[(k * P + c) * TL + lloc] = w[f][H + k];
-                lds[((H + k) * P + c) * TL + lloc] = w[f][K + k];
-            }
-            __syncthreads();
-#pragma unroll
-            for (int k = 0; k < H; k++) {
-                w[f][k] = lds[((H + k) * P + cl) * TL + lloc];
-                w[f][K + H + k] = lds[(k * P + cr) * TL + lloc];
+                lds[((e * 2 * H + k) * P + c) * TL + lloc] = x[f][k];
+                lds[((e * 2 * H + H + k) * P + c) * TL + lloc] =
+                    whole ? x[f][K - H + k] : x[f][K - H + k > 0 ? K - H + k - 1 : 0];
             }
         }
-    } else {
-        // halo rows through LDS: hb[(f*4 + k)*P + c][TL], k = chunk rows 0, 1, K-2, K-1
-        const int cl = c > 0 ? c - 1 : 0, cr = c + 1 < P ? c + 1 : P - 1;
+        if (!SW::kFilter && ax.seam && (first || last)) {
 #pragma unroll
-        for (int f = 0; f < NF; f++) {
-            lds[((f * 4 + 0) * P + c) * TL + lloc] = w[f][2];
-            lds[((f * 4 + 1) * P + c) * TL + lloc] = w[f][3];
-            lds[((f * 4 + 2) * P + c) * TL + lloc] = w[f][K];
-            lds[((f * 4 + 3) * P + c) * TL + lloc] = w[f][K + 1];
+            for (int i = 0; i < kLmd; i++)
+#pragma unroll
+                for (int f = 0; f < NF; f++)
+                    ends[(((first ? 0 : kLmd) + i) * NF + f) * TL + lloc] = first ? x[f][i] : x[f][K - 1 - i];
         }
         __syncthreads();
 #pragma unroll
-        for (int f = 0; f < NF; f++) {
-            w[f][0] = lds[((f * 4 + 2) * P + cl) * TL + lloc];
-            w[f][1] = lds[((f * 4 + 3) * P + cl) * TL + lloc];
-            w[f][K + 2] = lds[((f * 4 + 0) * P + cr) * TL + lloc];
-            w[f][K + 3] = lds[((f * 4 + 1) * P + cr) * TL + lloc];
+        for (int e = 0; e < FX; e++) {
+            const int f = f0 + e;
+            double w[W], right[H];
+#pragma unroll
+            for (int k = 0; k < H; k++) {
+                w[k] = lds[((e * 2 * H + H + k) * P + cl) * TL + lloc];
+                right[k] = lds[((e * 2 * H + k) * P + cr) * TL + lloc];
+            }
+#pragma unroll
+            for (int t = 0; t < K; t++) w[t + H] = x[f][t];
+            close_window<K, H, W>(w, right, whole);
+            if constexpr (SW::kFilter) filter_rhs<K, W>(w, r[f], first && !cyc, last && !cyc, ax.ftab + 6 * NP + 8);
+            else window_rhs<K, W>(w, r[f], first && !ax.seam, last && !ax.seam);
         }
     }
-    double pv[SW::kPv ? NF : 1][K];
-    if constexpr (SW::kPv) {
+    if (!SW::kFilter && ax.seam && (first || last))
+        seam_rows<K, NF>([&](int end, int i, double* v) {
 #pragma unroll
-        for (int f = 0; f < NF; f++)
-#pragma unroll
-            for (int t = 0; t < K; t++) pv[f][t] = w[f][t + 2];
-    }
-    double r[NF][K];
-    if constexpr (SW::kFilter) {
-        filter_rhs<K, NF, W>(w, r, s, N, cyc, ax.ftab + 6 * N + 8);
-    } else {
-        window_rhs<K, NF, W>(w, r, K, work && c == 0 && !ax.seam, work && c == P - 1 && !ax.seam);
-        if (work && ax.seam && (c == 0 || c == P - 1))
-            seam_rows<K, NF>(sw, base, st, N, K, c == 0, c == P - 1, cm.pb, r);
-    }
+            for (int f = 0; f < NF; f++) v[f] = ends[((end * kLmd + i) * NF + f) * TL + lloc];
+        }, first ? 0 : 1, K, cm.pb, r);
 
     double carry[NF], G[NF], X[NF];
-    forward_local<K, NF, true>(tab, N, s, K, r, carry);
-    if (AX == 0) {
-        scan_forward<NF>(cv ? tab[3 * N + s + K - 1] : 1.0, carry, cv, c, GS, G);
-    } else {
-        __syncthreads();                                // halo reads done: reuse LDS
+    forward_local<K, NF>(tab, NP, s, r, carry);
+    __syncthreads();                                // halo reads done: reuse LDS
 #pragma unroll
-        for (int f = 0; f < NF; f++) lds[(f * P + c) * TL + lloc] = carry[f];
-        // the waves' time-step maxima go past the carries of both folds
-        double* dl = lds + 3 * NF * P * TL;
-        if constexpr (kDt) {
-            if ((threadIdx.x & 63) == 0) {
-                dl[2 * (threadIdx.x >> 6)] = dm0;
-                dl[2 * (threadIdx.x >> 6) + 1] = dm1;
-            }
+    for (int f = 0; f < NF; f++) lds[(f * P + c) * TL + lloc] = carry[f];
+    // the waves' time-step maxima go past the carries of both folds
+    double* dl = lds + 3 * NF * P * TL;
+    if constexpr (kDt) {
+        if ((threadIdx.x & 63) == 0) {
+            dl[2 * (threadIdx.x >> 6)] = dm0;
+            dl[2 * (threadIdx.x >> 6) + 1] = dm1;
         }
-        __syncthreads();
-        if constexpr (kDt) {
-            if (threadIdx.x == 0) {
-                double a0 = 0.0, a1 = 0.0;
-                for (int v = 0; v < (int)(blockDim.x >> 6); v++) {
-                    a0 = fmax(a0, dl[2 * v]);
-                    a1 = fmax(a1, dl[2 * v + 1]);
-                }
-                sw.dtpart[2 * blockIdx.x] = a0;
-                sw.dtpart[2 * blockIdx.x + 1] = a1;
-            }
-        }
-        fold_forward<NF, true, K>(lds, tab, N, P, TL, c, lloc, G);
     }
-    apply_carry<K, NF, true>(tab, 3 * N, s, K, r, G);
-    backward_local<K, NF, true>(tab, N, s, K, r, carry);
-    if (AX == 0) {
-        scan_backward<NF>(cv ? tab[4 * N + s] : 0.0, carry, cv, c, P, GS, X);
-    } else {
-        double* xb = lds + NF * P * TL;
+    __syncthreads();
+    if constexpr (kDt) {
+        if (threadIdx.x == 0) {
+            double a0 = 0.0, a1 = 0.0;
+            for (int v = 0; v < (int)(blockDim.x >> 6); v++) {
+                a0 = fmax(a0, dl[2 * v]);
+                a1 = fmax(a1, dl[2 * v + 1]);
+            }
+            sw.dtpart[2 * blockIdx.x] = a0;
+            sw.dtpart[2 * blockIdx.x + 1] = a1;
+        }
+    }
+    fold_forward<NF, K, SW::kFilter>(lds, tab, NP, P, TL, c, lloc, G);
+    apply_carry<K, NF>(tab, 3 * NP, s, r, G);
+    if constexpr (!EX) zero_padding<K, NF>(r, whole);
+    backward_local<K, NF>(tab, NP, s, r, carry);
+    double* xb = lds + NF * P * TL;
 #pragma unroll
-        for (int f = 0; f < NF; f++) xb[(f * P + c) * TL + lloc] = carry[f];
-        __syncthreads();
-        fold_backward<NF, true, K>(xb, tab, N, P, TL, c, lloc, X);
-    }
-    apply_carry<K, NF, true>(tab, 4 * N, s, K, r, X);
-    if (AX != 0 && cyc) {
+    for (int f = 0; f < NF; f++) xb[(f * P + c) * TL + lloc] = carry[f];
+    __syncthreads();
+    fold_backward<NF, K, SW::kFilter>(xb, tab, NP, P, TL, c, lloc, X);
+    apply_carry<K, NF>(tab, 4 * NP, s, r, X);
+    if (cyc) {
         // rows 0 and N-1 of the modified system through LDS (after the folds' reads)
         double* ends = lds + 2 * NF * P * TL;
-        if (c == 0) {
+        if (first) {
 #pragma unroll
             for (int f = 0; f < NF; f++) ends[f * TL + lloc] = r[f][0];
         }
-        if (c == P - 1) {
+        if (last) {
 #pragma unroll
             for (int f = 0; f < NF; f++) ends[(NF + f) * TL + lloc] = r[f][K - 1];
         }
@@ -798,68 +863,96 @@ direct_kernel(AxisDesc ax, SweepCommon cm, SW sw) {
             y0[f] = ends[f * TL + lloc];
             yN1[f] = ends[(NF + f) * TL + lloc];
         }
-        cyclic_correction<K, NF>(tab, N, s, y0, yN1, r);
+        cyclic_correction<K, NF>(tab, NP, s, y0, yN1, r);
     }
 
-    if (!work) return;
-    face_corrections<K, NF, SW, GCBC, true>(sw, base, st, N, s, K, c == 0, c == P - 1, r, cm.sbcc);
-    // every row's epilogue loads before the first store
+    if (!act) return;
+    if constexpr (GCBC) {
+        if (first || last) {
+            const auto fc = sw.face_in(base + (uoff)(first ? 0 : N - 1) * st, first ? 0 : 1, cm.sbcc);
+            face_correction<K, NF, SW>(sw, fc, first ? 0 : 1, K, r);
+        }
+    }
+    // every row's epilogue loads before the first store, kRowsOut rows in flight
+    if constexpr (SW::kAdds) {
+        typename SW::Out out[kRowsOut];
 #pragma unroll
-    for (int t = 0; t < K; t++) {
-        double d[NF];
+        for (int t = 0; t < kRowsOut; t++) sw.template load_out<NT>(off(t), out[t]);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int f = 0; f < NF; f++) d[f] = r[f][t];
-        sw.fetch(base + (uoff)(s + t) * st, d);
+        for (int t = 0; t < K; t++) {
+            double d[NF];
 #pragma unroll
-        for (int f = 0; f < NF; f++) r[f][t] = d[f];
+            for (int f = 0; f < NF; f++) d[f] = r[f][t];
+            sw.add_out(out[t % kRowsOut], d);
+#pragma unroll
+            for (int f = 0; f < NF; f++) r[f][t] = d[f];
+            if (t + kRowsOut < K) {
+                sw.template load_out<NT>(off(t + kRowsOut), out[t % kRowsOut]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
     }
 #pragma unroll
     for (int t = 0; t < K; t++) {
-        double d[NF], p[NF];
+        if (EX || t < K - 1 || whole) {
+            double d[NF];
 #pragma unroll
-        for (int f = 0; f < NF; f++) { d[f] = r[f][t]; p[f] = SW::kPv ? pv[SW::kPv ? f : 0][t] : 0.0; }
-        sw.store(base + (uoff)(s + t) * st, d, p);
+            for (int f = 0; f < NF; f++) d[f] = r[f][t];
+            sw.template store<NT>(off(t), d);
+        }
     }
 }
 
 // ---------------------------------------------------------------------------
-// variant "direct" for x lines (equal chunks): one wave holds the GS-lane
-// chunk groups of 64/GS consecutive lines, which are one contiguous run of
-// memory.  Lanes load and evaluate that run with fully coalesced accesses (J
-// points per lane), the values are transposed field by field through a
-// wave-private LDS buffer into the chunk layout (halo rows included), the
-// line is solved with wave scans, and the results go back through the buffer
-// for coalesced stores.  No workgroup barrier: a workgroup is one wave.
+// variant "direct" for x lines: one wave holds the P chunks of 64/P
+// consecutive lines (lane = line * P + chunk), one contiguous run of memory.
+// Lanes load and evaluate that run with fully coalesced accesses (K points
+// per lane), the values are transposed field by field through a wave-private
+// LDS buffer into the chunk layout (halo and seam rows included), the line is
+// solved with wave scans, and the results go back through the buffer for
+// coalesced stores.  No workgroup barrier: a workgroup is one wave.
+//
+// Two waves a SIMD, each with its 8 points' loads in flight; at 256^3 the
+// sweeps run at the rate of a plain stream of the same fields (5.6 TB/s): S1x
+// 556 -> 520 us, filter 392 -> 240 us, S2x 606 -> 548 us in a step.  What held
+// them back were instructions, not bytes (the filter: 4150 a wave, 2000 now):
+// branches around every point, closure rows tested row by row, seam rows read
+// again from memory, scans over the whole line.
 // ---------------------------------------------------------------------------
-template <int K, class SW, bool GCBC>
-__global__ void __launch_bounds__(64) xt_kernel(AxisDesc ax, SweepCommon cm, SW sw) {
+template <int K, class SW, bool GCBC, bool EX, bool NT>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) xt_kernel(AxisDesc ax, SweepCommon cm, SW sw) {
     constexpr int NF = SW::NF;
-    constexpr int J = K;                  // points per lane: (64/GS)*P*K <= 64*K
+    constexpr int J = K;                  // points per lane: (64/P)*N <= 64*K
     constexpr int H = SW::kH;
     constexpr int W = K + 2 * H;
-    static_assert(H <= K, "halo rows come from the neighbouring chunks only");
-    // [64/GS lines][P chunks][K+1], then (kStash > 0) the stashed point
-    // values [kStash][J][64]
+    static_assert(K == 8, "row = 8 * chunk + t");
+    // [64/P lines][P chunks][K+1], 64 slots for lanes past the run, then
+    // (kStash > 0) the stashed point values [kStash][J][64]
     extern __shared__ double lds[];
 
-    const int N = ax.N, P = ax.P, GS = ax.GS;
+    const int N = ax.N, P = ax.P, NP = P * K;
+    const Chunks<K, EX> ch(N, P);
     const int lane = threadIdx.x;
-    const int lpw = 64 / GS;
-    double* stash = lds + lpw * P * (K + 1);
-    const long line0 = (long)blockIdx.x * lpw;
+    const int lpw = 64 / P;
+    double* stash = lds + lpw * P * (K + 1) + 64;
+    const long line0 = group_of(ax.xcd) * lpw;
     const int nl = (int)min((long)lpw, ax.nlines - line0);   // lines of this wave
     const int npts = nl * N;
-    const uoff st = (uoff)ax.st * 8u;                        // 8: x rows are adjacent
     const uoff run = line_off(0, (uoff)line0, (uoff)cm.lxi, (uoff)cm.plane);
+    // lanes past the run repeat its last point: no branches around the loads
+    auto off = [&](int j) { return run + (uoff)min(lane + 64 * j, npts - 1) * 8u; };
 
-    // coalesced evaluation: lane handles points lane + 64*j of the run
+    // coalesced evaluation: lane handles points lane + 64*j of the run.  A
+    // functor with too many values a point for all 8 in flight (kBlocks) takes
+    // one after the other: a branch a point keeps the compiler from hoisting
+    // the next ones' loads (S2C: 8 points at once spill 580 B a lane, 233 -> 541 us)
     double xq[NF][J];
 #pragma unroll
     for (int j = 0; j < J; j++) {
-        const int p = lane + 64 * j;
         double x[NF];
-        if (p < npts) {
-            sw.point(run + (uoff)p * st, x);
+        if (!SW::kBlocks || lane + 64 * j < npts) {
+            point<NT>(sw, off(j), x);
         } else {
 #pragma unroll
             for (int f = 0; f < NF; f++) x[f] = 0.0;
@@ -867,6 +960,13 @@ __global__ void __launch_bounds__(64) xt_kernel(AxisDesc ax, SweepCommon cm, SW 
 #pragma unroll
         for (int f = 0; f < NF; f++) xq[f][j] = x[f];
     }
+    const int li = lane / P, c = lane % P;
+    const bool work = li < nl;
+    const int lr = work ? li : 0;
+    const int s = c * K;
+    const bool first = c == 0, last = c == P - 1, whole = ch.whole(c);
+    const double* tab = SW::kFilter ? ax.ftab : ax.tab;
+    const bool cyc = SW::kFilter && ax.seam;
     if constexpr (SW::kStash > 0) {
         // lane-contiguous: no bank conflicts; each lane reads back only its own slots
 #pragma unroll
@@ -875,80 +975,94 @@ __global__ void __launch_bounds__(64) xt_kernel(AxisDesc ax, SweepCommon cm, SW 
             for (int j = 0; j < J; j++) stash[(f * J + j) * 64 + lane] = xq[f][j];
     }
 
-    // LDS slot of each of the lane's points (row and line tracked without division)
+    // LDS slot of each of the lane's points: chunk * (K+1) + row of the chunk;
+    // rows of whole chunks after the short ones, of the first, of the short ones
+    auto row_slot = [&](int row) {
+        const int a = row + ch.D, q = row - K;
+        const int cs = (q * 9363) >> 16;                         // q / 7, exact for q < 512
+        return EX || row < K || q >= (K - 1) * ch.D ? ((EX || row >= K ? a : row) >> 3) * (K + 1) + ((EX || row >= K ? a : row) & 7)
+                                                    : (cs + 1) * (K + 1) + (q - cs * (K - 1));
+    };
     int slot[J];
-    {
-        int l = 0, row = lane;
-        while (row >= N) { row -= N; l++; }
 #pragma unroll
-        for (int j = 0; j < J; j++) {
-            slot[j] = lane + 64 * j < npts ? xt_slot<K>(l, P, row / K, row % K) : 0;
-            row += 64;
-            while (row >= N) { row -= N; l++; }
+    for (int j = 0; j < J; j++) {
+        const int p = lane + 64 * j;
+        if (EX) {
+            slot[j] = (p >> 3) * (K + 1) + (p & 7);
+        } else {
+            // p / N by the reciprocal rounded up: exact for p < 512 <= 2^24 / N
+            const int l = (int)(((unsigned)p * ((0x1000000u + N - 1) / (unsigned)N)) >> 24);
+            slot[j] = xt_slot<K>(l, P, 0, 0) + row_slot(p - l * N);
         }
+        if (p >= npts) slot[j] = lpw * P * (K + 1) + lane;
     }
 
-    const int li = lane / GS, c = lane % GS;
-    const bool work = li < nl && c < P;
-    const int lr = li < nl ? li : 0;
-    const int cc = c < P ? c : P - 1;
-    const int s = cc * K;
-    const double* tab = SW::kFilter ? ax.ftab : ax.tab;
-    const uoff base = run + (uoff)lr * (uoff)N * st;
-    const bool cyc = SW::kFilter && ax.seam;
     // halo chunks: the neighbours, wrapped on a cyclic line (other lines clamp;
     // their values there are not used)
-    const int hl = cc > 0 ? cc - 1 : (cyc ? P - 1 : 0);
-    const int hr = cc + 1 < P ? cc + 1 : (cyc ? 0 : P - 1);
+    const int hl = c > 0 ? c - 1 : (cyc ? P - 1 : 0);
+    const int hr = c + 1 < P ? c + 1 : (cyc ? 0 : P - 1);
+    const int left = xt_slot<K>(lr, P, hl, K - H) - (ch.whole(hl) ? 0 : 1);
 
     double r[NF][K];
 #pragma unroll
     for (int f = 0; f < NF; f++) {
         __syncthreads();
 #pragma unroll
-        for (int j = 0; j < J; j++)
-            if (lane + 64 * j < npts) lds[slot[j]] = xq[f][j];
+        for (int j = 0; j < J; j++) lds[slot[j]] = xq[f][j];
         __syncthreads();
-        double w[1][W];
+        double w[W], right[H];
 #pragma unroll
         for (int u = 0; u < H; u++) {
-            w[0][u] = lds[xt_slot<K>(lr, P, hl, K - H + u)];
-            w[0][K + H + u] = lds[xt_slot<K>(lr, P, hr, u)];
+            w[u] = lds[left + u];
+            right[u] = lds[xt_slot<K>(lr, P, hr, u)];
         }
 #pragma unroll
-        for (int t = 0; t < K; t++) w[0][t + H] = lds[xt_slot<K>(lr, P, cc, t)];
-        double rf[1][K];
-        if constexpr (SW::kFilter)
-            filter_rhs<K, 1, W>(w, rf, s, N, cyc, ax.ftab + 6 * N + 8);
-        else
-            window_rhs<K, 1, W>(w, rf, K, work && c == 0 && !ax.seam, work && c == P - 1 && !ax.seam);
+        for (int t = 0; t < K; t++) w[t + H] = lds[xt_slot<K>(lr, P, c, t)];
+        close_window<K, H, W>(w, right, whole);
+        if constexpr (SW::kFilter) {
+            filter_rhs<K, W>(w, r[f], first && !cyc, last && !cyc, ax.ftab + 6 * NP + 8);
+        } else {
+            window_rhs<K, W>(w, r[f], first && !ax.seam, last && !ax.seam);
+            // both ends of the line are in the buffer; one pass serves the lanes of both
+            if (ax.seam && (first || last)) {
+                double rf[1][K];
 #pragma unroll
-        for (int t = 0; t < K; t++) r[f][t] = rf[0][t];
+                for (int t = 0; t < K; t++) rf[0][t] = r[f][t];
+                seam_rows<K, 1>([&](int end, int i, double* v) {
+                    v[0] = lds[end ? xt_slot<K>(lr, P, P - 1, K - 1 - i) : xt_slot<K>(lr, P, 0, i)];
+                }, first ? 0 : 1, K, cm.pb, rf);
+#pragma unroll
+                for (int t = 0; t < K; t++) r[f][t] = rf[0][t];
+            }
+        }
     }
-    if constexpr (!SW::kFilter)
-        if (work && ax.seam && (c == 0 || c == P - 1)) seam_rows<K, NF>(sw, base, st, N, K, c == 0, c == P - 1, cm.pb, r);
 
-    const bool cv = c < P;
+    constexpr int kReach = SW::kFilter ? 64 : 8;    // chunks (kCarryRows, rounded up to a power of two)
     double carry[NF], G[NF], X[NF];
-    forward_local<K, NF, true>(tab, N, s, K, r, carry);
-    scan_forward<NF>(cv ? tab[3 * N + s + K - 1] : 1.0, carry, cv, c, GS, G);
-    apply_carry<K, NF, true>(tab, 3 * N, s, K, r, G);
-    backward_local<K, NF, true>(tab, N, s, K, r, carry);
-    scan_backward<NF>(cv ? tab[4 * N + s] : 0.0, carry, cv, c, P, GS, X);
-    apply_carry<K, NF, true>(tab, 4 * N, s, K, r, X);
+    forward_local<K, NF>(tab, NP, s, r, carry);
+    scan_forward<NF>(tab[3 * NP + s + K - 1], carry, c, P, kReach, G);
+    apply_carry<K, NF>(tab, 3 * NP, s, r, G);
+    if constexpr (!EX) zero_padding<K, NF>(r, whole);
+    backward_local<K, NF>(tab, NP, s, r, carry);
+    scan_backward<NF>(tab[4 * NP + s], carry, c, P, kReach, X);
+    apply_carry<K, NF>(tab, 4 * NP, s, r, X);
     if (cyc) {
         double y0[NF], yN1[NF];
 #pragma unroll
         for (int f = 0; f < NF; f++) {
-            y0[f] = __shfl(r[f][0], 0, GS);
-            yN1[f] = __shfl(r[f][K - 1], P - 1, GS);
+            y0[f] = __shfl(r[f][0], lr * P);
+            yN1[f] = __shfl(r[f][K - 1], lr * P + P - 1);
         }
-        cyclic_correction<K, NF>(tab, N, s, y0, yN1, r);
+        cyclic_correction<K, NF>(tab, NP, s, y0, yN1, r);
     }
-    if (work) face_corrections<K, NF, SW, GCBC, true>(sw, base, st, N, s, K, c == 0, c == P - 1, r, cm.sbcc);
+    if constexpr (GCBC) {
+        if (work && (first || last)) {
+            const auto fc = sw.face_in(run + (uoff)(lr * N + (first ? 0 : N - 1)) * 8u, first ? 0 : 1, cm.sbcc);
+            face_correction<K, NF, SW>(sw, fc, first ? 0 : 1, K, r);
+        }
+    }
 
-    // back to the coalesced layout, one field at a time (the point values
-    // xq stay live only for a store that needs them)
+    // back to the coalesced layout, one field at a time
     double xo[NF][J];
 #pragma unroll
     for (int f = 0; f < NF; f++) {
@@ -963,22 +1077,22 @@ __global__ void __launch_bounds__(64) xt_kernel(AxisDesc ax, SweepCommon cm, SW 
     }
     double mm[2] = {0.0, 0.0};           // DtFold<SW>::close: the time step's maxima
     // every point's epilogue loads before the first store
+    if constexpr (SW::kAdds) {
 #pragma unroll
-    for (int j = 0; j < J; j++) {
-        const int p = lane + 64 * j;
-        if (p < npts) {
-            double d[NF];
+        for (int j = 0; j < J; j++) {
+            if (!SW::kBlocks || lane + 64 * j < npts) {
+                double d[NF];
 #pragma unroll
-            for (int f = 0; f < NF; f++) d[f] = xo[f][j];
-            sw.fetch(run + (uoff)p * st, d);
+                for (int f = 0; f < NF; f++) d[f] = xo[f][j];
+                add_out<NT>(sw, off(j), d);
 #pragma unroll
-            for (int f = 0; f < NF; f++) xo[f][j] = d[f];
+                for (int f = 0; f < NF; f++) xo[f][j] = d[f];
+            }
         }
     }
 #pragma unroll
     for (int j = 0; j < J; j++) {
-        const int p = lane + 64 * j;
-        if (p < npts) {
+        if (lane + 64 * j < npts) {
             double d[NF];
 #pragma unroll
             for (int f = 0; f < NF; f++) d[f] = xo[f][j];
@@ -986,13 +1100,10 @@ __global__ void __launch_bounds__(64) xt_kernel(AxisDesc ax, SweepCommon cm, SW 
                 double sv[SW::kStash > 0 ? SW::kStash : 1];
 #pragma unroll
                 for (int f = 0; f < SW::kStash; f++) sv[f] = stash[(f * J + j) * 64 + lane];
-                if constexpr (DtFold<SW>::close) sw.store_pv_dt(run + (uoff)p * st, d, sv, mm);
-                else sw.store_pv(run + (uoff)p * st, d, sv);
+                if constexpr (DtFold<SW>::close) sw.template store_pv_dt<NT>(off(j), d, sv, mm);
+                else sw.template store_pv<NT>(off(j), d, sv);
             } else {
-                double pv[NF];
-#pragma unroll
-                for (int f = 0; f < NF; f++) pv[f] = SW::kPv ? xq[f][j] : 0.0;
-                sw.store(run + (uoff)p * st, d, pv);
+                sw.template store<NT>(off(j), d);
             }
         }
     }
@@ -1011,118 +1122,6 @@ __global__ void __launch_bounds__(64) xt_kernel(AxisDesc ax, SweepCommon cm, SW 
 }
 
 // ---------------------------------------------------------------------------
-// variant "ragged": any line length; every chunk thread evaluates its rows and
-// halo rows itself (x lines: carries by shuffles; y/z: LDS folds)
-// ---------------------------------------------------------------------------
-template <int K, int AX, class SW, bool GCBC>
-__global__ void __launch_bounds__(AX == 0 ? 256 : kYLines * kMaxP) ragged_kernel(AxisDesc ax, SweepCommon cm, SW sw) {
-    constexpr int NF = SW::NF;
-    constexpr int W = K + 4;
-    extern __shared__ double lds[];
-
-    const int N = ax.N, P = ax.P;
-    int c, lloc = 0, GS = 1;
-    long line;
-    if (AX == 0) {
-        GS = ax.GS;
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-        const int lpw = 64 / GS;
-        c = lane % GS;
-        line = (long)blockIdx.x * (4 * lpw) + wave * lpw + lane / GS;
-    } else {
-        lloc = threadIdx.x % kYLines;
-        c = threadIdx.x / kYLines;
-        line = group_of(ax.xcd) * kYLines + lloc;
-    }
-    const bool act = line < ax.nlines;
-    const bool cv = c < P;
-    const bool work = act && cv;
-    const int s = cv ? (int)(((long)c * N) / P) : N;
-    const int L = cv ? (int)(((long)(c + 1) * N) / P) - s : 0;
-    const uoff st = (uoff)ax.st * 8u;
-    const uoff base = line_off(AX, act ? (uoff)line : 0u, (uoff)cm.lxi, (uoff)cm.plane);
-    const double* tab = ax.tab;
-
-    double r[NF][K];
-    double pv[SW::kPv ? NF : 1][K];
-    {
-        double w[NF][W];
-#pragma unroll
-        for (int u = 0; u < W; u++) {
-            const int row = s - 2 + u;
-            double x[NF];
-            if (work && u < L + 4 && row >= 0 && row < N) {
-                sw.point(base + (uoff)row * st, x);
-            } else {
-#pragma unroll
-                for (int f = 0; f < NF; f++) x[f] = 0.0;
-            }
-#pragma unroll
-            for (int f = 0; f < NF; f++) w[f][u] = x[f];
-        }
-        window_rhs<K, NF, W>(w, r, L, work && c == 0 && !ax.seam, work && c == P - 1 && !ax.seam);
-        if constexpr (SW::kPv) {
-#pragma unroll
-            for (int f = 0; f < NF; f++)
-#pragma unroll
-                for (int t = 0; t < K; t++) pv[f][t] = w[f][t + 2];
-        }
-    }
-    if (work && ax.seam && (c == 0 || c == P - 1)) seam_rows<K, NF>(sw, base, st, N, L, c == 0, c == P - 1, cm.pb, r);
-
-    double carry[NF], G[NF], X[NF];
-    forward_local<K, NF, false>(tab, N, s, L, r, carry);
-    if (AX == 0) {
-        scan_forward<NF>(cv ? tab[3 * N + s + L - 1] : 1.0, carry, cv, c, GS, G);
-    } else {
-        if (cv) {
-#pragma unroll
-            for (int f = 0; f < NF; f++) lds[(f * P + c) * kYLines + lloc] = carry[f];
-        }
-        __syncthreads();
-        fold_forward<NF, false, K>(lds, tab, N, P, kYLines, c, lloc, G);
-    }
-    apply_carry<K, NF, false>(tab, 3 * N, s, L, r, G);
-    backward_local<K, NF, false>(tab, N, s, L, r, carry);
-    if (AX == 0) {
-        scan_backward<NF>(cv ? tab[4 * N + s] : 0.0, carry, cv, c, P, GS, X);
-    } else {
-        double* xb = lds + NF * P * kYLines;
-        if (cv) {
-#pragma unroll
-            for (int f = 0; f < NF; f++) xb[(f * P + c) * kYLines + lloc] = carry[f];
-        }
-        __syncthreads();
-        fold_backward<NF, false, K>(xb, tab, N, P, kYLines, c, lloc, X);
-    }
-    apply_carry<K, NF, false>(tab, 4 * N, s, L, r, X);
-
-    if (!work) return;
-    face_corrections<K, NF, SW, GCBC, false>(sw, base, st, N, s, L, c == 0, c == P - 1, r, cm.sbcc);
-    // every row's epilogue loads before the first store
-#pragma unroll
-    for (int t = 0; t < K; t++) {
-        if (t < L) {
-            double d[NF];
-#pragma unroll
-            for (int f = 0; f < NF; f++) d[f] = r[f][t];
-            sw.fetch(base + (uoff)(s + t) * st, d);
-#pragma unroll
-            for (int f = 0; f < NF; f++) r[f][t] = d[f];
-        }
-    }
-#pragma unroll
-    for (int t = 0; t < K; t++) {
-        if (t < L) {
-            double d[NF], p[NF];
-#pragma unroll
-            for (int f = 0; f < NF; f++) { d[f] = r[f][t]; p[f] = SW::kPv ? pv[SW::kPv ? f : 0][t] : 0.0; }
-            sw.store(base + (uoff)(s + t) * st, d, p);
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------
 // variant "tile": the pointwise inputs of TL lines pass through an LDS tile
 // one row block (kCB chunks + halo) at a time with coalesced loads -- every
 // point is evaluated once -- and chunk threads stream their windows from the
@@ -1134,22 +1133,21 @@ constexpr int kCB = 8;   // chunks per row block
 template <int K>
 __host__ __device__ constexpr int tile_rows() { return kCB * K + 4; }
 
-template <int K, int AX, int TL, bool EX, class SW, bool GCBC>
+template <int K, int AX, int TL, class SW, bool GCBC>
 __global__ void __launch_bounds__(TL * kMaxP) tile_kernel(AxisDesc ax, SweepCommon cm, SW sw) {
     constexpr int NF = SW::NF;
     constexpr int TLP = TL + 1;
     constexpr int RB = tile_rows<K>();
     extern __shared__ double lds[];    // tile [NF][RB][TLP]
 
-    const int N = ax.N, P = ax.P;
+    const int N = ax.N, P = ax.P, NP = P * K;
     const int nthr = TL * P;
     const int tid = threadIdx.x;
     const int lloc = tid % TL, c = tid / TL;
     const long line0 = group_of(ax.xcd) * TL;
     const long line = line0 + lloc;
     const bool act = line < ax.nlines;
-    const int s = EX ? c * K : (int)(((long)c * N) / P);
-    const int L = EX ? K : (int)(((long)(c + 1) * N) / P) - s;
+    const int s = chunk_start(N, P, K, c), L = chunk_start(N, P, K, c + 1) - s;
     const uoff st = (uoff)ax.st * 8u;
     const uoff lxi = (uoff)cm.lxi, plane = (uoff)cm.plane;
     const uoff base = line_off(AX, act ? (uoff)line : 0u, lxi, plane);
@@ -1157,11 +1155,10 @@ __global__ void __launch_bounds__(TL * kMaxP) tile_kernel(AxisDesc ax, SweepComm
     const int nb = (P + kCB - 1) / kCB;
 
     double r[NF][K];
-    double pv[SW::kPv ? NF : 1][K];
     for (int b = 0; b < nb; b++) {
         const int c0 = b * kCB, c1 = min(P, c0 + kCB);
-        const int rs = max(0, (EX ? c0 * K : (int)(((long)c0 * N) / P)) - 2);
-        const int re = min(N, (EX ? c1 * K : (int)(((long)c1 * N) / P)) + 2);
+        const int rs = max(0, chunk_start(N, P, K, c0) - 2);
+        const int re = min(N, chunk_start(N, P, K, c1) + 2);
         const int nrows = re - rs;
         if (b > 0) __syncthreads();
         for (int p = tid; p < TL * nrows; p += nthr) {
@@ -1171,7 +1168,7 @@ __global__ void __launch_bounds__(TL * kMaxP) tile_kernel(AxisDesc ax, SweepComm
             const long ln = line0 + l;
             double x[NF];
             if (ln < ax.nlines) {
-                sw.point(line_off(AX, (uoff)ln, lxi, plane) + (uoff)row * st, x);
+                point<false>(sw, line_off(AX, (uoff)ln, lxi, plane) + (uoff)row * st, x);
             } else {
 #pragma unroll
                 for (int f = 0; f < NF; f++) x[f] = 0.0;
@@ -1183,62 +1180,64 @@ __global__ void __launch_bounds__(TL * kMaxP) tile_kernel(AxisDesc ax, SweepComm
         if (c >= c0 && c < c1) {
             auto row_of = [&](int u, double* x) {
                 const int row = s - 2 + u;
-                const bool in = (EX || u < L + 4) && row >= 0 && row < N;
+                const bool in = row >= 0 && row < N;
 #pragma unroll
                 for (int f = 0; f < NF; f++) x[f] = in ? lds[(f * RB + row - rs) * TLP + lloc] : 0.0;
             };
-            stream_rhs<K, NF>(row_of, r, L, c == 0 && !ax.seam, c == P - 1 && !ax.seam);
-            if constexpr (SW::kPv) {
-#pragma unroll
-                for (int t = 0; t < K; t++) {
-                    const int row = s + t;
-#pragma unroll
-                    for (int f = 0; f < NF; f++)
-                        pv[f][t] = (EX || t < L) ? lds[(f * RB + row - rs) * TLP + lloc] : 0.0;
-                }
-            }
+            stream_rhs<K, NF>(row_of, r, s, L, N, ax.seam);
         }
     }
-    if (act && ax.seam && (c == 0 || c == P - 1)) seam_rows<K, NF>(sw, base, st, N, L, c == 0, c == P - 1, cm.pb, r);
+    if (act && ax.seam && (c == 0 || c == P - 1))
+        seam_rows<K, NF>([&](int end, int i, double* v) { point<false>(sw, base + (uoff)(end ? N - 1 - i : i) * st, v); },
+                         c == 0 ? 0 : 1, L, cm.pb, r);
 
     double carry[NF], G[NF], X[NF];
-    forward_local<K, NF, EX>(tab, N, s, L, r, carry);
+    forward_local<K, NF>(tab, NP, c * K, r, carry);
     __syncthreads();                                   // tile reads done: reuse for carries
 #pragma unroll
     for (int f = 0; f < NF; f++) lds[(f * P + c) * TL + lloc] = carry[f];
     __syncthreads();
-    fold_forward<NF, EX, K>(lds, tab, N, P, TL, c, lloc, G);
-    apply_carry<K, NF, EX>(tab, 3 * N, s, L, r, G);
-    backward_local<K, NF, EX>(tab, N, s, L, r, carry);
+    fold_forward<NF, K, false>(lds, tab, NP, P, TL, c, lloc, G);
+    apply_carry<K, NF>(tab, 3 * NP, c * K, r, G);
+#pragma unroll
+    for (int t = 1; t < K; t++)
+#pragma unroll
+        for (int f = 0; f < NF; f++) r[f][t] = t < L ? r[f][t] : 0.0;
+    backward_local<K, NF>(tab, NP, c * K, r, carry);
     double* xb = lds + NF * P * TL;
 #pragma unroll
     for (int f = 0; f < NF; f++) xb[(f * P + c) * TL + lloc] = carry[f];
     __syncthreads();
-    fold_backward<NF, EX, K>(xb, tab, N, P, TL, c, lloc, X);
-    apply_carry<K, NF, EX>(tab, 4 * N, s, L, r, X);
+    fold_backward<NF, K, false>(xb, tab, NP, P, TL, c, lloc, X);
+    apply_carry<K, NF>(tab, 4 * NP, c * K, r, X);
 
-    if (act) face_corrections<K, NF, SW, GCBC, EX>(sw, base, st, N, s, L, c == 0, c == P - 1, r, cm.sbcc);
+    if constexpr (GCBC) {
+        if (act && (c == 0 || c == P - 1)) {
+            const auto fc = sw.face_in(base + (uoff)(c == 0 ? 0 : N - 1) * st, c == 0 ? 0 : 1, cm.sbcc);
+            face_correction<K, NF, SW>(sw, fc, c == 0 ? 0 : 1, L, r);
+        }
+    }
 
-    if (AX != 0 || SW::kPv) {             // (stores needing the point values stay per thread)
+    if (AX != 0) {
         if (!act) return;
 #pragma unroll
         for (int t = 0; t < K; t++) {
-            if (EX || t < L) {
+            if (t < L) {
                 double d[NF];
 #pragma unroll
                 for (int f = 0; f < NF; f++) d[f] = r[f][t];
-                sw.fetch(base + (uoff)(s + t) * st, d);
+                add_out<false>(sw, base + (uoff)(s + t) * st, d);
 #pragma unroll
                 for (int f = 0; f < NF; f++) r[f][t] = d[f];
             }
         }
 #pragma unroll
         for (int t = 0; t < K; t++) {
-            if (EX || t < L) {
-                double d[NF], p[NF];
+            if (t < L) {
+                double d[NF];
 #pragma unroll
-                for (int f = 0; f < NF; f++) { d[f] = r[f][t]; p[f] = SW::kPv ? pv[SW::kPv ? f : 0][t] : 0.0; }
-                sw.store(base + (uoff)(s + t) * st, d, p);
+                for (int f = 0; f < NF; f++) d[f] = r[f][t];
+                sw.template store<false>(base + (uoff)(s + t) * st, d);
             }
         }
         return;
@@ -1246,14 +1245,14 @@ __global__ void __launch_bounds__(TL * kMaxP) tile_kernel(AxisDesc ax, SweepComm
     // x lines: results back through the tile, one row block at a time, stored along the line
     for (int b = 0; b < nb; b++) {
         const int c0 = b * kCB, c1 = min(P, c0 + kCB);
-        const int rs = EX ? c0 * K : (int)(((long)c0 * N) / P);
-        const int re = EX ? c1 * K : (int)(((long)c1 * N) / P);
+        const int rs = chunk_start(N, P, K, c0);
+        const int re = chunk_start(N, P, K, c1);
         const int nrows = re - rs;
         __syncthreads();
         if (c >= c0 && c < c1) {
 #pragma unroll
             for (int t = 0; t < K; t++)
-                if (EX || t < L)
+                if (t < L)
 #pragma unroll
                     for (int f = 0; f < NF; f++) lds[(f * RB + s + t - rs) * TLP + lloc] = r[f][t];
         }
@@ -1262,12 +1261,12 @@ __global__ void __launch_bounds__(TL * kMaxP) tile_kernel(AxisDesc ax, SweepComm
             const int l = p / nrows, row = rs + p % nrows;
             const long ln = line0 + l;
             if (ln >= ax.nlines) continue;
-            double d[NF], pz[NF];
+            double d[NF];
 #pragma unroll
-            for (int f = 0; f < NF; f++) { d[f] = lds[(f * RB + row - rs) * TLP + l]; pz[f] = 0.0; }
+            for (int f = 0; f < NF; f++) d[f] = lds[(f * RB + row - rs) * TLP + l];
             const uoff bo = line_off(AX, (uoff)ln, lxi, plane) + (uoff)row * st;
-            sw.fetch(bo, d);
-            sw.store(bo, d, pz);
+            add_out<false>(sw, bo, d);
+            sw.template store<false>(bo, d);
         }
     }
 }
@@ -1275,118 +1274,135 @@ __global__ void __launch_bounds__(TL * kMaxP) tile_kernel(AxisDesc ax, SweepComm
 // ---------------------------------------------------------------------------
 // launch
 // ---------------------------------------------------------------------------
+// the descriptor a launch of `groups` workgroups runs with: its xcd field
+// becomes the run length code of group_of, runs of at most `most` groups
+inline AxisDesc with_runs(const AxisDesc& ax, long groups, bool on, int most) {
+    AxisDesc a = ax;
+    a.xcd = 0;
+    if (on) {
+        a.xcd = 1;
+        while ((2L << (a.xcd - 1)) <= most && (16L << (a.xcd - 1)) <= groups) a.xcd++;
+    }
+    return a;
+}
+
+// Streaming hints pay once a sweep passes over more than the 256 MB of the
+// last-level cache (below, the next sweep finds there what this one wrote:
+// 128^3 S2y 60 us without them against 71 with; above, 256^3 S2z 455 against
+// 526), and only where a row access covers whole cache lines: with rows off
+// the 128-byte grid a line is shared by two workgroups (201x160x176: S2y 323
+// against 366 us, S1x 214 against 243).  x lines are one run of memory, of
+// which only the ends are shared; rows of 16 bytes already pay there.
+template <class SW>
+static bool streams(const AxisDesc& ax, const SweepCommon& cm) {
+    const int align = ax.st == 1 ? 2 : 16;
+    return cm.lxi % align == 0 && (double)SW::kBytes * (double)ax.N * (double)ax.nlines > 256.0 * (1 << 20);
+}
+
+template <int K, class SW, bool GCBC>
+static const void* xt_symbol(bool exact, bool nt) {
+    if (exact) return nt ? (const void*)xt_kernel<K, SW, GCBC, true, true> : (const void*)xt_kernel<K, SW, GCBC, true, false>;
+    return nt ? (const void*)xt_kernel<K, SW, GCBC, false, true> : (const void*)xt_kernel<K, SW, GCBC, false, false>;
+}
+
+// 8 lines a workgroup are 64-byte rows: never streamed
 template <int K, int AX, class SW, bool GCBC>
-static int launch_sweep(const AxisDesc& ax, const SweepCommon& cm, const SW& sw, hipStream_t s) {
-    constexpr int NF = SW::NF;
-    const bool exact = ax.N == ax.P * K;
-    if constexpr (K == 8) {
-        if (ax.variant == 1) {
-            const size_t tile = (size_t)NF * tile_rows<K>() * (ax.tl + 1);
-            const size_t carries = (size_t)2 * NF * ax.P * ax.tl;
-            const size_t lds = sizeof(double) * (tile > carries ? tile : carries);
-            dim3 block(ax.tl * ax.P), grid((unsigned)((ax.nlines + ax.tl - 1) / ax.tl));
-            if (exact) {
-                if (ax.tl == 8) hipLaunchKernelGGL((tile_kernel<K, AX, 8, true, SW, GCBC>), grid, block, lds, s, ax, cm, sw);
-                else hipLaunchKernelGGL((tile_kernel<K, AX, 16, true, SW, GCBC>), grid, block, lds, s, ax, cm, sw);
-            } else {
-                if (ax.tl == 8) hipLaunchKernelGGL((tile_kernel<K, AX, 8, false, SW, GCBC>), grid, block, lds, s, ax, cm, sw);
-                else hipLaunchKernelGGL((tile_kernel<K, AX, 16, false, SW, GCBC>), grid, block, lds, s, ax, cm, sw);
-            }
-            CS_HIP(hipGetLastError());
-            return CS_OK;
-        }
-    }
-    if constexpr (K == 8 && AX == 0) {
-        if (exact) {
-            const int lpw = 64 / ax.GS;
-            const size_t lds = sizeof(double) * (lpw * ax.P * (K + 1) + SW::kStash * K * 64);
-            dim3 block(64), grid((unsigned)((ax.nlines + lpw - 1) / lpw));
-            hipLaunchKernelGGL((xt_kernel<K, SW, GCBC>), grid, block, lds, s, ax, cm, sw);
-            CS_HIP(hipGetLastError());
-            return CS_OK;
-        }
-    }
-    if (exact) {
-        dim3 block, grid;
-        size_t lds = 0;
-        const int TL = ax.tl == 8 ? 8 : 16;
-        if (AX == 0) {
-            const int lpb = 4 * (64 / ax.GS);
-            block = dim3(256);
-            grid = dim3((unsigned)((ax.nlines + lpb - 1) / lpb));
-        } else {
-            block = dim3(TL * ax.P);
-            grid = dim3((unsigned)((ax.nlines + TL - 1) / TL));
-            lds = sizeof(double) * 4 * NF * ax.P * TL;
-            if (lds > 65536) {
-                const void* k = TL == 8 ? (const void*)direct_kernel<K, AX, 8, SW, GCBC>
-                                        : (const void*)direct_kernel<K, AX, 16, SW, GCBC>;
-                CS_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-            }
-        }
-        if (AX != 0 && TL == 8)
-            hipLaunchKernelGGL((direct_kernel<K, AX, 8, SW, GCBC>), grid, block, lds, s, ax, cm, sw);
-        else
-            hipLaunchKernelGGL((direct_kernel<K, AX, 16, SW, GCBC>), grid, block, lds, s, ax, cm, sw);
-        CS_HIP(hipGetLastError());
-        return CS_OK;
-    }
-    dim3 block, grid;
-    size_t lds = 0;
-    if (AX == 0) {
-        const int lpb = 4 * (64 / ax.GS);
-        block = dim3(256);
-        grid = dim3((unsigned)((ax.nlines + lpb - 1) / lpb));
-    } else {
-        block = dim3(kYLines * ax.P);
-        grid = dim3((unsigned)((ax.nlines + kYLines - 1) / kYLines));
-        lds = sizeof(double) * 2 * NF * ax.P * kYLines;
-    }
-    hipLaunchKernelGGL((ragged_kernel<K, AX, SW, GCBC>), grid, block, lds, s, ax, cm, sw);
-    CS_HIP(hipGetLastError());
+static const void* direct_symbol(int TL, bool exact, bool nt) {
+    if (TL == 8) return exact ? (const void*)direct_kernel<K, AX, 8, SW, GCBC, true, false>
+                              : (const void*)direct_kernel<K, AX, 8, SW, GCBC, false, false>;
+    if (exact) return nt ? (const void*)direct_kernel<K, AX, 16, SW, GCBC, true, true>
+                         : (const void*)direct_kernel<K, AX, 16, SW, GCBC, true, false>;
+    return nt ? (const void*)direct_kernel<K, AX, 16, SW, GCBC, false, true>
+              : (const void*)direct_kernel<K, AX, 16, SW, GCBC, false, false>;
+}
+
+template <class SW>
+static int launch(const void* k, dim3 grid, dim3 block, size_t lds, AxisDesc a, SweepCommon cm, SW sw, hipStream_t s) {
+    if (lds > 65536) CS_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    void* args[] = {&a, &cm, &sw};
+    CS_HIP(hipLaunchKernel(k, grid, block, args, lds, s));
     return CS_OK;
 }
 
-// the filter sweep on equal chunks of K points (8 along x; 8 or 16 along y/z,
-// the axis's filter descriptor); SW = SF<AX> (five variables per workgroup)
+// x sweeps: a workgroup is the 64/P lines of one wave, runs of 64 an XCD
+// (measured 4.8 -> 5.3 TB/s for a copy of that shape)
+template <class SW, bool GCBC>
+static int launch_x(const AxisDesc& ax, const SweepCommon& cm, const SW& sw, unsigned gy, hipStream_t s) {
+    constexpr int K = 8;
+    const int lpw = 64 / ax.P;
+    const size_t lds = sizeof(double) * (lpw * ax.P * (K + 1) + 64 + SW::kStash * K * 64);
+    const dim3 grid((unsigned)((ax.nlines + lpw - 1) / lpw), gy);
+    return launch(xt_symbol<K, SW, GCBC>(ax.N == ax.P * K, streams<SW>(ax, cm)), grid, dim3(64), lds,
+                  with_runs(ax, grid.x, true, 64), cm, sw, s);
+}
+
+// y/z sweeps: TL lines a workgroup; along y runs of 128 neighbouring lines an
+// XCD, along z of 1024 (256^3: S1y 240 -> 216, S2y 529 -> 485, S2z 488 -> 440,
+// S1z 318 -> 279 us against plain order)
+template <int K, int AX, class SW, bool GCBC>
+static int launch_yz(const AxisDesc& ax, const SweepCommon& cm, const SW& sw, int TL, bool runs, size_t lds,
+                     unsigned gy, hipStream_t s) {
+    const dim3 grid((unsigned)((ax.nlines + TL - 1) / TL), gy);
+    return launch(direct_symbol<K, AX, SW, GCBC>(TL, ax.N == ax.P * K, streams<SW>(ax, cm)), grid, dim3(TL * ax.P),
+                  lds, with_runs(ax, grid.x, runs, (AX == 1 ? 128 : 1024) / TL), cm, sw, s);
+}
+
+template <int K, int AX, class SW, bool GCBC>
+static int launch_sweep(const AxisDesc& ax, const SweepCommon& cm, const SW& sw, hipStream_t s) {
+    constexpr int NF = SW::NF;
+    if constexpr (K == 8) {
+        // the tiles take any chunk lengths
+        if (ax.variant == 1 || !chunks_fit(ax.N, ax.P, K)) {
+            const size_t tile = (size_t)NF * tile_rows<K>() * (ax.tl + 1);
+            const size_t carries = (size_t)2 * NF * ax.P * ax.tl;
+            const size_t lds = sizeof(double) * (tile > carries ? tile : carries);
+            const dim3 grid((unsigned)((ax.nlines + ax.tl - 1) / ax.tl));
+            return launch(ax.tl == 8 ? (const void*)tile_kernel<K, AX, 8, SW, GCBC>
+                                     : (const void*)tile_kernel<K, AX, 16, SW, GCBC>,
+                          grid, dim3(ax.tl * ax.P), lds, with_runs(ax, grid.x, ax.xcd, 64), cm, sw, s);
+        }
+    }
+    if constexpr (AX == 0) {
+        static_assert(K == 8, "x lines run 8-point chunks");
+        return launch_x<SW, GCBC>(ax, cm, sw, 1u, s);
+    } else {
+        const int TL = ax.tl == 8 ? 8 : 16;
+        const size_t lds = sizeof(double) * NF * TL * (2 * SW::kH * ax.P + (ax.seam ? 2 * kLmd : 0));
+        return launch_yz<K, AX, SW, GCBC>(ax, cm, sw, TL, ax.xcd != 0, lds, 1u, s);
+    }
+}
+
+// the filter sweep on chunks of K points (8 along x; 8 or 16 along y/z, the
+// axis's filter descriptor); SW = SF<AX> (five variables per workgroup)
 // or SF1<AX> (one variable per workgroup, grid.y = 5)
 template <int K, int AX, class SW>
 static int launch_filter(const AxisDesc& ax, const SweepCommon& cm, const SW& sw, hipStream_t s) {
     constexpr int NF = SW::NF, H = SW::kH;
     static_assert(AX != 0 || K == 8, "x filter sweeps run 8-point chunks");
     const unsigned gy = NF == 1 ? 5u : 1u;
-    if (ax.K != K || ax.N != ax.P * K || !ax.ftab) return fail(CS_ERR_STATE, "fused filter needs equal chunks");
+    if (ax.K != K || !ax.ftab) return fail(CS_ERR_STATE, "fused filter without its table");
     if constexpr (AX == 0) {
-        const int lpw = 64 / ax.GS;
-        const size_t lds = sizeof(double) * lpw * ax.P * (K + 1);
-        dim3 block(64), grid((unsigned)((ax.nlines + lpw - 1) / lpw), gy);
-        hipLaunchKernelGGL((xt_kernel<K, SW, false>), grid, block, lds, s, ax, cm, sw);
+        return launch_x<SW, false>(ax, cm, sw, gy, s);
     } else {
         const int TL = ax.ftl == 8 ? 8 : 16;
         const size_t halo = (size_t)2 * H * ax.P * TL;
         const size_t carries = (size_t)2 * NF * ax.P * TL + 2 * NF * TL;
-        const size_t lds = sizeof(double) * (halo > carries ? halo : carries);
-        dim3 block(TL * ax.P), grid((unsigned)((ax.nlines + TL - 1) / TL), gy);
-        const void* k = TL == 8 ? (const void*)direct_kernel<K, AX, 8, SW, false>
-                                : (const void*)direct_kernel<K, AX, 16, SW, false>;
-        if (lds > 65536) CS_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        if (TL == 8) hipLaunchKernelGGL((direct_kernel<K, AX, 8, SW, false>), grid, block, lds, s, ax, cm, sw);
-        else hipLaunchKernelGGL((direct_kernel<K, AX, 16, SW, false>), grid, block, lds, s, ax, cm, sw);
+        return launch_yz<K, AX, SW, false>(ax, cm, sw, TL, true, sizeof(double) * (halo > carries ? halo : carries),
+                                           gy, s);
     }
-    CS_HIP(hipGetLastError());
-    return CS_OK;
 }
 
 template <int AX, class SW>
 static int dispatch(const AxisDesc& ax, const SweepCommon& cm, const SW& sw, hipStream_t s) {
-    if constexpr (SW::kGcbc) {
-        if (ax.K == 8) {
+    if constexpr (AX == 0) {
+        if constexpr (SW::kGcbc)
             if (ax.gcbc) return launch_sweep<8, AX, SW, true>(ax, cm, sw, s);
-            return launch_sweep<8, AX, SW, false>(ax, cm, sw, s);
-        }
-        if (ax.gcbc) return launch_sweep<16, AX, SW, true>(ax, cm, sw, s);
-        return launch_sweep<16, AX, SW, false>(ax, cm, sw, s);
+        return launch_sweep<8, AX, SW, false>(ax, cm, sw, s);
     } else {
+        if constexpr (SW::kGcbc) {
+            if (ax.gcbc && ax.K == 8) return launch_sweep<8, AX, SW, true>(ax, cm, sw, s);
+            if (ax.gcbc) return launch_sweep<16, AX, SW, true>(ax, cm, sw, s);
+        }
         if (ax.K == 8) return launch_sweep<8, AX, SW, false>(ax, cm, sw, s);
         return launch_sweep<16, AX, SW, false>(ax, cm, sw, s);
     }

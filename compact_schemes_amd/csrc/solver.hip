@@ -13,38 +13,42 @@
 namespace cs {
 namespace fused {
 
-// Derivative operator of one axis with balanced chunks (the table layout of
-// the line solver; closure rows for 0, seam rows for 1).
-int build_axis_table(int n, int seam, int K, int P, std::vector<double>& h) {
-    (void)K;
-    h.assign(5 * (size_t)n, 0.0);
-    std::vector<double> a(n, kAlpha), b(n, 1.0), c(n, kAlpha);
-    if (!seam) { a[0] = 0; c[0] = kAlpha01; a[1] = kAlpha10; c[1] = kAlpha10; }
-    else       { a[0] = 0; c[0] = kAlpha; }
-    if (!seam) { a[n - 1] = kAlpha01; c[n - 1] = 0; a[n - 2] = kAlpha10; c[n - 2] = kAlpha10; }
-    else       { a[n - 1] = kAlpha; c[n - 1] = 0; }
-    double* nu = &h[0];
-    double* mu = &h[n];
-    double* rho = &h[2 * (size_t)n];
-    double* Mf = &h[3 * (size_t)n];
-    double* Rb = &h[4 * (size_t)n];
-    double cp_prev = 0.0;
-    for (int i = 0; i < n; i++) {
-        double w = 1.0 / (b[i] - (i > 0 ? a[i] * cp_prev : 0.0));
-        nu[i] = w;
-        mu[i] = (i > 0) ? -a[i] * w : 0.0;
-        double cp = c[i] * w;
-        rho[i] = -cp;
-        cp_prev = cp;
-    }
-    rho[n - 1] = 0.0;
-    for (int ch = 0; ch < P; ch++) {
-        int s = (int)(((long)ch * n) / P), e = (int)(((long)(ch + 1) * n) / P) - 1;
+// A line operator's factors h (build_line_table's rows of n: nu, mu, rho and,
+// for a filter, z, then the scalars of a cyclic solve and the stencil
+// coefficients) laid out for chunks of K rows: [6][P*K] nu, mu, rho, Mf, Rb, z
+// and the 44 scalars.  Row t of chunk c is at c*K + t.  A padding row hands
+// the forward carry on (mu = 1), takes no right-hand side (nu = 0) and, set to
+// zero by the kernel before the backward recurrence, hands that carry on too
+// (rho = 1).
+void chunk_table(const std::vector<double>& h, int n, int K, int P, std::vector<double>& out) {
+    const size_t NP = (size_t)P * K;
+    out.assign(6 * NP + 44, 0.0);
+    for (int c = 0; c < P; c++) {
+        const int s = chunk_start(n, P, K, c), L = chunk_start(n, P, K, c + 1) - s;
+        const size_t o = (size_t)c * K;
+        for (int t = 0; t < K; t++) {
+            const bool row = t < L;
+            out[o + t] = row ? h[s + t] : 0.0;
+            out[NP + o + t] = row ? h[n + s + t] : 1.0;
+            out[2 * NP + o + t] = row ? h[2 * (size_t)n + s + t] : 1.0;
+            out[5 * NP + o + t] = row ? h[5 * (size_t)n + s + t] : 0.0;
+        }
         double p = 1.0;
-        for (int j = s; j <= e; j++) { p *= mu[j]; Mf[j] = p; }
+        for (int t = 0; t < K; t++) { p *= out[NP + o + t]; out[3 * NP + o + t] = p; }
         p = 1.0;
-        for (int j = e; j >= s; j--) { p *= rho[j]; Rb[j] = p; }
+        for (int t = K - 1; t >= 0; t--) { p *= out[2 * NP + o + t]; out[4 * NP + o + t] = p; }
     }
+    for (int i = 0; i < 44; i++) out[6 * NP + i] = h[6 * (size_t)n + i];
+}
+
+// device table of operator `op` along an axis of n rows, chunks of K rows
+static int upload_table(int op, int n, int seam, double af, int K, int P, double** dev) {
+    std::vector<double> h, t;
+    const int rc = build_line_table(op, n, seam, seam, af, K, h);
+    if (rc) return rc;
+    chunk_table(h, n, K, P, t);
+    CS_HIP(hipMalloc(dev, t.size() * sizeof(double)));
+    CS_HIP(hipMemcpy(*dev, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice));
     return CS_OK;
 }
 
@@ -129,24 +133,31 @@ int cs_solver_destroy(cs_solver* sv) {
     return CS_OK;
 }
 
-// the right-hand-side sweeps of `axis` on 16-point chunks (lines of 32..256
-// points, a multiple of 16); the filter and adjoint sweeps keep 8-point chunks
-static int use_chunks16(cs_solver* sv, int axis, int lines, int xcd) {
-    const AxisDesc& ax = sv->ax[axis];
+// y or z lines that 16-point chunks can cut (whole first and last chunks)
+static bool fits16(const AxisDesc& ax, int axis) {
+    return axis > 0 && ax.K == 8 && ax.N >= 32 && chunks_fit(ax.N, (ax.N + 15) / 16, 16);
+}
+
+// the shapes cs_solver_tune offers on 16-point chunks: equal ones
+static int check_chunks16(const AxisDesc& ax, int axis) {
     if (axis == 0 || ax.K != 8 || ax.N % 16 != 0 || ax.N < 32)
         return fail(CS_ERR_UNSUPPORTED, "16-point chunks: y or z lines of 32..256 points, a multiple of 16");
+    return CS_OK;
+}
+
+// the right-hand-side sweeps of `axis` on 16-point chunks; the adjoint sweeps
+// keep 8-point chunks
+static int use_chunks16(cs_solver* sv, int axis, int lines, int xcd) {
+    const AxisDesc& ax = sv->ax[axis];
+    if (!fits16(ax, axis)) return fail(CS_ERR_UNSUPPORTED, "16-point chunks do not cut this line");
     if (!sv->tabs16[axis]) {
-        std::vector<double> h;
-        int rc = build_axis_table(ax.N, ax.seam, 16, ax.N / 16, h);
+        const int rc = upload_table(OP_DERIV, ax.N, ax.seam, sv->cfg.alpha_f, 16, (ax.N + 15) / 16,
+                                    &sv->tabs16[axis]);
         if (rc) return rc;
-        CS_HIP(hipMalloc(&sv->tabs16[axis], h.size() * sizeof(double)));
-        CS_HIP(hipMemcpy(sv->tabs16[axis], h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice));
     }
     AxisDesc r = ax;
     r.K = 16;
-    r.P = ax.N / 16;
-    r.GS = 1;
-    while (r.GS < r.P) r.GS <<= 1;
+    r.P = (ax.N + 15) / 16;
     r.tab = sv->tabs16[axis];
     r.variant = 2;
     r.tl = lines;
@@ -165,19 +176,14 @@ static int filter_chunks(cs_solver* sv, int axis, int chunk) {
     if (chunk != ax.K && (ax.K != 8 || axis == 0))
         return fail(CS_ERR_UNSUPPORTED, "this axis's filter sweep runs " + std::to_string(ax.K) + "-point chunks");
     if (chunk == 16 && ax.K == 8) {
-        if (!ax.ftab || ax.N % 16 != 0 || ax.N < 32)
-            return fail(CS_ERR_UNSUPPORTED, "16-point filter chunks: y or z lines of 32..256 points, a multiple of 16");
+        if (!ax.ftab || !fits16(ax, axis)) return fail(CS_ERR_UNSUPPORTED, "16-point chunks do not cut this line");
         if (!sv->ftabs16[axis]) {
-            std::vector<double> hf;
-            int rc = build_line_table(OP_FILTER, ax.N, ax.seam, ax.seam, sv->cfg.alpha_f, 16, hf);
+            const int rc = upload_table(OP_FILTER, ax.N, ax.seam, sv->cfg.alpha_f, 16, (ax.N + 15) / 16,
+                                        &sv->ftabs16[axis]);
             if (rc) return rc;
-            CS_HIP(hipMalloc(&sv->ftabs16[axis], hf.size() * sizeof(double)));
-            CS_HIP(hipMemcpy(sv->ftabs16[axis], hf.data(), hf.size() * sizeof(double), hipMemcpyHostToDevice));
         }
         f.K = 16;
-        f.P = ax.N / 16;
-        f.GS = 1;
-        while (f.GS < f.P) f.GS <<= 1;
+        f.P = (ax.N + 15) / 16;
         f.ftab = sv->ftabs16[axis];
     }
     sv->fax[axis] = f;
@@ -212,66 +218,55 @@ int cs_solver_create(const cs_solver_config* cfg, cs_solver** out) {
     for (int a = 0; a < 3; a++) {
         AxisDesc& ax = sv->ax[a];
         ax.N = g.n(a);
-        // 8-point chunks up to 256 points, and along x up to 512 when they are
-        // equal (one line per wave of the transposing x kernel, 64 chunks);
-        // 16-point chunks otherwise
-        ax.K = (ax.N <= 256 || (a == 0 && ax.N % 8 == 0)) ? 8 : 16;
+        // 8-point chunks along x (one wave of the transposing x kernel holds 64
+        // of them) and up to 256 points, 16-point chunks otherwise
+        ax.K = a == 0 || ax.N <= 256 ? 8 : 16;
         ax.P = (ax.N + ax.K - 1) / ax.K;
-        ax.GS = 1;
-        while (ax.GS < ax.P) ax.GS <<= 1;
         ax.nlines = g.face_size(a);
         ax.st = g.stride(a);
         ax.seam = seam[a];
         ax.gcbc = gc[a];
-        // measured defaults (256^3, MI355X): x lines run the one-wave transposing
-        // kernel; y and z lines 16 per workgroup, y with XCD-grouped workgroups
+        // x lines run the one-wave transposing kernel, y and z lines 16 per
+        // workgroup, neighbouring workgroups on one XCD
         ax.variant = 0;
         ax.tl = 16;
-        ax.xcd = a == 1 ? 1 : 0;
+        ax.xcd = a > 0 ? 1 : 0;
         // filter sweeps: x all five variables per wave, y/z one per workgroup
         ax.ffields = a == 0 ? 5 : 1;
         ax.ftl = 16;
-        std::vector<double> h;
-        build_axis_table(ax.N, ax.seam, ax.K, ax.P, h);
-        if (hipMalloc(&sv->tabs[a], h.size() * sizeof(double)) != hipSuccess ||
-            hipMemcpy(sv->tabs[a], h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess) {
+        if ((rc = upload_table(OP_DERIV, ax.N, ax.seam, cfg->alpha_f, ax.K, ax.P, &sv->tabs[a]))) {
+            std::string msg = cs_last_error();
             cs_solver_destroy(sv);
-            return fail(CS_ERR_HIP, "operator table upload failed");
+            return fail(rc, msg);
         }
         ax.tab = sv->tabs[a];
         ax.ftab = nullptr;
-        if (cfg->filter && ax.N == ax.P * ax.K && (a == 0 ? ax.K == 8 : ax.P <= kMaxP)) {
-            // the filter of the five variables in one sweep per axis (equal chunks)
-            std::vector<double> hf;
-            const int sp = ax.seam;
-            if ((rc = build_line_table(OP_FILTER, ax.N, sp, sp, cfg->alpha_f, ax.K, hf))) {
+        if (cfg->filter && chunks_fit(ax.N, ax.P, ax.K)) {
+            // the filter of the five variables in one sweep per axis
+            if ((rc = upload_table(OP_FILTER, ax.N, ax.seam, cfg->alpha_f, ax.K, ax.P, &sv->ftabs[a]))) {
+                std::string msg = cs_last_error();
                 cs_solver_destroy(sv);
-                return rc;
-            }
-            if (hipMalloc(&sv->ftabs[a], hf.size() * sizeof(double)) != hipSuccess ||
-                hipMemcpy(sv->ftabs[a], hf.data(), hf.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess) {
-                cs_solver_destroy(sv);
-                return fail(CS_ERR_HIP, "filter table upload failed");
+                return fail(rc, msg);
             }
             ax.ftab = sv->ftabs[a];
         }
     }
     for (int a = 0; a < 3; a++) sv->rax[a] = sv->fax[a] = sv->ax[a];
-    // measured default (256^3, MI355X): the y and z filter sweeps run 16-point chunks
-    for (int a = 1; a < 3 && cfg->filter; a++)
-        if (sv->ax[a].ftab && sv->ax[a].K == 8 && sv->ax[a].N % 16 == 0 && sv->ax[a].N >= 32 &&
-            (rc = filter_chunks(sv, a, 16))) {
+    // y and z lines that 16-point chunks can cut run on them: half the chunk
+    // carries and halo rows, two 4-wave workgroups a CU (256^3, 8- against
+    // 16-point chunks: S1y 262 -> 216, S2y 498 -> 482, S1z 290 -> 275, S2z 471 ->
+    // 431, filter y 376 -> 344, filter z 420 -> 371 us)
+    for (int a = 1; a < 3; a++) {
+        rc = CS_OK;
+        if (fits16(sv->ax[a], a)) {
+            if (sv->ax[a].ftab) rc = filter_chunks(sv, a, 16);
+            if (!rc) rc = use_chunks16(sv, a, 16, 1);
+        }
+        if (rc) {
             std::string msg = cs_last_error();
             cs_solver_destroy(sv);
             return fail(rc, msg);
         }
-    // measured default (256^3, MI355X): z lines of up to 256 points run the
-    // right-hand-side sweeps on 16-point chunks (S1z 0.345 -> 0.305 ms, S2z
-    // 0.525 -> 0.518 ms; y lines measured the same or slower)
-    if (sv->ax[2].K == 8 && sv->ax[2].N % 16 == 0 && sv->ax[2].N >= 32 && (rc = use_chunks16(sv, 2, 16, 0))) {
-        std::string msg = cs_last_error();
-        cs_solver_destroy(sv);
-        return fail(rc, msg);
     }
     sv->red_blocks = (int)std::min<long>(2048, (lmx + 255) / 256);
     bool ok = hipMalloc(&sv->dpart, sizeof(double) * 5 * lmx) == hipSuccess &&
@@ -339,7 +334,7 @@ static int sweep_shape(cs_solver* sv, int axis, int variant, int lines, int xcd)
 static int filter_shape(cs_solver* sv, int axis, int fields, int lines, int chunk) {
     if ((fields != 1 && fields != 5) || (lines != 8 && lines != 16) || (chunk != 8 && chunk != 16))
         return fail(CS_ERR_ARG, "fields 1/5, lines 8/16, chunk 8/16");
-    if (!filter_axis_fused(sv, axis)) return fail(CS_ERR_UNSUPPORTED, "the filter of this axis has no fused sweep");
+    if (!filter_axis_tunable(sv, axis)) return fail(CS_ERR_UNSUPPORTED, "this axis does not split into equal chunks");
     int rc = filter_chunks(sv, axis, chunk);
     if (rc) return rc;
     sv->ax[axis].ffields = sv->fax[axis].ffields = fields;
@@ -361,15 +356,19 @@ static void apply_tuned(cs_solver* sv, bool filters) {
         ax.xcd = d[5];
         int v[3];
         if (!tuned_sweep(a, ax.N, ax.seam, sv->cfg.viscous ? sv->prec : 0, sv->curv, v) ||
-            sweep_shape(sv, a, v[0], v[1], v[2]))
+            (v[0] == 2 && check_chunks16(ax, a)) || sweep_shape(sv, a, v[0], v[1], v[2]))
             (void)sweep_shape(sv, a, d[0], d[1], d[2]);
-        if (filters && filter_axis_fused(sv, a) && tuned_filter(a, ax.N, ax.seam, v))
+        if (filters && filter_axis_tunable(sv, a) && tuned_filter(a, ax.N, ax.seam, v))
             (void)filter_shape(sv, a, v[0], v[1], v[2]);
     }
 }
 
 int cs_solver_tune(cs_solver* sv, int axis, int variant, int lines, int xcd) {
     if (!sv || axis < 0 || axis > 2) return fail(CS_ERR_ARG, "bad solver or axis");
+    if (variant == 2 && (lines == 8 || lines == 16)) {
+        const int rc = check_chunks16(sv->ax[axis], axis);
+        if (rc) return rc;
+    }
     return sweep_shape(sv, axis, variant, lines, xcd);
 }
 
@@ -431,7 +430,8 @@ int cs_solver_autotune(cs_solver* sv, const double* qa, const double* sbcc, int 
                     // grouping, the tiled one takes lines only
                     if (a == 0 && (x == 1 || (v == 0 && l == 8))) continue;
                     if (v == best[0] && l == best[1] && x == best[2]) continue;
-                    if (sweep_shape(sv, a, v, l, x)) continue;   // not admissible on this axis
+                    if ((v == 2 && check_chunks16(sv->ax[a], a)) || sweep_shape(sv, a, v, l, x))
+                        continue;   // not admissible on this axis
                     float t;
                     if ((rc = time_calls(sweeps, reps, s, ev, &t))) return rc;
                     if (t < kGain * tbest) {
@@ -446,7 +446,7 @@ int cs_solver_autotune(cs_solver* sv, const double* qa, const double* sbcc, int 
     if (!sv->cfg.filter) return CS_OK;
     CS_HIP(hipMemcpyAsync(out, qa, sizeof(double) * 5 * sv->g.lmx, hipMemcpyDeviceToDevice, s));
     for (int a = 0; a < 3; a++) {
-        if (!filter_axis_fused(sv, a)) continue;
+        if (!filter_axis_tunable(sv, a)) continue;
         auto filt = [&]() { return filter_sweeps(sv, out, s, a); };
         const AxisDesc cur = sv->fax[a];
         int best[3] = {cur.ffields, cur.ftl, cur.K};

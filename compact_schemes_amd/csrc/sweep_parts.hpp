@@ -18,6 +18,20 @@ __device__ __forceinline__ double ldg(const double* p, uoff bo) {
 __device__ __forceinline__ void stg(double* p, uoff bo, double v) {
     *reinterpret_cast<double*>(reinterpret_cast<char*>(p) + bo) = v;
 }
+// the same with the streaming hint where NT: the lines a sweep passes once and
+// that no cache can hold until they are used again
+template <bool NT>
+__device__ __forceinline__ double ldg(const double* p, uoff bo) {
+    const double* a = reinterpret_cast<const double*>(reinterpret_cast<const char*>(p) + bo);
+    if constexpr (NT) return __builtin_nontemporal_load(a);
+    else return *a;
+}
+template <bool NT>
+__device__ __forceinline__ void stg(double* p, uoff bo, double v) {
+    double* a = reinterpret_cast<double*>(reinterpret_cast<char*>(p) + bo);
+    if constexpr (NT) __builtin_nontemporal_store(v, a);
+    else *a = v;
+}
 
 struct Phys {
     cs_point umf;
@@ -30,7 +44,6 @@ __device__ __forceinline__ Prim prim_at(const double* const* q, uoff bo, double*
     for (int v = 0; v < 5; v++) qq[v] = ldg(q[v], bo);
     return primitive(qq);
 }
-
 // the two quantities of the time step at one point with constant diagonal
 // metrics (calc_time_step_kernel, src/cuda/kernels/physics.hpp:335-427, D9
 // corrected): the convective (c |grad xi| + |u . grad xi|) |J| and the
@@ -75,144 +88,148 @@ __device__ __forceinline__ uoff line_off(int axis, uoff f, uoff lxi, uoff plane)
     return f * 8u;
 }
 
-// recurrences of the solve (EX: every chunk has K rows)
-template <int K, int NF, bool EX>
-__device__ __forceinline__ void forward_local(const double* tab, int N, int s, int L, double (&r)[NF][K],
+// recurrences of the solve on the K rows of a chunk.  tab rows are chunk
+// rows: [5][P*K], rows past the line's end hold zeros (build_axis_table,
+// pad_line_table), so every chunk runs K rows; NP = P*K.  The products that
+// are fused are named, so that every kernel rounds alike.
+template <int K, int NF>
+__device__ __forceinline__ void forward_local(const double* tab, int NP, int s, double (&r)[NF][K],
                                               double (&carry)[NF]) {
-#pragma clang fp contract(fast)
 #pragma unroll
     for (int f = 0; f < NF; f++) carry[f] = 0.0;
 #pragma unroll
     for (int t = 0; t < K; t++) {
-        if (EX || t < L) {
-            const double nu = tab[s + t], mu = tab[N + s + t];
+        const double nu = tab[s + t], mu = tab[NP + s + t];
 #pragma unroll
-            for (int f = 0; f < NF; f++) { carry[f] = nu * r[f][t] + mu * carry[f]; r[f][t] = carry[f]; }
+        for (int f = 0; f < NF; f++) {
+            carry[f] = __builtin_fma(nu, r[f][t], mu * carry[f]);
+            r[f][t] = carry[f];
         }
     }
 }
 
-template <int K, int NF, bool EX>
-__device__ __forceinline__ void backward_local(const double* tab, int N, int s, int L, double (&r)[NF][K],
+template <int K, int NF>
+__device__ __forceinline__ void backward_local(const double* tab, int NP, int s, double (&r)[NF][K],
                                                double (&carry)[NF]) {
-#pragma clang fp contract(fast)
 #pragma unroll
     for (int f = 0; f < NF; f++) carry[f] = 0.0;
 #pragma unroll
     for (int t = K - 1; t >= 0; t--) {
-        if (EX || t < L) {
-            const double rh = tab[2 * N + s + t];
+        const double rh = tab[2 * NP + s + t];
 #pragma unroll
-            for (int f = 0; f < NF; f++) { carry[f] = r[f][t] + rh * carry[f]; r[f][t] = carry[f]; }
+        for (int f = 0; f < NF; f++) {
+            carry[f] = __builtin_fma(rh, carry[f], r[f][t]);
+            r[f][t] = carry[f];
         }
     }
 }
 
-template <int K, int NF, bool EX>
-__device__ __forceinline__ void apply_carry(const double* tab, int off, int s, int L, double (&r)[NF][K],
+template <int K, int NF>
+__device__ __forceinline__ void apply_carry(const double* tab, int off, int s, double (&r)[NF][K],
                                             const double (&G)[NF]) {
-#pragma clang fp contract(fast)
 #pragma unroll
     for (int t = 0; t < K; t++) {
-        if (EX || t < L) {
-            const double M = tab[off + s + t];
+        const double M = tab[off + s + t];
 #pragma unroll
-            for (int f = 0; f < NF; f++) r[f][t] += M * G[f];
-        }
+        for (int f = 0; f < NF; f++) r[f][t] = __builtin_fma(M, G[f], r[f][t]);
     }
 }
+
+// How many chunks away a carry of the derivative's solve still counts: the
+// interior LU factors of alpha = 1/3 shrink it by (3 - sqrt 5)/2 = 0.382 a row,
+// so after 48 rows it is below 1e-20 of its size, under the last bit of any
+// row it is added to.  The filter's factors (0.82 a row at alpha_f = 0.49)
+// reach across the whole line.
+constexpr int kCarryRows = 48;
+template <int K, bool FILTER>
+__device__ __forceinline__ int carry_reach(int P) { return FILTER ? P : kCarryRows / K; }
 
 // carries across the chunks of a line through LDS: buf = [NF][P][TL]
-template <int NF, bool EX, int K>
-__device__ __forceinline__ void fold_forward(const double* buf, const double* tab, int N, int P, int TL, int c,
+template <int NF, int K, bool FILTER>
+__device__ __forceinline__ void fold_forward(const double* buf, const double* tab, int NP, int P, int TL, int c,
                                              int lloc, double (&G)[NF]) {
-#pragma clang fp contract(fast)
 #pragma unroll
     for (int f = 0; f < NF; f++) G[f] = 0.0;
-    for (int cc = 0; cc < c; cc++) {
-        const int e = EX ? cc * K + K - 1 : (int)(((long)(cc + 1) * N) / P) - 1;
-        const double M = tab[3 * N + e];
+    for (int cc = max(0, c - carry_reach<K, FILTER>(P)); cc < c; cc++) {
+        const double M = tab[3 * NP + cc * K + K - 1];
 #pragma unroll
-        for (int f = 0; f < NF; f++) G[f] = buf[(f * P + cc) * TL + lloc] + M * G[f];
+        for (int f = 0; f < NF; f++) G[f] = __builtin_fma(M, G[f], buf[(f * P + cc) * TL + lloc]);
     }
 }
 
-template <int NF, bool EX, int K>
-__device__ __forceinline__ void fold_backward(const double* buf, const double* tab, int N, int P, int TL, int c,
+template <int NF, int K, bool FILTER>
+__device__ __forceinline__ void fold_backward(const double* buf, const double* tab, int NP, int P, int TL, int c,
                                               int lloc, double (&X)[NF]) {
-#pragma clang fp contract(fast)
 #pragma unroll
     for (int f = 0; f < NF; f++) X[f] = 0.0;
-    for (int cc = P - 1; cc > c; cc--) {
-        const int sc = EX ? cc * K : (int)(((long)cc * N) / P);
-        const double R = tab[4 * N + sc];
+    for (int cc = min(P - 1, c + carry_reach<K, FILTER>(P)); cc > c; cc--) {
+        const double R = tab[4 * NP + cc * K];
 #pragma unroll
-        for (int f = 0; f < NF; f++) X[f] = buf[(f * P + cc) * TL + lloc] + R * X[f];
+        for (int f = 0; f < NF; f++) X[f] = __builtin_fma(R, X[f], buf[(f * P + cc) * TL + lloc]);
     }
 }
 
-// carries across the chunks of a line held by GS consecutive lanes of a wave:
-// segmented Kogge-Stone scans of the affine maps x -> A*x + B
+// carries across the chunks of a line held by P consecutive lanes of a wave
+// (c = lane's chunk): segmented Kogge-Stone scans of the affine maps
+// x -> A*x + B over the `reach` nearest chunks (a power of two, or >= P)
 template <int NF>
-__device__ __forceinline__ void scan_forward(double A, const double (&carry)[NF], bool cv, int c, int GS,
+__device__ __forceinline__ void scan_forward(double A, const double (&carry)[NF], int c, int P, int reach,
                                              double (&G)[NF]) {
-#pragma clang fp contract(fast)
     double B[NF];
 #pragma unroll
-    for (int f = 0; f < NF; f++) B[f] = cv ? carry[f] : 0.0;
-    if (!cv) A = 1.0;
-    for (int d = 1; d < GS; d <<= 1) {
-        const double Au = __shfl_up(A, d, GS);
+    for (int f = 0; f < NF; f++) B[f] = carry[f];
+    for (int d = 1; d < min(P, reach); d <<= 1) {
+        const double Au = __shfl_up(A, d);
         double Bu[NF];
 #pragma unroll
-        for (int f = 0; f < NF; f++) Bu[f] = __shfl_up(B[f], d, GS);
+        for (int f = 0; f < NF; f++) Bu[f] = __shfl_up(B[f], d);
         if (c >= d) {
 #pragma unroll
-            for (int f = 0; f < NF; f++) B[f] += A * Bu[f];
+            for (int f = 0; f < NF; f++) B[f] = __builtin_fma(A, Bu[f], B[f]);
             A *= Au;
         }
     }
 #pragma unroll
     for (int f = 0; f < NF; f++) {
-        const double g = __shfl_up(B[f], 1, GS);
+        const double g = __shfl_up(B[f], 1);
         G[f] = (c == 0) ? 0.0 : g;
     }
 }
 
 template <int NF>
-__device__ __forceinline__ void scan_backward(double A, const double (&carry)[NF], bool cv, int c, int P, int GS,
+__device__ __forceinline__ void scan_backward(double A, const double (&carry)[NF], int c, int P, int reach,
                                               double (&X)[NF]) {
-#pragma clang fp contract(fast)
     double B[NF];
 #pragma unroll
-    for (int f = 0; f < NF; f++) B[f] = cv ? carry[f] : 0.0;
-    if (!cv) A = 0.0;
-    for (int d = 1; d < GS; d <<= 1) {
-        const double Ad = __shfl_down(A, d, GS);
+    for (int f = 0; f < NF; f++) B[f] = carry[f];
+    for (int d = 1; d < min(P, reach); d <<= 1) {
+        const double Ad = __shfl_down(A, d);
         double Bd[NF];
 #pragma unroll
-        for (int f = 0; f < NF; f++) Bd[f] = __shfl_down(B[f], d, GS);
-        if (c + d < GS) {
+        for (int f = 0; f < NF; f++) Bd[f] = __shfl_down(B[f], d);
+        if (c + d < P) {
 #pragma unroll
-            for (int f = 0; f < NF; f++) B[f] += A * Bd[f];
+            for (int f = 0; f < NF; f++) B[f] = __builtin_fma(A, Bd[f], B[f]);
             A *= Ad;
         }
     }
 #pragma unroll
     for (int f = 0; f < NF; f++) {
-        const double x = __shfl_down(B[f], 1, GS);
+        const double x = __shfl_down(B[f], 1);
         X[f] = (c + 1 < P) ? x : 0.0;
     }
 }
 
-// workgroup -> line group, neighbouring groups on the same XCD (workgroups
-// are dispatched round-robin over the 8 XCDs, each with its own L2)
+// workgroup -> line group.  Workgroups are dispatched round-robin over the 8
+// XCDs, each with its own L2; xcd = 1 + log2(G) gives runs of G neighbouring
+// groups to one XCD (0: plain order).
 __device__ __forceinline__ long group_of(int xcd) {
-    const long w = blockIdx.x;
+    const unsigned w = blockIdx.x;
     if (!xcd) return w;
-    const long G8 = ((long)gridDim.x / 8) * 8;
-    if (w >= G8) return w;
-    return (w % 8) * (G8 / 8) + w / 8;
+    const int g = xcd - 1;
+    const unsigned span = 8u << g, i = w / 8;
+    if (w >= gridDim.x / span * span) return w;
+    return (i >> g) * span + ((w % 8) << g) + (i & ((1u << g) - 1));
 }
 
 // LDS slot of row t of chunk c of line li in the transposing x kernels

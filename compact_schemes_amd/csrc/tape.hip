@@ -282,9 +282,9 @@ __global__ void __launch_bounds__(64) xtT_kernel(AxisDesc ax, SweepCommon cm, SW
     static_assert(H <= K, "halo rows come from the neighbouring chunks only");
     extern __shared__ double lds[];       // [64/GS lines][P chunks][K+1]
 
-    const int N = ax.N, P = ax.P, GS = ax.GS;
+    const int N = ax.N, P = ax.P;
     const int lane = threadIdx.x;
-    const int lpw = 64 / GS;
+    const int lpw = 64 / P;
     const long line0 = (long)blockIdx.x * lpw;
     const int nl = (int)min((long)lpw, ax.nlines - line0);
     const int npts = nl * N;
@@ -317,11 +317,10 @@ __global__ void __launch_bounds__(64) xtT_kernel(AxisDesc ax, SweepCommon cm, SW
         }
     }
 
-    const int li = lane / GS, c = lane % GS;
-    const bool work = li < nl && c < P;
-    const int lr = li < nl ? li : 0;
-    const int cc = c < P ? c : P - 1;
-    const int s = cc * K;
+    const int li = lane / P, c = lane % P;
+    const bool work = li < nl;
+    const int lr = work ? li : 0;
+    const int s = c * K;
     const long line = line0 + lr;
 
     double r[NF][K];
@@ -333,7 +332,7 @@ __global__ void __launch_bounds__(64) xtT_kernel(AxisDesc ax, SweepCommon cm, SW
             if (lane + 64 * j < npts) lds[slot[j]] = xq[f][j];
         __syncthreads();
 #pragma unroll
-        for (int t = 0; t < K; t++) r[f][t] = lds[xt_slot<K>(lr, P, cc, t)];
+        for (int t = 0; t < K; t++) r[f][t] = lds[xt_slot<K>(lr, P, c, t)];
     }
     if (mu && work) {
         const long nf = ax.nlines;
@@ -344,18 +343,18 @@ __global__ void __launch_bounds__(64) xtT_kernel(AxisDesc ax, SweepCommon cm, SW
         }
     }
 
-    const bool cv = c < P;
+    constexpr int kReach = ST == 0 ? 8 : 64;        // chunks (kCarryRows, rounded up to a power of two)
     double carry[NF], G[NF], X[NF];
-    forward_local<K, NF, true>(tabT, N, s, K, r, carry);
-    scan_forward<NF>(cv ? tabT[3 * N + s + K - 1] : 1.0, carry, cv, c, GS, G);
-    apply_carry<K, NF, true>(tabT, 3 * N, s, K, r, G);
-    backward_local<K, NF, true>(tabT, N, s, K, r, carry);
-    scan_backward<NF>(cv ? tabT[4 * N + s] : 0.0, carry, cv, c, P, GS, X);
-    apply_carry<K, NF, true>(tabT, 4 * N, s, K, r, X);
+    forward_local<K, NF>(tabT, N, s, r, carry);
+    scan_forward<NF>(tabT[3 * N + s + K - 1], carry, c, P, kReach, G);
+    apply_carry<K, NF>(tabT, 3 * N, s, r, G);
+    backward_local<K, NF>(tabT, N, s, r, carry);
+    scan_backward<NF>(tabT[4 * N + s], carry, c, P, kReach, X);
+    apply_carry<K, NF>(tabT, 4 * N, s, r, X);
 
     const bool wrap = ST == 0 && ax.seam;
-    const int hl = cc > 0 ? cc - 1 : (wrap ? P - 1 : 0);
-    const int hr = cc + 1 < P ? cc + 1 : (wrap ? 0 : P - 1);
+    const int hl = c > 0 ? c - 1 : (wrap ? P - 1 : 0);
+    const int hr = c + 1 < P ? c + 1 : (wrap ? 0 : P - 1);
 #pragma unroll
     for (int f = 0; f < NF; f++) {
         __syncthreads();
@@ -373,7 +372,7 @@ __global__ void __launch_bounds__(64) xtT_kernel(AxisDesc ax, SweepCommon cm, SW
 #pragma unroll
         for (int t = 0; t < K; t++) w[t + H] = r[f][t];
         double o[K];
-        stencil_t<K, ST, W>(w, o, s, N, cc, P, ax.seam, cm.pb, an);
+        stencil_t<K, ST, W>(w, o, s, N, c, P, ax.seam, cm.pb, an);
 #pragma unroll
         for (int t = 0; t < K; t++) r[f][t] = o[t];
     }
@@ -464,19 +463,19 @@ __global__ void __launch_bounds__(TL * kMaxP) __attribute__((amdgpu_waves_per_eu
     }
 
     double carry[NF], G[NF], X[NF];
-    forward_local<K, NF, true>(tabT, N, s, K, r, carry);
+    forward_local<K, NF>(tabT, N, s, r, carry);
 #pragma unroll
     for (int f = 0; f < NF; f++) lds[(f * P + c) * TL + lloc] = carry[f];
     __syncthreads();
-    fold_forward<NF, true, K>(lds, tabT, N, P, TL, c, lloc, G);
-    apply_carry<K, NF, true>(tabT, 3 * N, s, K, r, G);
-    backward_local<K, NF, true>(tabT, N, s, K, r, carry);
+    fold_forward<NF, K, ST != 0>(lds, tabT, N, P, TL, c, lloc, G);
+    apply_carry<K, NF>(tabT, 3 * N, s, r, G);
+    backward_local<K, NF>(tabT, N, s, r, carry);
     double* xb = lds + NF * P * TL;
 #pragma unroll
     for (int f = 0; f < NF; f++) xb[(f * P + c) * TL + lloc] = carry[f];
     __syncthreads();
-    fold_backward<NF, true, K>(xb, tabT, N, P, TL, c, lloc, X);
-    apply_carry<K, NF, true>(tabT, 4 * N, s, K, r, X);
+    fold_backward<NF, K, ST != 0>(xb, tabT, N, P, TL, c, lloc, X);
+    apply_carry<K, NF>(tabT, 4 * N, s, r, X);
 
     // halo rows hb[(f*2H + k)*P + c][TL]: k < H the first H rows of chunk c,
     // k >= H its last H rows (neighbours wrap on seam lines of the
@@ -614,7 +613,7 @@ int launch_t(const AxisDesc& ax, const SweepCommon& cm, const SW& sw, const doub
     constexpr int K = 8, NF = SW::NF, H = ST == 0 ? 2 : 5;
     const unsigned gy = NF == 1 ? 5u : 1u;
     if constexpr (AX == 0) {
-        const int lpw = 64 / ax.GS;
+        const int lpw = 64 / ax.P;
         const size_t lds = sizeof(double) * lpw * ax.P * (K + 1);
         dim3 block(64), grid((unsigned)((ax.nlines + lpw - 1) / lpw), gy);
         hipLaunchKernelGGL((xtT_kernel<K, SW, ST>), grid, block, lds, s, ax, cm, sw, tabT, mu, an);

@@ -99,12 +99,12 @@ class FusedSolver:
         self.order = 1
         self.precision = 0
         # the filter of cs_solver_rk4_step runs one fused sweep per axis where the
-        # axis splits into equal chunks (x: 8-point chunks up to 512 points; y/z:
-        # 8 or 16 points up to 256, 16 up to 512), else a line-solver launch
-        self.filter_axes = [bool(filt) and ((n % 8 == 0 and n <= 256) or (a == 0 and n % 8 == 0 and n <= 512) or
-                                            (a > 0 and n % 16 == 0 and n <= 512))
+        # axis splits into chunks at most one row short, else a line-solver launch
+        self.filter_axes = [bool(filt) and self._chunks_fit(n, 8 if (a == 0 or n <= 256) else 16)
                             for a, n in enumerate(self.dims)]
-        self.filter_fused = all(self.filter_axes)
+        # the single-sweep calls (sweep 7..10, tune_filter) take equal chunks
+        self.filter_fused = all(f and n % (8 if (a == 0 or n <= 256) else 16) == 0
+                                for a, (f, n) in enumerate(zip(self.filter_axes, self.dims)))
 
     def close(self):
         if getattr(self, "h", None):
@@ -154,40 +154,57 @@ class FusedSolver:
         check(lib().cs_solver_set_order(self.h, int(order)))
         self.order = int(order)
 
+    @staticmethod
+    def _chunks_fit(n, K):
+        P = -(-n // K)
+        return P * K - n <= (P - 2 if P > 2 else 0)
+
+    def _streams(self, which, ax):
+        """The launch's rule for streaming loads and stores: more than 256 MB
+        passed over, rows on whole cache lines (x: on 16 bytes)."""
+        ts = 4 if self.precision == 1 else 8
+        c = self.curvilinear
+        if which >= 8:
+            per = 40
+        elif which < 3:
+            per = 40 + ts * (17 if which == 2 else 4) + (80 if which == 2 and c else 0)
+        else:
+            per = 80 + (ts * (9 if c else 4) if self.viscous else 0) + (24 if c else 0) + {5: 40, 6: 80}.get(which, 0)
+        return self.dims[0] % (2 if ax == 0 else 16) == 0 and per * self.lmx > 256 * 2 ** 20
+
     def kernel_name(self, which):
         """Name of the HIP kernel instantiation a sweep launches (as profilers
         print it, without the argument list)."""
         if which == 7:
             return " + ".join(self.kernel_name(w) for w in FILTER_SWEEPS)
+        b = lambda v: str(bool(v)).lower()
         if which >= 8:
             ax = which - 8
             fields, lines, chunk = self.get_tune(ax)[1]
             sf = f"cs::fused::SF{'1' if fields == 1 else ''}<{ax}>"
+            nt = self._streams(which, ax)
             if ax == 0:
-                return f"cs::fused::xt_kernel<8, {sf}, false>"
-            return f"cs::fused::direct_kernel<{chunk}, {ax}, {lines}, {sf}, false>"
+                return f"cs::fused::xt_kernel<8, {sf}, false, {b(self.dims[0] % 8 == 0)}, {b(nt)}>"
+            ex = self.dims[ax] % chunk == 0
+            return f"cs::fused::direct_kernel<{chunk}, {ax}, {lines}, {sf}, false, {b(ex)}, {b(nt and lines == 16)}>"
         ax = S1_AXES[self.order][which] if which < 3 else S2_AXES[self.order][min(which, 5) - 3]
         n = self.dims[ax]
         variant, lines, _ = self.get_tune(ax)[0]
-        K = 8 if (n <= 256 or (ax == 0 and n % 8 == 0)) and variant != 2 else 16
-        P = (n + K - 1) // K
-        exact = n == P * K
+        K = 16 if ax > 0 and (variant == 2 or n > 256) else 8
         nbc = self.nbc_flat
         gcbc = nbc[ax] == 10 and nbc[3 + ax] == 10
         f32 = ("C" if self.curvilinear else "") + ("F" if (self.viscous and self.precision == 1) else "")
         if which < 3:
-            sw, gc = f"cs::fused::S1{f32}<{ax}, {str(which == 2).lower()}>", "false"
+            sw, gc = f"cs::fused::S1{f32}<{ax}, {b(which == 2)}>", "false"
         else:
             mode = {3: 0, 4: 1, 5: 2, 6: 3}[which]
-            sw, gc = f"cs::fused::S2{f32}<{ax}, {mode}, {str(self.viscous).lower()}>", str(gcbc).lower()
-        if variant == 1 and K == 8:
-            return f"cs::fused::tile_kernel<{K}, {ax}, {lines}, {str(exact).lower()}, {sw}, {gc}>"
-        if exact and ax == 0 and K == 8:
-            return f"cs::fused::xt_kernel<{K}, {sw}, {gc}>"
-        if exact:
-            tl = 16 if ax == 0 or lines != 8 else 8
-            return f"cs::fused::direct_kernel<{K}, {ax}, {tl}, {sw}, {gc}>"
-        return f"cs::fused::ragged_kernel<{K}, {ax}, {sw}, {gc}>"
+            sw, gc = f"cs::fused::S2{f32}<{ax}, {mode}, {b(self.viscous)}>", b(gcbc)
+        if K == 8 and (variant == 1 or not self._chunks_fit(n, K)):
+            return f"cs::fused::tile_kernel<{K}, {ax}, {lines}, {sw}, {gc}>"
+        nt = self._streams(which, ax)
+        if ax == 0:
+            return f"cs::fused::xt_kernel<{K}, {sw}, {gc}, {b(n % K == 0)}, {b(nt)}>"
+        return f"cs::fused::direct_kernel<{K}, {ax}, {lines}, {sw}, {gc}, {b(n % K == 0)}, {b(nt and lines == 16)}>"
 
     def time_step(self, q, stream=None):
         dt = ctypes.c_double()

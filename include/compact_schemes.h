@@ -252,7 +252,7 @@ int cs_solver_rhs(cs_solver* sv, const double* qa, double* de, const double* sbc
  * divergence sweeps; 6 = the last sweep fused with the last RK4 stage update
  * de = qa - dt*yaco*RHS, dt from the last time step, 0 before any; 7 = the
  * compact filter of the five variables of qa along x, y, z into de, three
- * launches, when every axis has 8-point chunks; 8, 9, 10 = that filter along
+ * launches, when every axis has equal chunks; 8, 9, 10 = that filter along
  * x, y or z only)
  * on the solver's scratch state; no reference counterpart -- it exists to
  * time and profile single kernels.  Sweeps depend on the outputs of the
@@ -264,7 +264,8 @@ int cs_solver_sweep(cs_solver* sv, int which, const double* qa, double* de, cons
  * src/numerics_rtc.hpp:120-126): variant 0 = each chunk thread evaluates its
  * own rows (halo rows exchanged between chunks), 1 = LDS row-block tiles
  * with coalesced loads, 2 = variant 0 on 16-point chunks (y/z lines of 32 to
- * 256 points, a multiple of 16; the default along z); lines = 8 or 16 lines
+ * 256 points, a multiple of 16; the default along y and z, there also on
+ * lines that 16-point chunks one row short can cut); lines = 8 or 16 lines
  * per workgroup (y/z lines of variants 0 and 2, all lines of variant 1);
  * xcd = 1 keeps neighbouring line groups on one XCD.  Results agree to
  * rounding whatever the choice. */
@@ -328,7 +329,7 @@ int cs_solver_time_step(cs_solver* sv, const double* qa, double* dte, cs_stream 
  * (the same value bit for bit; a viscous solver in the default sweep order
  * reduces it inside a gradient sweep of the first stage: with constant
  * metrics the first one where it runs whole waves of y lines, with per-point
- * metrics the closing x sweep where x lines split into 8-point chunks), stages q_k = q0 - dt/(5-k) * yaco * de(q_{k-1}),
+ * metrics the closing x sweep where it runs the transposing kernel), stages q_k = q0 - dt/(5-k) * yaco * de(q_{k-1}),
  * k = 1..4, then the compact filter along x, y, z when cfg.filter.  dt_out
  * (host, may be NULL) receives the step used; passing it synchronises the
  * stream. */
