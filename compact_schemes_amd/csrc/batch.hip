@@ -14,8 +14,8 @@
 // device, so the uneven subdomains share the CUs instead of each paying the
 // tail of a small launch.
 //
-// An item runs the same device body as the single-subdomain kernels
-// (line_body in line_solver.hip) with the same operator table, so every
+// An item runs the code of the single-subdomain kernels (line_sweeps.hip, or
+// line_body in line_solver.hip) with the same operator table, so every
 // subdomain's result is bit-identical to cs_deriv / cs_filter on it alone.
 //
 // The launches can be recorded into a hipGraph (cs_batch_capture) and
@@ -33,6 +33,7 @@ constexpr int kLanes = 8;      // streams of a grid-mode-2 step
 
 struct Launch {                // one kernel variant (K, axis) and chunk count P of a phase
     int K = 8, axis = 0, P = 1;
+    bool sweep = false;         // the sweep kernels (line_sweeps.hip), else line_solver.hip's
     int first = 0, nitems = 0;  // range in the phase's item list
     int threads = 0, grid = 0;
     size_t lds = 0;
@@ -41,6 +42,7 @@ struct Launch {                // one kernel variant (K, axis) and chunk count P
 struct Phase {
     int op = OP_DERIV;
     LineArgs* args = nullptr;   // device
+    unsigned char* recs = nullptr;   // device: the operators' records for the sweep kernels
     int2* items = nullptr;      // device
     int nitems = 0;
     std::vector<Launch> launches;
@@ -69,6 +71,7 @@ struct cs_batch {
 
 static void free_phase(Phase& p) {
     if (p.args) (void)hipFree(p.args);
+    if (p.recs) (void)hipFree(p.recs);
     if (p.items) (void)hipFree(p.items);
     p = Phase();
 }
@@ -111,7 +114,6 @@ static int line_args(cs_numerics* num, int op, int axis, const double* in, doubl
     *a = LineArgs{};
     a->in = in;
     a->out = out;
-    a->tab = t->dev;
     a->pb = num->pb;
     a->recv = nullptr;     // seam sums formed inside the kernel (single-subdomain wrap)
     a->drva = nullptr;
@@ -121,19 +123,18 @@ static int line_args(cs_numerics* num, int op, int axis, const double* in, doubl
     a->lxi = num->g.lxi;
     a->plane = (long)num->g.lxi * num->g.let;
     a->st = num->g.stride(axis);
-    a->P = t->P;
     a->seam0 = op == OP_DERIV ? start : 0;
     a->seam1 = op == OP_DERIV ? end : 0;
     a->cyclic = op == OP_FILTER ? (start == 1 && end == 1) : 0;
-    a->tab32 = t->dev32;
     a->mixed = 0;              // batched operators solve in FP64
-    *K = t->K;
+    choose_kernel(*t, op, axis, a, K);
     return CS_OK;
 }
 
 static int build_phase(cs_batch* b, Phase& p, int op, int axis_lo, int axis_hi) {
     struct Item { int variant; double cost; int2 it; };
     std::vector<LineArgs> args;
+    std::vector<unsigned char> recs;
     std::vector<Item> work;
     std::vector<Launch> var;                       // one per (K, axis) present
     p.op = op;
@@ -145,21 +146,26 @@ static int build_phase(cs_batch* b, Phase& p, int op, int axis_lo, int axis_hi) 
             int rc = line_args(b->num[s], op, axis, b->f[s], out, &a, &K);
             if (rc) return rc;
             int v = -1;
+            const bool sweep = line_sweep_ok(op, axis, K, a);
             for (size_t k = 0; k < var.size(); k++)
-                if (var[k].K == K && var[k].axis == axis && var[k].P == a.P) v = (int)k;
+                if (var[k].K == K && var[k].axis == axis && var[k].P == a.P && var[k].sweep == sweep) v = (int)k;
             if (v < 0) {
                 Launch l;
+                l.sweep = sweep;
                 l.K = K;
                 l.axis = axis;
                 l.P = a.P;
                 var.push_back(l);
                 v = (int)var.size() - 1;
             }
-            const int TL = batch_lines_per_item(K, axis, a.P);
-            var[v].threads = std::max(var[v].threads, TL * a.P);
-            var[v].lds = std::max(var[v].lds, batch_lds_bytes(K, axis, a.N));
+            const int TL = sweep ? batch_sweep_lines(axis, a.P) : batch_lines_per_item(K, axis, a.P);
+            var[v].threads = sweep ? batch_sweep_threads(axis, a.P) : std::max(var[v].threads, TL * a.P);
+            var[v].lds = sweep ? batch_sweep_lds(op, K, axis, a.P)
+                               : std::max(var[v].lds, batch_lds_bytes(K, axis, a.N));
             const int idx = (int)args.size();
             args.push_back(a);
+            recs.resize(recs.size() + batch_sweep_bytes());
+            batch_sweep_pack(op, K, a, &recs[recs.size() - batch_sweep_bytes()]);
             const int nblk = (a.nlines + TL - 1) / TL;
             const double cost = (double)a.N * std::min(TL, a.nlines);
             for (int k = 0; k < nblk; k++) work.push_back({v, cost, make_int2(idx, k)});
@@ -182,13 +188,16 @@ static int build_phase(cs_batch* b, Phase& p, int op, int axis_lo, int axis_hi) 
         while (pos < work.size() && work[pos].variant == (int)v) pos++;
         l.nitems = (int)pos - l.first;
         int nb = 1;
-        int rc = batch_blocks_per_cu(op, l.K, l.axis, l.P, l.threads, l.lds, &nb);
+        const int rc = l.sweep ? batch_sweep_blocks_per_cu(op, l.K, l.axis, l.P, l.lds, &nb)
+                               : batch_blocks_per_cu(op, l.K, l.axis, l.P, l.threads, l.lds, &nb);
         if (rc) return rc;
         l.grid = std::max(1, std::min(l.nitems, ncu * nb));
     }
     p.launches = var;
 
     CS_HIP(hipMalloc(&p.args, sizeof(LineArgs) * std::max<size_t>(1, args.size())));
+    CS_HIP(hipMalloc(&p.recs, std::max<size_t>(16, recs.size())));
+    CS_HIP(hipMemcpy(p.recs, recs.data(), recs.size(), hipMemcpyHostToDevice));
     CS_HIP(hipMalloc(&p.items, sizeof(int2) * std::max<size_t>(1, items.size())));
     CS_HIP(hipMemcpy(p.args, args.data(), sizeof(LineArgs) * args.size(), hipMemcpyHostToDevice));
     CS_HIP(hipMemcpy(p.items, items.data(), sizeof(int2) * items.size(), hipMemcpyHostToDevice));
@@ -260,8 +269,10 @@ static int run_phase(cs_batch* b, int k, int persistent, hipStream_t s) {
     const Phase& p = b->ph[k];
     for (const Launch& l : p.launches) {
         const int grid = persistent ? l.grid : l.nitems;
-        int rc = launch_batch_lines(p.op, l.K, l.axis, l.P, p.args, p.items + l.first, l.nitems, grid, l.threads,
-                                    l.lds, s);
+        const int rc = l.sweep ? launch_batch_sweeps(p.op, l.K, l.axis, l.P, p.recs, p.items + l.first, l.nitems,
+                                                     grid, l.lds, s)
+                               : launch_batch_lines(p.op, l.K, l.axis, l.P, p.args, p.items + l.first, l.nitems,
+                                                    grid, l.threads, l.lds, s);
         if (rc) return rc;
     }
     return CS_OK;
@@ -453,12 +464,11 @@ int cs_batch_autotune(cs_batch* b, int reps, cs_stream stream) {
             int Kd = 0;
             double* out = b->d[3 * c.s + c.axis];
             if ((rc = line_args(num, c.op, c.axis, b->f[c.s], out, &a, &Kd))) { free_line_op(t); break; }
-            a.tab = t.dev;
-            a.P = t.P;
+            choose_kernel(t, c.op, c.axis, &a, &Kd);
             float ms = 0.f;
-            rc = launch_line(c.op, c.axis, K, a, s);
+            rc = launch_line(c.op, c.axis, Kd, a, s);
             if (!rc && hipEventRecord(e0, s) != hipSuccess) rc = fail(CS_ERR_HIP, "event record failed");
-            for (int r = 0; r < reps && !rc; r++) rc = launch_line(c.op, c.axis, K, a, s);
+            for (int r = 0; r < reps && !rc; r++) rc = launch_line(c.op, c.axis, Kd, a, s);
             if (!rc && (hipEventRecord(e1, s) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
                         hipEventElapsedTime(&ms, e0, e1) != hipSuccess))
                 rc = fail(CS_ERR_HIP, "event timing failed");

@@ -104,16 +104,19 @@ struct LineOpKey {
 
 struct LineOpTable {
     int n = 0, K = 0, P = 0;
-    double* dev = nullptr;     // FP64 table (build_line_table)
+    double* dev = nullptr;     // FP64 table (build_line_table); owns the memory of the others
     float* dev32 = nullptr;    // FP32 factorisation for the mixed-precision solve
+    // the operator on the sweep kernels (line_sweeps.hip), y/z lines and x
+    // lines: chunk length and count, chunk_table (null: general kernels)
+    struct { int K = 0, P = 0; double* chunks = nullptr; } sweep[2];
     size_t count = 0;
 };
 
 inline void free_line_op(LineOpTable& t) {
     if (t.dev) (void)hipFree(t.dev);
-    if (t.dev32) (void)hipFree(t.dev32);
-    t.dev = nullptr;
+    t.sweep[0].chunks = t.sweep[1].chunks = nullptr;
     t.dev32 = nullptr;
+    t.dev = nullptr;
 }
 
 int choose_chunk(int n, int* K, int* P);
@@ -143,6 +146,7 @@ struct LineArgs {
     int P;
     int seam0, seam1;     // deriv: seam rows at the start / end of the line
     int cyclic;           // filter: cyclic system
+    const double* chunks; // chunk_table layout of the operator, or null
     const float* tab32;   // FP32 factorisation (mixed precision)
     int mixed;            // k > 0: FP32 solve + k FP64-residual refinement sweeps
     int nfields;          // fields processed by one launch (grid y), 0 or 1 = one
@@ -150,6 +154,19 @@ struct LineArgs {
 };
 
 int launch_line(int op, int axis, int K, const LineArgs& a, hipStream_t s);
+
+// the operators that run the kernels of the fused sweeps (line_sweeps.hip),
+// single and batched; batched records are batch_sweep_bytes each
+bool line_sweep_ok(int op, int axis, int K, const LineArgs& a);
+int launch_line_sweep(int op, int axis, int K, const LineArgs& a, hipStream_t s);
+int batch_sweep_lines(int axis, int P);
+int batch_sweep_threads(int axis, int P);
+size_t batch_sweep_bytes();
+size_t batch_sweep_lds(int op, int K, int axis, int P);
+void batch_sweep_pack(int op, int K, const LineArgs& a, unsigned char* dst);
+int batch_sweep_blocks_per_cu(int op, int K, int axis, int P, size_t lds, int* nb);
+int launch_batch_sweeps(int op, int K, int axis, int P, const void* ops, const int2* items, int nitems, int grid,
+                        size_t lds, hipStream_t s);
 
 // most chunks per line of a K-point chunked line operator
 int max_chunks(int K);
@@ -212,6 +229,9 @@ struct cs_physics {
 namespace cs {
 int get_line_op(cs_numerics* num, int op, int axis, int start, int end, LineOpTable** t);
 int make_line_op(const cs_numerics* num, int op, int n, int start, int end, int K, LineOpTable* t);
+// the operator's part of a (filled but for table and chunks) for lines along
+// `axis`, and the chunk length to launch with
+void choose_kernel(const LineOpTable& t, int op, int axis, LineArgs* a, int* K);
 int adjoint_workspace(cs_numerics* num, double** w);
 int deriv_adjoint(cs_numerics* num, int axis, const double* in, double* out, hipStream_t s);
 int filter_adjoint(cs_numerics* num, int axis, const double* in, double* out, hipStream_t s);

@@ -69,6 +69,8 @@ struct S1T {
     static constexpr int kStash = CLOSE ? 3 : 0;
     static constexpr int kH = 2;           // derivative stencil half-width
     static constexpr int kWpe = 3;         // waves per SIMD of the y/z kernels (168 VGPRs)
+    static constexpr int kWpe16 = 2;       // with 16-point chunks
+    static constexpr bool kEnds = false;   // end_value takes the results at a line's ends
     static constexpr bool kFilter = false;
     // DT: a sweep that also reduces the time step's maxima over the points it
     // evaluates, one pair per workgroup: a y/z gradient sweep
@@ -221,6 +223,8 @@ struct S2T {
     static constexpr int kStash = 0;
     static constexpr int kH = 2;
     static constexpr int kWpe = 3;
+    static constexpr int kWpe16 = 2;
+    static constexpr bool kEnds = false;
     static constexpr bool kFilter = false;
     const double* q[5];
     const TS* tr[3];          // row AX of the stress tensor
@@ -424,6 +428,8 @@ struct SF {
     static constexpr int kStash = 0;
     static constexpr int kH = 5;
     static constexpr int kWpe = 3;
+    static constexpr int kWpe16 = 2;
+    static constexpr bool kEnds = false;
     static constexpr bool kFilter = true;
     double* q[5];
     struct Raw { double q[5]; };
@@ -455,6 +461,8 @@ struct SF1 {
     static constexpr int kStash = 0;
     static constexpr int kH = 5;
     static constexpr int kWpe = 3;
+    static constexpr int kWpe16 = 2;
+    static constexpr bool kEnds = false;
     static constexpr bool kFilter = true;
     double* q;
     long lmx;
@@ -677,6 +685,48 @@ struct DtFold<SW, std::void_t<decltype(SW::kDt)>> {
     static constexpr bool close = SW::kDt && SW::kCurv;
 };
 
+// Many operators in one launch (batched subdomains): a direct or x kernel
+// launched with a BatchItems argument takes its descriptor from operator
+// items[i].x and runs that operator's workgroup items[i].y, items round-robin
+// over the grid.  Without one these are no-ops.
+template <class SW>
+struct BatchOp {
+    AxisDesc ax;
+    SweepCommon cm;
+    SW sw;
+};
+template <class SW>
+struct BatchItems {
+    const BatchOp<SW>* ops;
+    const int2* items;
+    int n;
+    __device__ __forceinline__ bool more(int& it) const { return (it += gridDim.x) < n; }
+    // the operator is the same for the whole workgroup: into scalar registers
+    // word by word, as a by-value kernel argument is
+    __device__ __forceinline__ void take(int it, AxisDesc& ax, SweepCommon& cm, SW& sw, long& group) const {
+        static_assert(sizeof(BatchOp<SW>) % 4 == 0, "moves as 32-bit words");
+        constexpr int kWords = sizeof(BatchOp<SW>) / 4;
+        const unsigned* src =
+            reinterpret_cast<const unsigned*>(ops + __builtin_amdgcn_readfirstlane(items[it].x));
+        group = __builtin_amdgcn_readfirstlane(items[it].y);
+        unsigned words[kWords];
+#pragma unroll
+        for (int i = 0; i < kWords; i++) words[i] = __builtin_amdgcn_readfirstlane(src[i]);
+        BatchOp<SW> o;
+        __builtin_memcpy(&o, words, sizeof o);
+        ax = o.ax;
+        cm = o.cm;
+        sw = o.sw;
+    }
+};
+struct NoBatch {
+    __device__ __forceinline__ bool more(int&) const { return false; }
+    template <class SW>
+    __device__ __forceinline__ void take(int, AxisDesc& ax, SweepCommon&, SW&, long& group) const {
+        group = group_of(ax.xcd);
+    }
+};
+
 // ---------------------------------------------------------------------------
 // variant "direct", y/z lines: TL consecutive lines x P chunks per workgroup;
 // each thread evaluates the pointwise inputs of its own K rows once, the halo
@@ -697,21 +747,27 @@ struct DtFold<SW, std::void_t<decltype(SW::kDt)>> {
 constexpr int kRowsAhead = 2;   // rows whose loads are in flight while a row is evaluated
 constexpr int kRowsOut = 4;     // rows whose epilogue loads are in flight
 
-template <int K, int AX, int TL, class SW, bool GCBC, bool EX, bool NT>
-__global__ void __launch_bounds__(TL * kMaxP) __attribute__((amdgpu_waves_per_eu(K == 16 ? 2 : SW::kWpe)))
-direct_kernel(AxisDesc ax, SweepCommon cm, SW sw) {
+template <int K, int AX, int TL, class SW, bool GCBC, bool EX, bool NT, class BATCH = NoBatch>
+__global__ void __launch_bounds__(TL * kMaxP < 1024 ? TL * kMaxP : 1024)
+__attribute__((amdgpu_waves_per_eu(K == 16 ? SW::kWpe16 : SW::kWpe)))
+direct_kernel(AxisDesc ax, SweepCommon cm, SW sw, BATCH batch) {
+    extern __shared__ double lds[];       // direct_lds
     constexpr int NF = SW::NF;
     constexpr int H = SW::kH;
     constexpr int W = K + 2 * H;
     static_assert(AX != 0, "x lines run xt_kernel");
     static_assert(H <= K, "halo rows come from the neighbouring chunks only");
-    extern __shared__ double lds[];
+    int it = blockIdx.x;
+    do {
+    long group;
+    batch.take(it, ax, cm, sw, group);
 
     const int N = ax.N, P = ax.P, NP = P * K;
     const Chunks<K, EX> ch(N, P);
     const int lloc = threadIdx.x % TL;
-    const int c = threadIdx.x / TL;
-    const long line = group_of(ax.xcd) * TL + lloc;
+    // 64 lines: one chunk a wave, its table entries come by scalar loads
+    const int c = TL == 64 ? __builtin_amdgcn_readfirstlane(threadIdx.x / TL) : threadIdx.x / TL;
+    const long line = group * TL + lloc;
     const bool act = line < ax.nlines;
     const int s = c * K, row0 = ch.start(c);      // table and line position of the chunk
     const bool whole = ch.whole(c);
@@ -866,7 +922,11 @@ direct_kernel(AxisDesc ax, SweepCommon cm, SW sw) {
         cyclic_correction<K, NF>(tab, NP, s, y0, yN1, r);
     }
 
-    if (!act) return;
+    if (act) {
+    if constexpr (SW::kEnds) {
+        if (first) sw.end_value(0, line, r[0][0]);
+        if (last) sw.end_value(1, line, r[0][K - 1]);
+    }
     if constexpr (GCBC) {
         if (first || last) {
             const auto fc = sw.face_in(base + (uoff)(first ? 0 : N - 1) * st, first ? 0 : 1, cm.sbcc);
@@ -902,6 +962,9 @@ direct_kernel(AxisDesc ax, SweepCommon cm, SW sw) {
             sw.template store<NT>(off(t), d);
         }
     }
+    }
+    if constexpr (!std::is_same_v<BATCH, NoBatch>) __syncthreads();      // the LDS is free for the next item
+    } while (batch.more(it));
 }
 
 // ---------------------------------------------------------------------------
@@ -920,23 +983,29 @@ direct_kernel(AxisDesc ax, SweepCommon cm, SW sw) {
 // branches around every point, closure rows tested row by row, seam rows read
 // again from memory, scans over the whole line.
 // ---------------------------------------------------------------------------
-template <int K, class SW, bool GCBC, bool EX, bool NT>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) xt_kernel(AxisDesc ax, SweepCommon cm, SW sw) {
+template <int K, class SW, bool GCBC, bool EX, bool NT, class BATCH = NoBatch>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
+xt_kernel(AxisDesc ax, SweepCommon cm, SW sw, BATCH batch) {
+    extern __shared__ double lds[];       // xt_lds
     constexpr int NF = SW::NF;
     constexpr int J = K;                  // points per lane: (64/P)*N <= 64*K
     constexpr int H = SW::kH;
     constexpr int W = K + 2 * H;
-    static_assert(K == 8, "row = 8 * chunk + t");
-    // [64/P lines][P chunks][K+1], 64 slots for lanes past the run, then
+    constexpr int LK = K == 8 ? 3 : 4;
+    static_assert(K == 8 || K == 16, "chunks of 8 or 16 points");
+    int it = blockIdx.x;
+    do {
+    long group;
+    batch.take(it, ax, cm, sw, group);
+    // lds: [64/P lines][P chunks][K+1], 64 slots for lanes past the run, then
     // (kStash > 0) the stashed point values [kStash][J][64]
-    extern __shared__ double lds[];
 
     const int N = ax.N, P = ax.P, NP = P * K;
     const Chunks<K, EX> ch(N, P);
     const int lane = threadIdx.x;
     const int lpw = 64 / P;
     double* stash = lds + lpw * P * (K + 1) + 64;
-    const long line0 = group_of(ax.xcd) * lpw;
+    const long line0 = group * lpw;
     const int nl = (int)min((long)lpw, ax.nlines - line0);   // lines of this wave
     const int npts = nl * N;
     const uoff run = line_off(0, (uoff)line0, (uoff)cm.lxi, (uoff)cm.plane);
@@ -975,22 +1044,22 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) xt
             for (int j = 0; j < J; j++) stash[(f * J + j) * 64 + lane] = xq[f][j];
     }
 
-    // LDS slot of each of the lane's points: chunk * (K+1) + row of the chunk;
-    // rows of whole chunks after the short ones, of the first, of the short ones
+    // LDS slot of each of the lane's points: chunk * (K+1) + row of the chunk
+    auto whole_slot = [](int row) { return (row >> LK) * (K + 1) + (row & (K - 1)); };
     auto row_slot = [&](int row) {
-        const int a = row + ch.D, q = row - K;
-        const int cs = (q * 9363) >> 16;                         // q / 7, exact for q < 512
-        return EX || row < K || q >= (K - 1) * ch.D ? ((EX || row >= K ? a : row) >> 3) * (K + 1) + ((EX || row >= K ? a : row) & 7)
-                                                    : (cs + 1) * (K + 1) + (q - cs * (K - 1));
+        const int q = row - K;                                   // rows after the first chunk
+        const int cs = (q * (65536 / (K - 1) + 1)) >> 16;        // q / (K-1), exact for q < 1024
+        if (row < K) return row;
+        return q < (K - 1) * ch.D ? (cs + 1) * (K + 1) + (q - cs * (K - 1)) : whole_slot(row + ch.D);
     };
     int slot[J];
 #pragma unroll
     for (int j = 0; j < J; j++) {
         const int p = lane + 64 * j;
         if (EX) {
-            slot[j] = (p >> 3) * (K + 1) + (p & 7);
+            slot[j] = whole_slot(p);
         } else {
-            // p / N by the reciprocal rounded up: exact for p < 512 <= 2^24 / N
+            // p / N by the reciprocal rounded up: exact for p < 1024, N <= 1024
             const int l = (int)(((unsigned)p * ((0x1000000u + N - 1) / (unsigned)N)) >> 24);
             slot[j] = xt_slot<K>(l, P, 0, 0) + row_slot(p - l * N);
         }
@@ -1037,7 +1106,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) xt
         }
     }
 
-    constexpr int kReach = SW::kFilter ? 64 : 8;    // chunks (kCarryRows, rounded up to a power of two)
+    constexpr int kReach = SW::kFilter ? 64 : 64 / K;    // chunks (kCarryRows, rounded up to a power of two)
     double carry[NF], G[NF], X[NF];
     forward_local<K, NF>(tab, NP, s, r, carry);
     scan_forward<NF>(tab[3 * NP + s + K - 1], carry, c, P, kReach, G);
@@ -1054,6 +1123,10 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) xt
             yN1[f] = __shfl(r[f][K - 1], lr * P + P - 1);
         }
         cyclic_correction<K, NF>(tab, NP, s, y0, yN1, r);
+    }
+    if constexpr (SW::kEnds) {
+        if (work && first) sw.end_value(0, line0 + li, r[0][0]);
+        if (work && last) sw.end_value(1, line0 + li, r[0][K - 1]);
     }
     if constexpr (GCBC) {
         if (work && (first || last)) {
@@ -1119,6 +1192,8 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) xt
             sw.dtpart[2 * blockIdx.x + 1] = mm[1];
         }
     }
+    if constexpr (!std::is_same_v<BATCH, NoBatch>) __syncthreads();
+    } while (batch.more(it));
 }
 
 // ---------------------------------------------------------------------------
@@ -1316,21 +1391,31 @@ static const void* direct_symbol(int TL, bool exact, bool nt) {
               : (const void*)direct_kernel<K, AX, 16, SW, GCBC, false, false>;
 }
 
-template <class SW>
-static int launch(const void* k, dim3 grid, dim3 block, size_t lds, AxisDesc a, SweepCommon cm, SW sw, hipStream_t s) {
+template <class SW, class BATCH = NoBatch>
+static int launch(const void* k, dim3 grid, dim3 block, size_t lds, AxisDesc a, SweepCommon cm, SW sw, hipStream_t s,
+                  BATCH batch = BATCH()) {
     if (lds > 65536) CS_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    void* args[] = {&a, &cm, &sw};
+    void* args[] = {&a, &cm, &sw, &batch};
     CS_HIP(hipLaunchKernel(k, grid, block, args, lds, s));
     return CS_OK;
 }
 
+// LDS of a workgroup
+template <int K, class SW>
+static size_t xt_lds(int P) { return sizeof(double) * ((64 / P) * P * (K + 1) + 64 + SW::kStash * K * 64); }
+template <class SW>
+static size_t direct_lds(int P, int TL, bool seam) {
+    const size_t halo = (size_t)(SW::kFilter ? 1 : SW::NF) * 2 * SW::kH * P + (!SW::kFilter && seam ? SW::NF * 2 * kLmd : 0);
+    const size_t carries = (size_t)2 * SW::NF * P + (SW::kFilter ? 2 * SW::NF : 0);
+    return sizeof(double) * TL * (halo > carries ? halo : carries);
+}
+
 // x sweeps: a workgroup is the 64/P lines of one wave, runs of 64 an XCD
 // (measured 4.8 -> 5.3 TB/s for a copy of that shape)
-template <class SW, bool GCBC>
+template <int K, class SW, bool GCBC>
 static int launch_x(const AxisDesc& ax, const SweepCommon& cm, const SW& sw, unsigned gy, hipStream_t s) {
-    constexpr int K = 8;
     const int lpw = 64 / ax.P;
-    const size_t lds = sizeof(double) * (lpw * ax.P * (K + 1) + 64 + SW::kStash * K * 64);
+    const size_t lds = xt_lds<K, SW>(ax.P);
     const dim3 grid((unsigned)((ax.nlines + lpw - 1) / lpw), gy);
     return launch(xt_symbol<K, SW, GCBC>(ax.N == ax.P * K, streams<SW>(ax, cm)), grid, dim3(64), lds,
                   with_runs(ax, grid.x, true, 64), cm, sw, s);
@@ -1364,11 +1449,10 @@ static int launch_sweep(const AxisDesc& ax, const SweepCommon& cm, const SW& sw,
     }
     if constexpr (AX == 0) {
         static_assert(K == 8, "x lines run 8-point chunks");
-        return launch_x<SW, GCBC>(ax, cm, sw, 1u, s);
+        return launch_x<K, SW, GCBC>(ax, cm, sw, 1u, s);
     } else {
         const int TL = ax.tl == 8 ? 8 : 16;
-        const size_t lds = sizeof(double) * NF * TL * (2 * SW::kH * ax.P + (ax.seam ? 2 * kLmd : 0));
-        return launch_yz<K, AX, SW, GCBC>(ax, cm, sw, TL, ax.xcd != 0, lds, 1u, s);
+        return launch_yz<K, AX, SW, GCBC>(ax, cm, sw, TL, ax.xcd != 0, direct_lds<SW>(ax.P, TL, ax.seam), 1u, s);
     }
 }
 
@@ -1377,18 +1461,15 @@ static int launch_sweep(const AxisDesc& ax, const SweepCommon& cm, const SW& sw,
 // or SF1<AX> (one variable per workgroup, grid.y = 5)
 template <int K, int AX, class SW>
 static int launch_filter(const AxisDesc& ax, const SweepCommon& cm, const SW& sw, hipStream_t s) {
-    constexpr int NF = SW::NF, H = SW::kH;
+    constexpr int NF = SW::NF;
     static_assert(AX != 0 || K == 8, "x filter sweeps run 8-point chunks");
     const unsigned gy = NF == 1 ? 5u : 1u;
     if (ax.K != K || !ax.ftab) return fail(CS_ERR_STATE, "fused filter without its table");
     if constexpr (AX == 0) {
-        return launch_x<SW, false>(ax, cm, sw, gy, s);
+        return launch_x<K, SW, false>(ax, cm, sw, gy, s);
     } else {
         const int TL = ax.ftl == 8 ? 8 : 16;
-        const size_t halo = (size_t)2 * H * ax.P * TL;
-        const size_t carries = (size_t)2 * NF * ax.P * TL + 2 * NF * TL;
-        return launch_yz<K, AX, SW, false>(ax, cm, sw, TL, true, sizeof(double) * (halo > carries ? halo : carries),
-                                           gy, s);
+        return launch_yz<K, AX, SW, false>(ax, cm, sw, TL, true, direct_lds<SW>(ax.P, TL, false), gy, s);
     }
 }
 

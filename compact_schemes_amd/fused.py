@@ -184,9 +184,9 @@ class FusedSolver:
             sf = f"cs::fused::SF{'1' if fields == 1 else ''}<{ax}>"
             nt = self._streams(which, ax)
             if ax == 0:
-                return f"cs::fused::xt_kernel<8, {sf}, false, {b(self.dims[0] % 8 == 0)}, {b(nt)}>"
+                return f"cs::fused::xt_kernel<8, {sf}, false, {b(self.dims[0] % 8 == 0)}, {b(nt)}, cs::fused::NoBatch>"
             ex = self.dims[ax] % chunk == 0
-            return f"cs::fused::direct_kernel<{chunk}, {ax}, {lines}, {sf}, false, {b(ex)}, {b(nt and lines == 16)}>"
+            return f"cs::fused::direct_kernel<{chunk}, {ax}, {lines}, {sf}, false, {b(ex)}, {b(nt and lines == 16)}, cs::fused::NoBatch>"
         ax = S1_AXES[self.order][which] if which < 3 else S2_AXES[self.order][min(which, 5) - 3]
         n = self.dims[ax]
         variant, lines, _ = self.get_tune(ax)[0]
@@ -203,8 +203,9 @@ class FusedSolver:
             return f"cs::fused::tile_kernel<{K}, {ax}, {lines}, {sw}, {gc}>"
         nt = self._streams(which, ax)
         if ax == 0:
-            return f"cs::fused::xt_kernel<{K}, {sw}, {gc}, {b(n % K == 0)}, {b(nt)}>"
-        return f"cs::fused::direct_kernel<{K}, {ax}, {lines}, {sw}, {gc}, {b(n % K == 0)}, {b(nt and lines == 16)}>"
+            return f"cs::fused::xt_kernel<{K}, {sw}, {gc}, {b(n % K == 0)}, {b(nt)}, cs::fused::NoBatch>"
+        return f"cs::fused::direct_kernel<{K}, {ax}, {lines}, {sw}, {gc}, {b(n % K == 0)}, {b(nt and lines == 16)}, "\
+               "cs::fused::NoBatch>"
 
     def time_step(self, q, stream=None):
         dt = ctypes.c_double()
