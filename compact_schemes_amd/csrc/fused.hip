@@ -151,18 +151,11 @@ static int fold_blocks(const cs_solver* sv, int pos) {
 int rhs_sweeps(cs_solver* sv, const double* q, const double* sbcc, double* out, const double* q0, int div,
                hipStream_t s) {
     const SweepCommon cm = common_of(sv, sbcc);
+    // One stream: the two gradient sweeps that do not depend on each other
+    // side by side on two streams shared the memory rate each reaches alone,
+    // and the fork and the join cost 6-11 us each (a step on 48 x 40 x 32
+    // points 331 us with them, 259 without; 256^3 10.92 and 10.81 ms).
     for (int pos = sv->cfg.viscous ? 0 : 3; pos < 6; pos++) {
-        if (pos == 0) {
-            // the second gradient sweep on the aux stream, concurrently with
-            // the first; the closing sweep waits for both
-            CS_HIP(hipEventRecord(sv->ev_fork, s));
-            CS_HIP(hipStreamWaitEvent(sv->aux, sv->ev_fork, 0));
-            const int rc = sweep_at(sv, 1, cm, q, out, nullptr, div, sv->aux);
-            if (rc) return rc;
-            CS_HIP(hipEventRecord(sv->ev_join, sv->aux));
-        }
-        if (pos == 1) continue;
-        if (pos == 2) CS_HIP(hipStreamWaitEvent(s, sv->ev_join, 0));
         const int rc = sweep_at(sv, pos, cm, q, out, pos == 5 ? q0 : nullptr, div, s);
         if (rc) return rc;
         if (sv->dt_fold == pos + 1) {
