@@ -110,6 +110,15 @@ static int seam_pair(const cs_numerics* num, int axis) {
     return -1;
 }
 
+// derivatives along an axis of the nf fields ifs apart at `in`, of variables
+// var, var + 1, ..., into fields 3*lmx apart, their boundary values into drva
+static int deriv_fields(cs_numerics* num, int axis, const double* in, long ifs, double* out, int var, int nf,
+                        hipStream_t s) {
+    const int sp = seam_pair(num, axis);
+    if (sp < 0) return fail(CS_ERR_UNSUPPORTED, "axis with one seam face needs a neighbour subdomain");
+    return line_apply(num, OP_DERIV, axis, in, out, sp, sp, nullptr, var, true, s, nf, ifs, 3 * num->g.lmx);
+}
+
 }  // namespace cs
 
 using namespace cs;
@@ -347,8 +356,7 @@ int cs_physics_create(const cs_dims* dims, int viscous, cs_point umf, cs_physics
               hipMalloc(&ph->red, sizeof(double) * (2 * ph->red_blocks + 2)) == hipSuccess &&
               hipHostMalloc(&ph->red_host, sizeof(double) * 2) == hipSuccess;
     if (ok && ph->viscous)
-        ok = hipMalloc(&ph->ss, sizeof(double) * 3 * lmx) == hipSuccess &&
-             hipMalloc(&ph->stress, sizeof(double) * 6 * lmx) == hipSuccess &&
+        ok = hipMalloc(&ph->stress, sizeof(double) * 6 * lmx) == hipSuccess &&
              hipMalloc(&ph->heat, sizeof(double) * 3 * lmx) == hipSuccess;
     if (!ok) {
         cs_physics_destroy(ph);
@@ -366,7 +374,6 @@ int cs_physics_destroy(cs_physics* ph) {
     if (!ph) return CS_OK;
     if (ph->buffer) (void)hipFree(ph->buffer);
     if (ph->buffer_deriv) (void)hipFree(ph->buffer_deriv);
-    if (ph->ss) (void)hipFree(ph->ss);
     if (ph->stress) (void)hipFree(ph->stress);
     if (ph->heat) (void)hipFree(ph->heat);
     if (ph->red) (void)hipFree(ph->red);
@@ -415,18 +422,12 @@ int cs_calc_fluxes(cs_physics* ph, cs_numerics* num, const double* qa, const dou
     const long lmx = ph->g.lmx;
     rc = launch_fluxes_pre(ph->viscous, ph->buffer, qa, p, de, xim, etm, zem, ph->stress, ph->heat, ph->umf, lmx, s);
     if (rc) return rc;
-    for (int m = 0; m < kNV; m++) {
-        for (int a = 0; a < 3; a++) {
-            int sp = seam_pair(num, a);
-            if (sp < 0) return fail(CS_ERR_UNSUPPORTED, "axis with one seam face needs a neighbour subdomain");
-            const long off = (long)m * 3 * lmx + (long)a * lmx;
-            rc = line_apply(num, OP_DERIV, a, ph->buffer + off, ph->buffer_deriv + off, sp, sp, nullptr, m, true, s);
-            if (rc) return rc;
-        }
-        rc = launch_fluxes_post(de, ph->buffer_deriv, m, lmx, s);
+    // the five fluxes along an axis in one launch: they lie 3*lmx apart
+    for (int a = 0; a < 3; a++) {
+        rc = deriv_fields(num, a, ph->buffer + (long)a * lmx, 3 * lmx, ph->buffer_deriv + (long)a * lmx, 0, kNV, s);
         if (rc) return rc;
     }
-    return CS_OK;
+    return launch_fluxes_post(de, ph->buffer_deriv, lmx, s);
 }
 
 int cs_calc_viscous_shear_stress(cs_physics* ph, cs_numerics* num, double* de, const double* ssk, const double* xim,
@@ -437,20 +438,12 @@ int cs_calc_viscous_shear_stress(cs_physics* ph, cs_numerics* num, double* de, c
     if (!de || !ssk || !xim || !etm || !zem || !yaco) return fail(CS_ERR_ARG, "null field pointer");
     hipStream_t s = (hipStream_t)stream;
     const long lmx = ph->g.lmx;
-    rc = launch_visc_init(ph->buffer, de, lmx, s);
-    if (rc) return rc;
-    for (int m = 1; m < kNV; m++) {
-        for (int a = 0; a < 3; a++) {
-            int sp = seam_pair(num, a);
-            if (sp < 0) return fail(CS_ERR_UNSUPPORTED, "axis with one seam face needs a neighbour subdomain");
-            rc = line_apply(num, OP_DERIV, a, ph->buffer + (long)m * 3 * lmx,
-                            ph->buffer_deriv + (long)m * 3 * lmx + (long)a * lmx, sp, sp, nullptr, m, true, s);
-            if (rc) return rc;
-        }
-        rc = launch_visc_post(ph->stress, ph->heat, ph->ss, ph->buffer_deriv, xim, etm, zem, m, lmx, s);
+    // u, v, w, c^2 from de[1..4], one launch an axis
+    for (int a = 0; a < 3; a++) {
+        rc = deriv_fields(num, a, de + lmx, lmx, ph->buffer_deriv + (3 + (long)a) * lmx, 1, kNV - 1, s);
         if (rc) return rc;
     }
-    return launch_visc_final(de, ssk, yaco, ph->ss, ph->stress, ph->heat, lmx, s);
+    return launch_visc(de, ssk, yaco, ph->buffer_deriv, xim, etm, zem, ph->stress, ph->heat, lmx, s);
 }
 
 int cs_calc_time_step(cs_physics* ph, const double* xim, const double* etm, const double* zem, const double* de,

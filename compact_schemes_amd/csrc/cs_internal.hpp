@@ -150,7 +150,8 @@ struct LineArgs {
     const float* tab32;   // FP32 factorisation (mixed precision)
     int mixed;            // k > 0: FP32 solve + k FP64-residual refinement sweeps
     int nfields;          // fields processed by one launch (grid y), 0 or 1 = one
-    long fstride;         // distance between those fields
+    long fstride;         // distance between those fields at `in`
+    long ostride;         // and at `out`
 };
 
 int launch_line(int op, int axis, int K, const LineArgs& a, hipStream_t s);
@@ -218,7 +219,6 @@ struct cs_physics {
     cs_point dudtmf{0, 0, 0};
     double* buffer = nullptr;        // [5][3][lmx]
     double* buffer_deriv = nullptr;  // [5][3][lmx]
-    double* ss = nullptr;            // [3][lmx]
     double* stress = nullptr;        // [6][lmx]
     double* heat = nullptr;          // [3][lmx]
     double* red = nullptr;           // time-step partial maxima
@@ -236,6 +236,7 @@ int adjoint_workspace(cs_numerics* num, double** w);
 int deriv_adjoint(cs_numerics* num, int axis, const double* in, double* out, hipStream_t s);
 int filter_adjoint(cs_numerics* num, int axis, const double* in, double* out, hipStream_t s);
 int line_apply(cs_numerics* num, int op, int axis, const double* in, double* out, int start, int end,
-               const double* recv, int var, bool write_drva, hipStream_t s, int nfields = 1);
+               const double* recv, int var, bool write_drva, hipStream_t s, int nfields = 1, long fstride = 0,
+               long ostride = 0);
 int check_dims(const cs_dims* d, Geo* g);
 }  // namespace cs

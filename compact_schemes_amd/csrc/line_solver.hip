@@ -543,7 +543,7 @@ __global__ void __launch_bounds__(max_threads(K)) line_kernel(LineArgs a) {
     extern __shared__ double smem[];
     if (blockIdx.y > 0) {
         a.in += (long)blockIdx.y * a.fstride;
-        a.out += (long)blockIdx.y * a.fstride;
+        a.out += (long)blockIdx.y * a.ostride;
     }
     line_body<K, OP, AX, TL, MIX>(a, blockIdx.x, smem);
 }
@@ -589,7 +589,20 @@ static int launch_axis(int axis, const LineArgs& a, hipStream_t s) {
 int launch_line(int op, int axis, int K, const LineArgs& a, hipStream_t s) {
     if (a.P < 1 || a.P > max_chunks(K)) return fail(CS_ERR_SHAPE, "chunk count out of range");
     if (line_sweep_ok(op, axis, K, a)) return launch_line_sweep(op, axis, K, a, s);
-    if (a.nfields > 1 && (a.drva || a.recv)) return fail(CS_ERR_ARG, "multi-field launches write no boundary data");
+    if (a.nfields > 1 && a.recv) return fail(CS_ERR_ARG, "multi-field launches take no received seam sums");
+    if (a.nfields > 1 && a.drva) {
+        // the general kernels write the boundary values of one variable
+        for (int f = 0; f < a.nfields; f++) {
+            LineArgs b = a;
+            b.in += f * a.fstride;
+            b.out += f * a.ostride;
+            b.var += f;
+            b.nfields = 1;
+            const int rc = launch_line(op, axis, K, b, s);
+            if (rc) return rc;
+        }
+        return CS_OK;
+    }
     if ((long)a.P * K < a.N) return fail(CS_ERR_SHAPE, "chunks do not cover the line");
     if (axis == 0 && (size_t)a.N * (kXLines + 1) * 8 + 4 * (size_t)a.P * kXLines * 8 > 160 * 1024)
         return fail(CS_ERR_SHAPE, "x line too long for the LDS tile");
@@ -821,7 +834,8 @@ void choose_kernel(const LineOpTable& t, int op, int axis, LineArgs* a, int* K) 
 }
 
 int line_apply(cs_numerics* num, int op, int axis, const double* in, double* out, int start, int end,
-               const double* recv, int var, bool write_drva, hipStream_t s, int nfields) {
+               const double* recv, int var, bool write_drva, hipStream_t s, int nfields, long fstride,
+               long ostride) {
     if (axis < 0 || axis > 2) return fail(CS_ERR_ARG, "axis must be 0, 1 or 2");
     if (!in || !out) return fail(CS_ERR_ARG, "null field pointer");
     if (op == OP_DERIV && (start == 1 || end == 1) && !num->table_set)
@@ -846,7 +860,8 @@ int line_apply(cs_numerics* num, int op, int axis, const double* in, double* out
     a.cyclic = (op == OP_FILTER) ? (start == 1 && end == 1) : 0;
     a.mixed = num->precision;
     a.nfields = nfields;
-    a.fstride = num->g.lmx;
+    a.fstride = fstride ? fstride : num->g.lmx;
+    a.ostride = ostride ? ostride : num->g.lmx;
     int K = 0;
     choose_kernel(*t, op, axis, &a, &K);
     return launch_line(op, axis, K, a, s);

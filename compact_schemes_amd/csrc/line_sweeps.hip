@@ -10,7 +10,7 @@ namespace cs {
 namespace fused {
 
 // One field from `in` to `out` (which may be the same: every row of a line is
-// loaded before one is stored); grid.y runs fields fstride apart.
+// loaded before one is stored); grid.y runs fields fstride (ostride) apart.
 template <bool FILTER>
 struct LineSweep {
     static constexpr int NF = 1;
@@ -26,16 +26,15 @@ struct LineSweep {
     static constexpr bool kEnds = !FILTER;
     const double* in;
     double* out;
-    long fstride;
+    long fstride, ostride;
     double* drva;     // [2 face][5 var][nface] from the first field's variable on, or null
     long nface;
     struct Raw { double q; };
-    __device__ __forceinline__ long field() const { return (long)blockIdx.y * fstride; }
     template <bool NT>
-    __device__ __forceinline__ void load(uoff bo, Raw& w) const { w.q = ldg<NT>(in + field(), bo); }
+    __device__ __forceinline__ void load(uoff bo, Raw& w) const { w.q = ldg<NT>(in + (long)blockIdx.y * fstride, bo); }
     __device__ __forceinline__ void eval(const Raw& w, double* v) const { v[0] = w.q; }
     template <bool NT>
-    __device__ __forceinline__ void store(uoff bo, const double* d) const { stg<NT>(out + field(), bo, d[0]); }
+    __device__ __forceinline__ void store(uoff bo, const double* d) const { stg<NT>(out + (long)blockIdx.y * ostride, bo, d[0]); }
     // boundary derivatives for the characteristic BCs
     __device__ __forceinline__ void end_value(int face, long line, double v) const {
         if (drva) drva[((long)face * kNV + (long)blockIdx.y) * nface + line] = v;
@@ -74,6 +73,7 @@ static LineSweep<FILTER> sweep_of(const LineArgs& a) {
     w.in = a.in;
     w.out = a.out;
     w.fstride = a.fstride;
+    w.ostride = a.ostride;
     w.nface = a.nlines;
     w.drva = a.drva ? a.drva + (long)a.var * a.nlines : nullptr;
     return w;

@@ -33,10 +33,11 @@ __global__ void __launch_bounds__(kBlock) primitives_kernel(const double* qa, do
 }
 
 // calc_fluxes_pre_compute_kernel, src/cuda/kernels/physics.hpp:42-193
-// (D21 intended: stress/heat are not read when Visc is false).
+// (D21 intended: stress/heat are not read when Visc is false; the E + p it
+// leaves in de is overwritten by the flux divergence and not written here).
 template <bool Visc>
 __global__ void __launch_bounds__(kBlock) fluxes_pre_kernel(double* buffer, const double* qa, const double* pr,
-                                                            double* de, const double* xim, const double* etm,
+                                                            const double* de, const double* xim, const double* etm,
                                                             const double* zem, const double* stress,
                                                             const double* heat, cs_point umf, long lmx) {
     long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -55,60 +56,46 @@ __global__ void __launch_bounds__(kBlock) fluxes_pre_kernel(double* buffer, cons
     flux_all<Visc>(q, pr[t], u, mt, tau, hf, umf, F);
     for (int m = 0; m < 5; m++)
         for (int j = 0; j < 3; j++) buffer[t + (long)j * lmx + (long)m * 3 * lmx] = F[m][j];
-    de[t + 4 * lmx] = q[4] + pr[t];
 }
 
-// calc_fluxes_post_compute_kernel<m>, src/cuda/kernels/physics.hpp:195-209
-__global__ void __launch_bounds__(kBlock) fluxes_post_kernel(double* de, const double* bd, int m, long lmx) {
+// calc_fluxes_post_compute_kernel<m>, src/cuda/kernels/physics.hpp:195-209,
+// for all five variables
+__global__ void __launch_bounds__(kBlock) fluxes_post_kernel(double* de, const double* bd, long lmx) {
     long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= lmx) return;
-    const double* d = bd + (long)m * 3 * lmx;
-    de[t + (long)m * lmx] = d[t] + d[t + lmx] + d[t + 2 * lmx];
+    double d[kNV][3];
+    for (int m = 0; m < kNV; m++)
+        for (int j = 0; j < 3; j++) d[m][j] = bd[t + (long)(3 * m + j) * lmx];
+    for (int m = 0; m < kNV; m++) de[t + (long)m * lmx] = d[m][0] + d[m][1] + d[m][2];
 }
 
-// calc_viscous_shear_stress_init_kernel, src/cuda/kernels/physics.hpp:211-225
-__global__ void __launch_bounds__(kBlock) visc_init_kernel(double* buffer, const double* de, long lmx) {
+// calc_viscous_shear_stress_post_compute_kernel<m> (m = 1..4) and
+// calc_viscous_shear_stress_final_kernel, src/cuda/kernels/physics.hpp:228-333,
+// D8 intended (reads the derivatives): the physical gradients of u, v, w, c^2
+// from the index-space ones bd[m][3] and the metrics, then stress and heat
+// flux.  The reference passes the twelve gradients through the stress and
+// heat arrays (five kernels, 84 fields read or written); in registers the
+// 26 reads and 11 writes are left, and they are the bound (160x128x96: five
+// kernels 229 us, this one 108 = 5.4 TB/s).
+__global__ void __launch_bounds__(kBlock) visc_kernel(double* de, const double* ssk, const double* yaco,
+                                                      const double* bd, const double* xim, const double* etm,
+                                                      const double* zem, double* stress, double* heat, long lmx) {
     long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= lmx) return;
-    for (int m = 1; m < 5; m++) buffer[t + (long)m * 3 * lmx] = de[t + (long)m * lmx];
-}
-
-// calc_viscous_shear_stress_post_compute_kernel<m>, src/cuda/kernels/physics.hpp:228-283,
-// D8 intended (reads the derivatives).  Slot map as the reference: m=1 ->
-// (S.xx, H.zz, S.zx), m=2 -> (S.xy, S.yy, H.xx), m=3 -> (H.yy, S.yz, S.zz), m=4 -> ss.
-__global__ void __launch_bounds__(kBlock) visc_post_kernel(double* stress, double* heat, double* ss,
-                                                           const double* bd, const double* xim,
-                                                           const double* etm, const double* zem, int m,
-                                                           long lmx) {
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= lmx) return;
-    double *o0, *o1, *o2;
-    if (m == 1)      { o0 = stress;           o1 = heat + 2 * lmx;   o2 = stress + 5 * lmx; }
-    else if (m == 2) { o0 = stress + 3 * lmx; o1 = stress + lmx;     o2 = heat; }
-    else if (m == 3) { o0 = heat + lmx;       o1 = stress + 4 * lmx; o2 = stress + 2 * lmx; }
-    else             { o0 = ss;               o1 = ss + lmx;         o2 = ss + 2 * lmx; }
-    const double* d = bd + (long)m * 3 * lmx;
-    double f0 = d[t], f1 = d[t + lmx], f2 = d[t + 2 * lmx];
-    o0[t] = xim[t] * f0 + etm[t] * f1 + zem[t] * f2;
-    o1[t] = xim[t + lmx] * f0 + etm[t + lmx] * f1 + zem[t + lmx] * f2;
-    o2[t] = xim[t + 2 * lmx] * f0 + etm[t + 2 * lmx] * f1 + zem[t + 2 * lmx] * f2;
-}
-
-// calc_viscous_shear_stress_final_kernel, src/cuda/kernels/physics.hpp:285-333
-__global__ void __launch_bounds__(kBlock) visc_final_kernel(double* de, const double* ssk, const double* yaco,
-                                                            const double* ss, double* stress, double* heat,
-                                                            long lmx) {
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= lmx) return;
-    double g[9];   // (u_x, u_y, u_z, v_x, v_y, v_z, w_x, w_y, w_z) from the slot map
-    g[0] = stress[t];           g[1] = heat[t + 2 * lmx];   g[2] = stress[t + 5 * lmx];
-    g[3] = stress[t + 3 * lmx]; g[4] = stress[t + lmx];     g[5] = heat[t];
-    g[6] = heat[t + lmx];       g[7] = stress[t + 4 * lmx]; g[8] = stress[t + 2 * lmx];
-    double c2g[3] = {ss[t], ss[t + lmx], ss[t + 2 * lmx]};
-    double u[3] = {de[t + lmx], de[t + 2 * lmx], de[t + 3 * lmx]};
+    double mt[3][3], f[4][3], u[3];
+    for (int d = 0; d < 3; d++) {
+        mt[0][d] = xim[t + d * lmx]; mt[1][d] = etm[t + d * lmx]; mt[2][d] = zem[t + d * lmx];
+        u[d] = de[t + (d + 1) * lmx];
+    }
+    for (int m = 0; m < 4; m++)
+        for (int j = 0; j < 3; j++) f[m][j] = bd[t + (long)(3 * (m + 1) + j) * lmx];
+    const double mu = ssk[t], J = yaco[t];
+    double g[12];   // (u_x, u_y, u_z, v_x, v_y, v_z, w_x, w_y, w_z, c2_x, c2_y, c2_z)
+    for (int m = 0; m < 4; m++)
+        for (int d = 0; d < 3; d++) g[3 * m + d] = mt[0][d] * f[m][0] + mt[1][d] * f[m][1] + mt[2][d] * f[m][2];
     double tau[6], hf[3], d4;
-    viscous_closure(ssk[t], yaco[t], g, c2g, u, tau, hf, &d4);
-    de[t] = ssk[t];
+    viscous_closure(mu, J, g, g + 9, u, tau, hf, &d4);
+    de[t] = mu;
     de[t + 4 * lmx] = d4;
     for (int k = 0; k < 6; k++) stress[t + k * lmx] = tau[k];
     for (int k = 0; k < 3; k++) heat[t + k * lmx] = hf[k];
@@ -237,9 +224,9 @@ int launch_primitives(const double* qa, double* de, double* p, long lmx, hipStre
     return CS_OK;
 }
 
-int launch_fluxes_pre(bool visc, double* buffer, const double* qa, const double* p, double* de, const double* xim,
-                      const double* etm, const double* zem, const double* stress, const double* heat,
-                      cs_point umf, long lmx, hipStream_t s) {
+int launch_fluxes_pre(bool visc, double* buffer, const double* qa, const double* p, const double* de,
+                      const double* xim, const double* etm, const double* zem, const double* stress,
+                      const double* heat, cs_point umf, long lmx, hipStream_t s) {
     if (visc)
         hipLaunchKernelGGL(fluxes_pre_kernel<true>, grid_for(lmx), dim3(kBlock), 0, s, buffer, qa, p, de, xim, etm,
                            zem, stress, heat, umf, lmx);
@@ -250,29 +237,16 @@ int launch_fluxes_pre(bool visc, double* buffer, const double* qa, const double*
     return CS_OK;
 }
 
-int launch_fluxes_post(double* de, const double* bd, int m, long lmx, hipStream_t s) {
-    hipLaunchKernelGGL(fluxes_post_kernel, grid_for(lmx), dim3(kBlock), 0, s, de, bd, m, lmx);
+int launch_fluxes_post(double* de, const double* bd, long lmx, hipStream_t s) {
+    hipLaunchKernelGGL(fluxes_post_kernel, grid_for(lmx), dim3(kBlock), 0, s, de, bd, lmx);
     CS_HIP(hipGetLastError());
     return CS_OK;
 }
 
-int launch_visc_init(double* buffer, const double* de, long lmx, hipStream_t s) {
-    hipLaunchKernelGGL(visc_init_kernel, grid_for(lmx), dim3(kBlock), 0, s, buffer, de, lmx);
-    CS_HIP(hipGetLastError());
-    return CS_OK;
-}
-
-int launch_visc_post(double* stress, double* heat, double* ss, const double* bd, const double* xim,
-                     const double* etm, const double* zem, int m, long lmx, hipStream_t s) {
-    hipLaunchKernelGGL(visc_post_kernel, grid_for(lmx), dim3(kBlock), 0, s, stress, heat, ss, bd, xim, etm, zem, m,
+int launch_visc(double* de, const double* ssk, const double* yaco, const double* bd, const double* xim,
+                const double* etm, const double* zem, double* stress, double* heat, long lmx, hipStream_t s) {
+    hipLaunchKernelGGL(visc_kernel, grid_for(lmx), dim3(kBlock), 0, s, de, ssk, yaco, bd, xim, etm, zem, stress, heat,
                        lmx);
-    CS_HIP(hipGetLastError());
-    return CS_OK;
-}
-
-int launch_visc_final(double* de, const double* ssk, const double* yaco, const double* ss, double* stress,
-                      double* heat, long lmx, hipStream_t s) {
-    hipLaunchKernelGGL(visc_final_kernel, grid_for(lmx), dim3(kBlock), 0, s, de, ssk, yaco, ss, stress, heat, lmx);
     CS_HIP(hipGetLastError());
     return CS_OK;
 }

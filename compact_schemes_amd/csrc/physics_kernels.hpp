@@ -140,15 +140,12 @@ struct EigT {
 using Eig = EigT<double>;
 
 int launch_primitives(const double* qa, double* de, double* p, long lmx, hipStream_t s);
-int launch_fluxes_pre(bool visc, double* buffer, const double* qa, const double* p, double* de, const double* xim,
-                      const double* etm, const double* zem, const double* stress, const double* heat,
-                      cs_point umf, long lmx, hipStream_t s);
-int launch_fluxes_post(double* de, const double* bd, int m, long lmx, hipStream_t s);
-int launch_visc_init(double* buffer, const double* de, long lmx, hipStream_t s);
-int launch_visc_post(double* stress, double* heat, double* ss, const double* bd, const double* xim,
-                     const double* etm, const double* zem, int m, long lmx, hipStream_t s);
-int launch_visc_final(double* de, const double* ssk, const double* yaco, const double* ss, double* stress,
-                      double* heat, long lmx, hipStream_t s);
+int launch_fluxes_pre(bool visc, double* buffer, const double* qa, const double* p, const double* de,
+                      const double* xim, const double* etm, const double* zem, const double* stress,
+                      const double* heat, cs_point umf, long lmx, hipStream_t s);
+int launch_fluxes_post(double* de, const double* bd, long lmx, hipStream_t s);
+int launch_visc(double* de, const double* ssk, const double* yaco, const double* bd, const double* xim,
+                const double* etm, const double* zem, double* stress, double* heat, long lmx, hipStream_t s);
 int time_step_blocks(long lmx);
 int launch_time_step(const double* xim, const double* etm, const double* zem, const double* de, const double* yaco,
                      const double* ssk, cs_point umf, double* part, int nblocks, long lmx, hipStream_t s);

@@ -27,7 +27,6 @@ class Stepper:
         self.de = torch.zeros(5 * self.lmx, dtype=torch.float64, device="cuda")
         self.p = torch.zeros(self.lmx, dtype=torch.float64, device="cuda")
         self.q0 = torch.zeros(5 * self.lmx, dtype=torch.float64, device="cuda")
-        self.work = torch.zeros(self.lmx, dtype=torch.float64, device="cuda")
         self.char = any(c in (10, 20, 25, 30) for row in nbc for c in row)
 
     def time_step(self, q, cfl):
@@ -54,8 +53,6 @@ class Stepper:
         if filt:
             for v in range(5):
                 f = q[v * self.lmx:(v + 1) * self.lmx]
-                self.num.filter(0, f, self.work)
-                self.num.filter(1, self.work, f)
-                self.num.filter(2, f, self.work)
-                f.copy_(self.work)
+                for axis in range(3):
+                    self.num.filter(axis, f, f)
         return dt

@@ -144,7 +144,8 @@ int cs_physics_destroy(cs_physics* phys);
 int cs_physics_set_frame(cs_physics* phys, cs_point umf, cs_point dudtmf);
 /* stress = [6][lmx] (xx,yy,zz,xy,yz,zx), heat = [3][lmx] (xx,yy,zz):
  * the device storage behind physics_base::stress_tensor / heat_fluxes,
- * src/physics_base.hpp:57-86. */
+ * src/physics_base.hpp:57-86.  buffer and buffer_deriv = [5 var][3][lmx], scratch:
+ * the fluxes of calc_fluxes and the index-space derivatives of the last call. */
 int cs_physics_buffers(cs_physics* phys, double** stress, double** heat, double** buffer,
                        double** buffer_deriv);
 
