@@ -188,13 +188,6 @@ int one_sweep(cs_solver* sv, int which, const double* q, const double* sbcc, dou
     return sweep_at(sv, which, cm, q, out, nullptr, 0, s);
 }
 
-bool filter_fusable(const cs_solver* sv) {
-    for (int a = 0; a < 3; a++)
-        if (sv->ax[a].K != 8 || sv->ax[a].N != sv->ax[a].P * 8 || sv->ax[a].P > kMaxP || !sv->ax[a].ftab)
-            return false;
-    return true;
-}
-
 bool filter_axis_fused(const cs_solver* sv, int a) { return sv->fax[a].ftab != nullptr; }
 
 bool filter_axis_tunable(const cs_solver* sv, int a) {

@@ -41,6 +41,11 @@ struct AxisDesc {
     int ftl;
 };
 
+// y or z lines that 16-point chunks can cut (whole first and last chunks)
+inline bool fits16(const AxisDesc& ax, int axis) {
+    return axis > 0 && ax.K == 8 && ax.N >= 32 && chunks_fit(ax.N, (ax.N + 15) / 16, 16);
+}
+
 // per-point geometry of a curvilinear solver (cs_solver_set_metrics; caller's
 // device arrays): m[a][k] = component k of the metric row of axis a (xim, etm,
 // zem of the reference, [3][lmx] each), J = yaco [lmx], cm[a] = the face
@@ -65,7 +70,7 @@ struct cs_solver {
     cs_solver_config cfg;
     cs::Geo g;
     cs_numerics* num = nullptr;         // interface table, filter operators
-    cs::fused::AxisDesc ax[3];     // 8-point chunks up to 256 points: filter sweeps, adjoint sweeps
+    cs::fused::AxisDesc ax[3];     // 8-point chunks along x and up to 256 points
     // the right-hand-side sweeps: ax, or the same axis cut into 16-point
     // chunks (cs_solver_tune variant 2, with tabs16)
     cs::fused::AxisDesc rax[3];
@@ -94,8 +99,10 @@ struct cs_solver {
     double* dt = nullptr;      // [0] dt, [1..2] maxima
     double* dt_host = nullptr; // pinned
     double* vjp = nullptr;     // [41][lmx] adjoint scratch (allocated on the first adjoint call)
-    // adjoint sweeps (tape.hip, set up on the first call that needs them)
-    double* ttabs[3] = {nullptr, nullptr, nullptr};   // LU of A^T of the derivative, 8-point chunks
+    // adjoint sweeps (tape.hip, set up on the first call that needs them):
+    // the axes with the transposed tables of the derivative and of the filter
+    cs::fused::AxisDesc tax[3]{}, ftax[3]{};
+    double* ttabs[3] = {nullptr, nullptr, nullptr};   // LU of A^T of the derivative
     double* fttabs[3] = {nullptr, nullptr, nullptr};  // LU of A^T of the closure-line filter
     double* adj = nullptr;     // seed, accumulator (5 fields each), face buffers, internal tape
     double* rec = nullptr;     // faces of the RHS being evaluated go here when set ([3 axes][2][5][face])
@@ -128,8 +135,6 @@ int time_step(cs_solver* sv, const double* q, double dt_fixed, hipStream_t s);
 int dt_fold_pos(const cs_solver* sv);
 int one_sweep(cs_solver* sv, int which, const double* q, const double* sbcc, double* out, hipStream_t s);
 void chunk_table(const std::vector<double>& h, int n, int K, int P, std::vector<double>& out);
-// every axis filters with the 8-point fused sweep of ax (the adjoint's assumption)
-bool filter_fusable(const cs_solver* sv);
 // the filter along axis a runs a fused sweep (fax), else the line solver
 bool filter_axis_fused(const cs_solver* sv, int a);
 // that sweep runs equal chunks and takes the shapes of cs_solver_tune_filter

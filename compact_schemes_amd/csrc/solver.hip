@@ -130,11 +130,6 @@ int cs_solver_destroy(cs_solver* sv) {
     return CS_OK;
 }
 
-// y or z lines that 16-point chunks can cut (whole first and last chunks)
-static bool fits16(const AxisDesc& ax, int axis) {
-    return axis > 0 && ax.K == 8 && ax.N >= 32 && chunks_fit(ax.N, (ax.N + 15) / 16, 16);
-}
-
 // the shapes cs_solver_tune offers on 16-point chunks: equal ones
 static int check_chunks16(const AxisDesc& ax, int axis) {
     if (axis == 0 || ax.K != 8 || ax.N % 16 != 0 || ax.N < 32)
@@ -142,8 +137,7 @@ static int check_chunks16(const AxisDesc& ax, int axis) {
     return CS_OK;
 }
 
-// the right-hand-side sweeps of `axis` on 16-point chunks; the adjoint sweeps
-// keep 8-point chunks
+// the right-hand-side sweeps of `axis` on 16-point chunks
 static int use_chunks16(cs_solver* sv, int axis, int lines, int xcd) {
     const AxisDesc& ax = sv->ax[axis];
     if (!fits16(ax, axis)) return fail(CS_ERR_UNSUPPORTED, "16-point chunks do not cut this line");

@@ -21,7 +21,7 @@
 // Tape of one step: the stage states q0..q3 and, for every stage, the
 // boundary derivatives of the flux divergence along each axis (what the
 // characteristic BC linearises about), [4 stages][3 axes][2 face][5][face].
-#include "sweep_parts.hpp"
+#include "fused_kernels.hpp"
 #include "vjp_parts.hpp"
 
 namespace cs {
@@ -78,63 +78,85 @@ __device__ __forceinline__ void flux_jt_m(const double* q, const double* nu, con
 template <int AX, int MODE, bool CURV = false>
 struct AT {
     static constexpr int NF = 5;
+    static constexpr bool kFilter = false;
     static constexpr int kWpe = 3;        // waves per SIMD of the y/z kernels (168 VGPRs)
+    // bytes a point: seed, q, result; the accumulator; lam (and the next seed)
+    static constexpr int kBytes = 120 + (MODE > 0 ? 40 : 0) + (MODE == 2 ? 80 : MODE == 3 ? 40 : 0) + (CURV ? 24 : 0);
     const double* q[5];       // the stage state the RHS was evaluated at
     const double* t[5];       // seed
     const double* gin[5];
     double* gout[5];
     double* lam[5];
     double* tout[5];
-    const double* G;          // [2 face][5][nface] face-point terms, or null
+    const double* mu;         // [2 face][5][nface] face seeds (added to the seed at the face rows), or null
+    const double* G;          // the same layout, face-point terms
     long nface;
     double ck;
     double m, uf;
     cs_point umf;
     Metric mt;
+    template <bool NT>
     __device__ __forceinline__ void seed(uoff bo, double* v) const {
 #pragma unroll
-        for (int f = 0; f < 5; f++) v[f] = ldg(t[f], bo);
+        for (int f = 0; f < 5; f++) v[f] = ldg<NT>(t[f], bo);
     }
-    // J^T nu at one point folded into d with the stage's combination (loads
-    // only); store() then writes.  The kernels fetch all their points before
-    // their first store: the outputs may alias q, gin or lam for all the
-    // compiler knows, so a load placed after a store waits for it.
-    __device__ __forceinline__ void fetch(uoff bo, double* d, int face, long line) const {
-        double qq[5], g[5];
-        const double c = ck;
+    __device__ __forceinline__ void face_seed(int face, long line, double* v) const {
+        if (!mu) return;
 #pragma unroll
-        for (int v = 0; v < 5; v++) qq[v] = ldg(q[v], bo);
-        if constexpr (CURV) {
-            const double mr[3] = {ldg(mt.m[AX][0], bo), ldg(mt.m[AX][1], bo), ldg(mt.m[AX][2], bo)};
-            flux_jt_m(qq, d, mr, umf, g);
-        } else {
-            flux_jt<AX>(qq, d, m, uf, g);
+        for (int f = 0; f < 5; f++) v[f] += mu[(face * 5 + f) * nface + line];
+    }
+    // what a point's result needs (loads only), the result from it and nu (in
+    // d; face: 0, 1 at a face point, else -1), and its stores: the kernels
+    // issue the loads of the next rows before a row's stores, which may alias
+    // them for all the compiler knows
+    struct Out {
+        double q[5];
+        double g[MODE > 0 ? 5 : 1], l[MODE > 1 ? 5 : 1], m[CURV ? 3 : 1];
+    };
+    template <bool NT>
+    __device__ __forceinline__ void load_out(uoff bo, Out& e) const {
+#pragma unroll
+        for (int v = 0; v < 5; v++) e.q[v] = ldg<NT>(q[v], bo);
+        if constexpr (MODE > 0) {
+#pragma unroll
+            for (int v = 0; v < 5; v++) e.g[v] = ldg<NT>(gin[v], bo);
         }
+        if constexpr (MODE > 1) {
+#pragma unroll
+            for (int v = 0; v < 5; v++) e.l[v] = ldg<NT>(lam[v], bo);
+        }
+        if constexpr (CURV) {
+#pragma unroll
+            for (int k = 0; k < 3; k++) e.m[k] = ldg<NT>(mt.m[AX][k], bo);
+        }
+    }
+    __device__ __forceinline__ void combine(Out& e, double* d, int face, long line) const {
+        double g[5];
+        const double c = ck;
+        if constexpr (CURV) flux_jt_m(e.q, d, e.m, umf, g);
+        else flux_jt<AX>(e.q, d, m, uf, g);
         if (G && face >= 0) {
 #pragma unroll
             for (int v = 0; v < 5; v++) g[v] += G[(face * 5 + v) * nface + line];
         }
 #pragma unroll
         for (int v = 0; v < 5; v++) {
-            if (MODE == 0) d[v] = g[v];
-            else if (MODE == 1) d[v] = ldg(gin[v], bo) + g[v];
-            else if (MODE == 2) d[v] = -c * (ldg(gin[v], bo) + g[v]);
-            else d[v] = ldg(lam[v], bo) - c * (ldg(gin[v], bo) + g[v]);
+            if constexpr (MODE == 0) d[v] = g[v];
+            else if constexpr (MODE == 1) d[v] = e.g[v] + g[v];
+            else if constexpr (MODE == 2) { d[v] = -c * (e.g[v] + g[v]); e.l[v] = e.l[v] + d[v]; }
+            else d[v] = e.l[v] - c * (e.g[v] + g[v]);
         }
     }
-    __device__ __forceinline__ void store(uoff bo, const double* d) const {
-        if (MODE == 2) {
-            double l[5];
+    template <bool NT>
+    __device__ __forceinline__ void store(uoff bo, const double* d, const double* l) const {
 #pragma unroll
-            for (int v = 0; v < 5; v++) l[v] = ldg(lam[v], bo);
-#pragma unroll
-            for (int v = 0; v < 5; v++) {
-                stg(tout[v], bo, d[v]);
-                stg(lam[v], bo, l[v] + d[v]);
+        for (int v = 0; v < 5; v++) {
+            if constexpr (MODE == 2) {
+                stg<NT>(tout[v], bo, d[v]);
+                stg<NT>(lam[v], bo, l[v]);
+            } else {
+                stg<NT>(MODE == 3 ? lam[v] : gout[v], bo, d[v]);
             }
-        } else {
-#pragma unroll
-            for (int v = 0; v < 5; v++) stg(MODE == 3 ? lam[v] : gout[v], bo, d[v]);
         }
     }
 };
@@ -144,49 +166,52 @@ struct AT {
 template <int NFV>
 struct FT {
     static constexpr int NF = NFV;
-    static constexpr int kWpe = NFV == 1 ? 4 : 2;
+    static constexpr bool kFilter = true;
+    static constexpr int kWpe = 4;
+    static constexpr int kBytes = 16 * NFV;
     double* q;
     long lmx;
+    const double* an;         // the filter's coefficient sets (filter_bt)
     __device__ __forceinline__ double* field(int f) const {
         return q + (long)(NFV == 1 ? (int)blockIdx.y : f) * lmx;
     }
+    template <bool NT>
     __device__ __forceinline__ void seed(uoff bo, double* v) const {
 #pragma unroll
-        for (int f = 0; f < NFV; f++) v[f] = ldg(field(f), bo);
+        for (int f = 0; f < NFV; f++) v[f] = ldg<NT>(field(f), bo);
     }
-    __device__ __forceinline__ void fetch(uoff, double*, int, long) const {}
-    __device__ __forceinline__ void store(uoff bo, const double* d) const {
+    __device__ __forceinline__ void face_seed(int, long, double*) const {}
+    struct Out { double l[1]; };
+    template <bool NT>
+    __device__ __forceinline__ void load_out(uoff, Out&) const {}
+    __device__ __forceinline__ void combine(Out&, double*, int, long) const {}
+    template <bool NT>
+    __device__ __forceinline__ void store(uoff bo, const double* d, const double*) const {
 #pragma unroll
-        for (int f = 0; f < NFV; f++) stg(field(f), bo, d[f]);
+        for (int f = 0; f < NFV; f++) stg<NT>(field(f), bo, d[f]);
     }
 };
 
-// B^T of the derivative on the K rows of chunk c from a window w holding rows
-// s-2+u (wrapped on seam lines).  Rows i in [2, N-3] are interior rows, so
-// column j receives B[i][j] = +bb, +aa, -aa, -bb from i = j-2, j-1, j+1, j+2;
-// the closure rows (forward_system in adjoint.hip; build_system,
-// src/cuda/kernels/numerics_device_pc.hpp:176-293) or the seam rows
-// (pbci on the own side, pbco on the far side of the wrap) add at the ends.
+// B^T of the derivative on the rows of a chunk from a window w holding rows
+// s-2+u (wrapped on seam lines; `last` chunks are whole).  Rows i in [2, N-3]
+// are interior rows, so column j receives B[i][j] = +bb, +aa, -aa, -bb from
+// i = j-2, j-1, j+1, j+2: the same formula in every chunk with the other rows
+// of the window taken as zero.  The closure rows (forward_system in
+// adjoint.hip; build_system, src/cuda/kernels/numerics_device_pc.hpp:176-293)
+// or the seam rows (pbci on the own side, pbco on the far side of the wrap)
+// add at the ends.
 template <int K>
-__device__ __forceinline__ void deriv_bt(const double (&w)[K + 4], double (&o)[K], int s, int N, int c, int P,
-                                         bool seam, const double* pb) {
-    if (c > 0 && c < P - 1) {
+__device__ __forceinline__ void deriv_bt(const double (&w)[K + 4], double (&o)[K], bool first, bool last, bool seam,
+                                         const double* pb) {
+    double v[K + 4];
 #pragma unroll
-        for (int t = 0; t < K; t++) o[t] = kAa * (w[t + 1] - w[t + 3]) + kBb * (w[t] - w[t + 4]);
-        return;
-    }
+    for (int u = 0; u < K + 4; u++)
+        v[u] = u < 4 ? (first ? 0.0 : w[u]) : u >= K ? (last ? 0.0 : w[u]) : w[u];
 #pragma unroll
-    for (int t = 0; t < K; t++) {
-        const int j = s + t;
-        double acc = 0.0;
-        if (j - 2 >= 2 && j - 2 <= N - 3) acc += kBb * w[t];
-        if (j - 1 >= 2 && j - 1 <= N - 3) acc += kAa * w[t + 1];
-        if (j + 1 >= 2 && j + 1 <= N - 3) acc -= kAa * w[t + 3];
-        if (j + 2 >= 2 && j + 2 <= N - 3) acc -= kBb * w[t + 4];
-        o[t] = acc;
-    }
+    for (int t = 0; t < K; t++) o[t] = kAa * (v[t + 1] - v[t + 3]) + kBb * (v[t] - v[t + 4]);
+    if (!first && !last) return;
     if (!seam) {
-        if (c == 0) {
+        if (first) {
             const double y0 = w[2], y1 = w[3];
             o[0] += kAb00 * y0 - kAb10 * y1;
             o[1] += kAb01 * y0;
@@ -201,7 +226,7 @@ __device__ __forceinline__ void deriv_bt(const double (&w)[K + 4], double (&o)[K
         static_assert(K == kLmd, "seam columns span one 8-point chunk");
         const double* pbco = pb;              // pbco[16] | pbci[16]
         const double* pbci = pb + 2 * kLmd;
-        if (c == 0) {
+        if (first) {
             const double y0 = w[2], y1 = w[3], yN1 = w[1], yN2 = w[0];
 #pragma unroll
             for (int t = 0; t < K; t++)
@@ -209,152 +234,170 @@ __device__ __forceinline__ void deriv_bt(const double (&w)[K + 4], double (&o)[K
         } else {
             const double y0 = w[K + 2], y1 = w[K + 3], yN1 = w[K + 1], yN2 = w[K];
 #pragma unroll
-            for (int t = 0; t < K; t++) {
-                const int i = K - 1 - t;
-                o[t] += pbco[i] * y0 + pbco[kLmd + i] * y1 - pbci[i] * yN1 - pbci[kLmd + i] * yN2;
-            }
+            for (int i = 0; i < K; i++)
+                o[K - 1 - i] += pbco[i] * y0 + pbco[kLmd + i] * y1 - pbci[i] * yN1 - pbci[kLmd + i] * yN2;
         }
     }
 }
 
-// B^T of the closure-line filter from a window w holding rows s-5+u: column j
-// receives B[i][j] from rows i = j-5..j+5, where row i has order 2*min(d,5),
-// d = min(i, N-1-i) its distance from the nearer end, and is the identity at
-// d = 0 (an + 6M = coefficient set M, as in filter_rhs of fused.hip)
+// B^T of the closure-line filter from a window w holding rows s-5+u: row i has
+// order 2*M, M = min(d, 5), d its distance from the nearer end, and is the
+// identity at d = 0 (an + 6M = coefficient set M, as in filter_rhs).  Every
+// chunk runs the order-10 formula with the rows next to the ends (d < 5) and
+// past them taken as zero; those rows reach M columns each way, so they add in
+// the end chunks and, of 8-point chunks, row d = 4 one column beyond.
 template <int K>
-__device__ __forceinline__ void filter_bt(const double (&w)[K + 10], double (&o)[K], int s, int N, int c, int P,
+__device__ __forceinline__ void filter_bt(const double (&w)[K + 10], double (&o)[K], int c, int P, bool whole,
                                           const double* an) {
     constexpr int H = 5;
-    if (c >= 2 && c <= P - 3) {
+    const bool first = c == 0, last = c == P - 1;
+    // rows next to the ends in the neighbour chunk's window (K = 8: d = 3, 4)
+    const bool second = K == 8 && c == 1, before = K == 8 && c == P - 2;
+    double v[K + 10];
 #pragma unroll
-        for (int t = 0; t < K; t++) {
-            double v = an[30] * w[t + H];
-#pragma unroll
-            for (int m = 1; m <= 5; m++) v += 0.5 * an[30 + m] * (w[t + H + m] + w[t + H - m]);
-            o[t] = v;
-        }
-        return;
+    for (int u = 0; u < K + 10; u++) {
+        bool zero = false;
+        if (u < 2 * H) zero |= first;
+        if (u < 2) zero |= second;
+        if (u >= K) zero |= last;
+        if (u >= K + 8) zero |= before;
+        if (u == K + 7) zero |= before && !whole;
+        v[u] = zero ? 0.0 : w[u];
     }
 #pragma unroll
     for (int t = 0; t < K; t++) {
-        const int j = s + t;
-        double acc = 0.0;
+        double x = an[30] * v[t + H];
 #pragma unroll
-        for (int m = -H; m <= H; m++) {
-            const int i = j + m;
-            if (i < 0 || i >= N) continue;
-            const int d = min(i, N - 1 - i);
-            const int am = m < 0 ? -m : m;
-            double cf = 0.0;
-            if (d == 0) {
-                cf = m == 0 ? 1.0 : 0.0;
-            } else {
-                const int M = min(d, H);
-                if (am <= M) cf = am == 0 ? an[6 * M] : 0.5 * an[6 * M + am];
+        for (int m = 1; m <= 5; m++) x += 0.5 * an[30 + m] * (v[t + H + m] + v[t + H - m]);
+        o[t] = x;
+    }
+    if (first || last) {
+        // row at distance M from the end into the column at distance e
+#pragma unroll
+        for (int M = 0; M < H; M++) {
+            const double y = first ? w[H + M] : w[K + H - 1 - M];
+#pragma unroll
+            for (int e = 0; e <= 2 * M && e < K; e++) {
+                const int am = e < M ? M - e : e - M;
+                const double cf = M == 0 ? 1.0 : am == 0 ? an[6 * M] : 0.5 * an[6 * M + am];
+                if (first) o[e] += cf * y;
+                else o[K - 1 - e] += cf * y;
             }
-            acc += cf * w[t + H + m];
         }
-        o[t] = acc;
+    }
+    if (second) o[0] += 0.5 * an[28] * w[1];
+    if (before) {
+        if (whole) o[K - 1] += 0.5 * an[28] * w[K + 8];
+        else o[K - 2] += 0.5 * an[28] * w[K + 7];
     }
 }
 
-template <int K, int ST, int W>
-__device__ __forceinline__ void stencil_t(const double (&w)[W], double (&o)[K], int s, int N, int c, int P,
-                                          bool seam, const double* pb, const double* an) {
-    if constexpr (ST == 0)
-        deriv_bt<K>(w, o, s, N, c, P, seam, pb);
-    else
-        filter_bt<K>(w, o, s, N, c, P, an);
+template <int K, class SW, int W>
+__device__ __forceinline__ void stencil_t(const SW& sw, const double (&w)[W], double (&o)[K], int c, int P,
+                                          bool whole, bool seam, const double* pb) {
+    if constexpr (SW::kFilter) filter_bt<K>(w, o, c, P, whole, sw.an);
+    else deriv_bt<K>(w, o, c == 0, c == P - 1, seam, pb);
 }
 
+constexpr int kRowsT = 2;       // rows whose epilogue loads are in flight in the y/z kernel
+constexpr int kPointsT = 3;     // points of a lane in the x kernel
+
 // ---------------------------------------------------------------------------
-// transposed sweep, x lines: one wave holds the chunk groups of 64/GS lines
+// transposed sweep, x lines: one wave holds the chunk groups of 64/P lines
 // (a contiguous run); coalesced loads and stores, LDS transposes field by
-// field, carries by wave scans.  ST: 0 = derivative, 1 = closure filter.
+// field, carries by wave scans.
+//
+// Bound by the 15 fields it reads and 10 it writes: 128^3 MODE 2 116 -> 103 us
+// (4.9 TB/s), MODE 3 95 -> 89.
 // ---------------------------------------------------------------------------
-template <int K, class SW, int ST>
-__global__ void __launch_bounds__(64) xtT_kernel(AxisDesc ax, SweepCommon cm, SW sw, const double* tabT,
-                                                 const double* mu, const double* an) {
+template <int K, class SW, bool EX, bool NT>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
+xtT_kernel(AxisDesc ax, SweepCommon cm, SW sw) {
     constexpr int NF = SW::NF;
     constexpr int J = K;
-    constexpr int H = ST == 0 ? 2 : 5;
+    constexpr int H = SW::kFilter ? 5 : 2;
     constexpr int W = K + 2 * H;
-    static_assert(H <= K, "halo rows come from the neighbouring chunks only");
-    extern __shared__ double lds[];       // [64/GS lines][P chunks][K+1]
+    static_assert(K == 8 && H <= K, "8-point chunks; halo rows come from the neighbouring chunks only");
+    extern __shared__ double lds[];       // [64/P lines][P chunks][K+1], 64 slots for lanes past the run
 
-    const int N = ax.N, P = ax.P;
+    const int N = ax.N, P = ax.P, NP = P * K;
+    const Chunks<K, EX> ch(N, P);
     const int lane = threadIdx.x;
     const int lpw = 64 / P;
-    const long line0 = (long)blockIdx.x * lpw;
+    const long line0 = group_of(ax.xcd) * lpw;
     const int nl = (int)min((long)lpw, ax.nlines - line0);
     const int npts = nl * N;
     const uoff run = line_off(0, (uoff)line0, (uoff)cm.lxi, (uoff)cm.plane);
+    // lanes past the run repeat its last point: no branches around the loads
+    auto off = [&](int j) { return run + (uoff)min(lane + 64 * j, npts - 1) * 8u; };
 
     double xq[NF][J];
 #pragma unroll
     for (int j = 0; j < J; j++) {
-        const int p = lane + 64 * j;
         double x[NF];
-        if (p < npts) {
-            sw.seed(run + (uoff)p * 8u, x);
-        } else {
-#pragma unroll
-            for (int f = 0; f < NF; f++) x[f] = 0.0;
-        }
+        sw.template seed<NT>(off(j), x);
 #pragma unroll
         for (int f = 0; f < NF; f++) xq[f][j] = x[f];
     }
     int slot[J], lrw[J];                 // LDS slot; line << 10 | row
-    {
-        int l = 0, row = lane;
-        while (row >= N) { row -= N; l++; }
 #pragma unroll
-        for (int j = 0; j < J; j++) {
-            slot[j] = lane + 64 * j < npts ? xt_slot<K>(l, P, row / K, row % K) : 0;
-            lrw[j] = (l << 10) | row;
-            row += 64;
-            while (row >= N) { row -= N; l++; }
+    for (int j = 0; j < J; j++) {
+        const int p = lane + 64 * j;
+        // p / N by the reciprocal rounded up: exact for p < 1024, N <= 1024
+        const int l = (int)(((unsigned)p * ((0x1000000u + N - 1) / (unsigned)N)) >> 24), row = p - l * N;
+        int c = row >> 3, t = row & 7;
+        if (!EX && row >= K) {
+            const int q = row - K, cs = (q * (65536 / (K - 1) + 1)) >> 16;   // q / (K-1), exact for q < 1024
+            if (q < (K - 1) * ch.D) { c = cs + 1; t = q - cs * (K - 1); }
+            else { c = (row + ch.D) >> 3; t = (row + ch.D) & 7; }
         }
+        slot[j] = p < npts ? xt_slot<K>(l, P, c, t) : lpw * P * (K + 1) + lane;
+        lrw[j] = (l << 10) | row;
     }
 
     const int li = lane / P, c = lane % P;
     const bool work = li < nl;
     const int lr = work ? li : 0;
     const int s = c * K;
-    const long line = line0 + lr;
+    const bool first = c == 0, last = c == P - 1, whole = ch.whole(c);
+    const double* tab = SW::kFilter ? ax.ftab : ax.tab;
 
     double r[NF][K];
 #pragma unroll
     for (int f = 0; f < NF; f++) {
         __syncthreads();
 #pragma unroll
-        for (int j = 0; j < J; j++)
-            if (lane + 64 * j < npts) lds[slot[j]] = xq[f][j];
+        for (int j = 0; j < J; j++) lds[slot[j]] = xq[f][j];
         __syncthreads();
 #pragma unroll
-        for (int t = 0; t < K; t++) r[f][t] = lds[xt_slot<K>(lr, P, c, t)];
+        for (int t = 0; t < K; t++) r[f][t] = lds[xt_slot<K>(lr, P, c, EX || t < K - 1 || whole ? t : K - 2)];
     }
-    if (mu && work) {
-        const long nf = ax.nlines;
+    if (first || last) {
+        double v[NF];
+#pragma unroll
+        for (int f = 0; f < NF; f++) v[f] = first ? r[f][0] : r[f][K - 1];
+        sw.face_seed(first ? 0 : 1, line0 + lr, v);
 #pragma unroll
         for (int f = 0; f < NF; f++) {
-            if (c == 0) r[f][0] += mu[f * nf + line];
-            if (c == P - 1) r[f][K - 1] += mu[(5 + f) * nf + line];
+            r[f][0] = first ? v[f] : r[f][0];
+            r[f][K - 1] = first ? r[f][K - 1] : v[f];
         }
     }
 
-    constexpr int kReach = ST == 0 ? 8 : 64;        // chunks (kCarryRows, rounded up to a power of two)
+    constexpr int kReach = SW::kFilter ? 64 : 8;        // chunks (kCarryRows, rounded up to a power of two)
     double carry[NF], G[NF], X[NF];
-    forward_local<K, NF>(tabT, N, s, r, carry);
-    scan_forward<NF>(tabT[3 * N + s + K - 1], carry, c, P, kReach, G);
-    apply_carry<K, NF>(tabT, 3 * N, s, r, G);
-    backward_local<K, NF>(tabT, N, s, r, carry);
-    scan_backward<NF>(tabT[4 * N + s], carry, c, P, kReach, X);
-    apply_carry<K, NF>(tabT, 4 * N, s, r, X);
+    forward_local<K, NF>(tab, NP, s, r, carry);
+    scan_forward<NF>(tab[3 * NP + s + K - 1], carry, c, P, kReach, G);
+    apply_carry<K, NF>(tab, 3 * NP, s, r, G);
+    if constexpr (!EX) zero_padding<K, NF>(r, whole);
+    backward_local<K, NF>(tab, NP, s, r, carry);
+    scan_backward<NF>(tab[4 * NP + s], carry, c, P, kReach, X);
+    apply_carry<K, NF>(tab, 4 * NP, s, r, X);
 
-    const bool wrap = ST == 0 && ax.seam;
+    const bool wrap = !SW::kFilter && ax.seam;
     const int hl = c > 0 ? c - 1 : (wrap ? P - 1 : 0);
     const int hr = c + 1 < P ? c + 1 : (wrap ? 0 : P - 1);
+    const int left = xt_slot<K>(lr, P, hl, K - H) - (ch.whole(hl) ? 0 : 1);
 #pragma unroll
     for (int f = 0; f < NF; f++) {
         __syncthreads();
@@ -363,16 +406,17 @@ __global__ void __launch_bounds__(64) xtT_kernel(AxisDesc ax, SweepCommon cm, SW
             for (int t = 0; t < K; t++) lds[xt_slot<K>(li, P, c, t)] = r[f][t];
         }
         __syncthreads();
-        double w[W];
+        double w[W], right[H];
 #pragma unroll
         for (int u = 0; u < H; u++) {
-            w[u] = lds[xt_slot<K>(lr, P, hl, K - H + u)];
-            w[K + H + u] = lds[xt_slot<K>(lr, P, hr, u)];
+            w[u] = lds[left + u];
+            right[u] = lds[xt_slot<K>(lr, P, hr, u)];
         }
 #pragma unroll
         for (int t = 0; t < K; t++) w[t + H] = r[f][t];
+        close_window<K, H, W>(w, right, whole);
         double o[K];
-        stencil_t<K, ST, W>(w, o, s, N, c, P, ax.seam, cm.pb, an);
+        stencil_t<K, SW, W>(sw, w, o, c, P, whole, ax.seam, cm.pb);
 #pragma unroll
         for (int t = 0; t < K; t++) r[f][t] = o[t];
     }
@@ -389,30 +433,27 @@ __global__ void __launch_bounds__(64) xtT_kernel(AxisDesc ax, SweepCommon cm, SW
 #pragma unroll
         for (int j = 0; j < J; j++) xo[f][j] = lds[slot[j]];
     }
-    // every point's loads before the first store
+    // the loads of kPointsT points ahead of the stores
+    typename SW::Out e[kPointsT];
+#pragma unroll
+    for (int j = 0; j < kPointsT; j++) sw.template load_out<NT>(off(j), e[j]);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < J; j++) {
-        const int p = lane + 64 * j;
-        if (p < npts) {
-            double d[NF];
+        double d[NF], l[NF];
+        typename SW::Out& ej = e[j % kPointsT];
 #pragma unroll
-            for (int f = 0; f < NF; f++) d[f] = xo[f][j];
-            const int row = lrw[j] & 1023;
-            const int face = row == 0 ? 0 : (row == N - 1 ? 1 : -1);
-            sw.fetch(run + (uoff)p * 8u, d, face, line0 + (lrw[j] >> 10));
+        for (int f = 0; f < NF; f++) d[f] = xo[f][j];
+        const int row = lrw[j] & 1023;
+        sw.combine(ej, d, row == 0 ? 0 : (row == N - 1 ? 1 : -1),
+                   min(line0 + (lrw[j] >> 10), ax.nlines - 1));
 #pragma unroll
-            for (int f = 0; f < NF; f++) xo[f][j] = d[f];
+        for (int f = 0; f < NF; f++) l[f] = ej.l[sizeof(ej.l) > sizeof(double) ? f : 0];
+        if (j + kPointsT < J) {
+            sw.template load_out<NT>(off(j + kPointsT), ej);
+            __builtin_amdgcn_sched_barrier(0);
         }
-    }
-#pragma unroll
-    for (int j = 0; j < J; j++) {
-        const int p = lane + 64 * j;
-        if (p < npts) {
-            double d[NF];
-#pragma unroll
-            for (int f = 0; f < NF; f++) d[f] = xo[f][j];
-            sw.store(run + (uoff)p * 8u, d);
-        }
+        if (lane + 64 * j < npts) sw.template store<NT>(off(j), d, l);
     }
 }
 
@@ -420,119 +461,126 @@ __global__ void __launch_bounds__(64) xtT_kernel(AxisDesc ax, SweepCommon cm, SW
 // transposed sweep, y/z lines: TL lines x P chunks per workgroup, each thread
 // loads and stores its own chunk rows (coalesced across the TL lines), carries
 // by LDS folds, halo rows of the solution through LDS
+//
+// Bound by latency at three waves a SIMD, as the forward sweeps are.  What it
+// spent beside that were branches: one around each row's loads for the face
+// terms kept them from being in flight together, and the end chunks tested
+// every tap of the stencil (128^3: flux y 88 -> 64 us, z 70 -> 63, filter y
+// 84 -> 42, z 90 -> 50).
 // ---------------------------------------------------------------------------
-template <int K, int AX, int TL, class SW, int ST>
-__global__ void __launch_bounds__(TL * kMaxP) __attribute__((amdgpu_waves_per_eu(SW::kWpe))) directT_kernel(AxisDesc ax, SweepCommon cm, SW sw, const double* tabT,
-                                                             const double* mu, const double* an) {
+template <int K, int AX, int TL, class SW, bool EX, bool NT>
+__global__ void __launch_bounds__(TL * kMaxP)
+__attribute__((amdgpu_waves_per_eu(SW::kWpe)))
+directT_kernel(AxisDesc ax, SweepCommon cm, SW sw) {
     constexpr int NF = SW::NF;
-    constexpr int H = ST == 0 ? 2 : 5;
+    constexpr int H = SW::kFilter ? 5 : 2;
     constexpr int W = K + 2 * H;
     static_assert(H <= K, "halo rows come from the neighbouring chunks only");
     extern __shared__ double lds[];
 
-    const int N = ax.N, P = ax.P;
+    const int N = ax.N, P = ax.P, NP = P * K;
+    const Chunks<K, EX> ch(N, P);
     const int lloc = threadIdx.x % TL;
     const int c = threadIdx.x / TL;
     const long line = group_of(ax.xcd) * TL + lloc;
     const bool act = line < ax.nlines;
-    const bool work = act;                // blockDim = TL*P: every thread owns a chunk
+    const long ln = act ? line : ax.nlines - 1;
     const int s = c * K;
+    const bool first = c == 0, last = c == P - 1, whole = ch.whole(c);
     const uoff st = (uoff)ax.st * 8u;
-    const uoff base = line_off(AX, act ? (uoff)line : 0u, (uoff)cm.lxi, (uoff)cm.plane);
+    // threads past the last line repeat it, a padding row repeats the chunk's
+    // last: no branches around the loads, and nothing of theirs is stored
+    const uoff cbase = line_off(AX, (uoff)ln, (uoff)cm.lxi, (uoff)cm.plane) + (uoff)ch.start(c) * st;
+    auto off = [&](int t) { return cbase + (uoff)(EX || t < K - 1 || whole ? t : K - 2) * st; };
+    const double* tab = SW::kFilter ? ax.ftab : ax.tab;
 
     double r[NF][K];
 #pragma unroll
     for (int t = 0; t < K; t++) {
         double x[NF];
-        if (work) {
-            sw.seed(base + (uoff)(s + t) * st, x);
-        } else {
-#pragma unroll
-            for (int f = 0; f < NF; f++) x[f] = 0.0;
-        }
+        sw.template seed<NT>(off(t), x);
 #pragma unroll
         for (int f = 0; f < NF; f++) r[f][t] = x[f];
     }
-    if (mu && work) {
-        const long nf = ax.nlines;
+    if (first || last) {
+        double v[NF];
+#pragma unroll
+        for (int f = 0; f < NF; f++) v[f] = first ? r[f][0] : r[f][K - 1];
+        sw.face_seed(first ? 0 : 1, ln, v);
 #pragma unroll
         for (int f = 0; f < NF; f++) {
-            if (c == 0) r[f][0] += mu[f * nf + line];
-            if (c == P - 1) r[f][K - 1] += mu[(5 + f) * nf + line];
+            r[f][0] = first ? v[f] : r[f][0];
+            r[f][K - 1] = first ? r[f][K - 1] : v[f];
         }
     }
 
     double carry[NF], G[NF], X[NF];
-    forward_local<K, NF>(tabT, N, s, r, carry);
+    forward_local<K, NF>(tab, NP, s, r, carry);
 #pragma unroll
     for (int f = 0; f < NF; f++) lds[(f * P + c) * TL + lloc] = carry[f];
     __syncthreads();
-    fold_forward<NF, K, ST != 0>(lds, tabT, N, P, TL, c, lloc, G);
-    apply_carry<K, NF>(tabT, 3 * N, s, r, G);
-    backward_local<K, NF>(tabT, N, s, r, carry);
+    fold_forward<NF, K, SW::kFilter>(lds, tab, NP, P, TL, c, lloc, G);
+    apply_carry<K, NF>(tab, 3 * NP, s, r, G);
+    if constexpr (!EX) zero_padding<K, NF>(r, whole);
+    backward_local<K, NF>(tab, NP, s, r, carry);
     double* xb = lds + NF * P * TL;
 #pragma unroll
     for (int f = 0; f < NF; f++) xb[(f * P + c) * TL + lloc] = carry[f];
     __syncthreads();
-    fold_backward<NF, K, ST != 0>(xb, tabT, N, P, TL, c, lloc, X);
-    apply_carry<K, NF>(tabT, 4 * N, s, r, X);
+    fold_backward<NF, K, SW::kFilter>(xb, tab, NP, P, TL, c, lloc, X);
+    apply_carry<K, NF>(tab, 4 * NP, s, r, X);
 
     // halo rows hb[(f*2H + k)*P + c][TL]: k < H the first H rows of chunk c,
-    // k >= H its last H rows (neighbours wrap on seam lines of the
-    // derivative); the derivative's five fields in one exchange, the filter
-    // one field at a time
-    const bool wrap = ST == 0 && ax.seam;
+    // k >= H its last H rows (neighbours wrap on seam lines of the derivative)
+    const bool wrap = !SW::kFilter && ax.seam;
     const int cl = c > 0 ? c - 1 : (wrap ? P - 1 : 0), cr = c + 1 < P ? c + 1 : (wrap ? 0 : P - 1);
-    constexpr int FX = ST == 0 ? NF : 1;      // fields per exchange
+    __syncthreads();                      // earlier reads of the LDS are done
 #pragma unroll
-    for (int f0 = 0; f0 < NF; f0 += FX) {
-        __syncthreads();                  // earlier reads of the LDS are done
+    for (int f = 0; f < NF; f++) {
 #pragma unroll
-        for (int e = 0; e < FX; e++) {
-#pragma unroll
-            for (int k = 0; k < H; k++) {
-                lds[((e * 2 * H + k) * P + c) * TL + lloc] = r[f0 + e][k];
-                lds[((e * 2 * H + H + k) * P + c) * TL + lloc] = r[f0 + e][K - H + k];
-            }
+        for (int k = 0; k < H; k++) {
+            lds[((f * 2 * H + k) * P + c) * TL + lloc] = r[f][k];
+            lds[((f * 2 * H + H + k) * P + c) * TL + lloc] = whole ? r[f][K - H + k] : r[f][K - H + k - 1];
         }
-        __syncthreads();
+    }
+    __syncthreads();
 #pragma unroll
-        for (int e = 0; e < FX; e++) {
-            const int f = f0 + e;
-            double w[W];
+    for (int f = 0; f < NF; f++) {
+        double w[W], right[H];
 #pragma unroll
-            for (int k = 0; k < H; k++) {
-                w[k] = lds[((e * 2 * H + H + k) * P + cl) * TL + lloc];
-                w[K + H + k] = lds[((e * 2 * H + k) * P + cr) * TL + lloc];
-            }
-#pragma unroll
-            for (int t = 0; t < K; t++) w[t + H] = r[f][t];
-            double o[K];
-            stencil_t<K, ST, W>(w, o, s, N, c, P, ax.seam, cm.pb, an);
-#pragma unroll
-            for (int t = 0; t < K; t++) r[f][t] = o[t];
+        for (int k = 0; k < H; k++) {
+            w[k] = lds[((f * 2 * H + H + k) * P + cl) * TL + lloc];
+            right[k] = lds[((f * 2 * H + k) * P + cr) * TL + lloc];
         }
+#pragma unroll
+        for (int t = 0; t < K; t++) w[t + H] = r[f][t];
+        close_window<K, H, W>(w, right, whole);
+        double o[K];
+        stencil_t<K, SW, W>(sw, w, o, c, P, whole, ax.seam, cm.pb);
+#pragma unroll
+        for (int t = 0; t < K; t++) r[f][t] = o[t];
     }
 
-    if (!work) return;
-    // every row's loads before the first store
+    if (!act) return;
+    // the loads of kRowsT rows ahead of the stores
+    typename SW::Out e[kRowsT];
+#pragma unroll
+    for (int t = 0; t < kRowsT; t++) sw.template load_out<NT>(off(t), e[t]);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int t = 0; t < K; t++) {
-        const int row = s + t;
-        double d[NF];
+        double d[NF], l[NF];
+        typename SW::Out& et = e[t % kRowsT];
 #pragma unroll
         for (int f = 0; f < NF; f++) d[f] = r[f][t];
-        const int face = row == 0 ? 0 : (row == N - 1 ? 1 : -1);
-        sw.fetch(base + (uoff)row * st, d, face, line);
+        sw.combine(et, d, t == 0 && first ? 0 : (t == K - 1 && last ? 1 : -1), ln);
 #pragma unroll
-        for (int f = 0; f < NF; f++) r[f][t] = d[f];
-    }
-#pragma unroll
-    for (int t = 0; t < K; t++) {
-        double d[NF];
-#pragma unroll
-        for (int f = 0; f < NF; f++) d[f] = r[f][t];
-        sw.store(base + (uoff)(s + t) * st, d);
+        for (int f = 0; f < NF; f++) l[f] = et.l[sizeof(et.l) > sizeof(double) ? f : 0];
+        if (t + kRowsT < K) {
+            sw.template load_out<NT>(off(t + kRowsT), et);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (EX || t < K - 1 || whole) sw.template store<NT>(off(t), d, l);
     }
 }
 
@@ -605,34 +653,39 @@ __global__ void __launch_bounds__(256) face_adjoint_kernel(const double* q, cons
     }
 }
 
-// transposed sweep along AX: x lines one wave per workgroup, y/z lines
-// ax.tl lines per workgroup; FT<1> spreads the five fields over grid.y
-template <int AX, int ST, class SW>
-int launch_t(const AxisDesc& ax, const SweepCommon& cm, const SW& sw, const double* tabT, const double* mu,
-             const double* an, hipStream_t s) {
-    constexpr int K = 8, NF = SW::NF, H = ST == 0 ? 2 : 5;
+// transposed sweep along AX on chunks of K points: x lines one wave a
+// workgroup, y/z lines 16 lines; FT<1> spreads the five fields over grid.y
+template <int K, int AX, class SW>
+int launch_k(const AxisDesc& ax, const SweepCommon& cm, const SW& sw, hipStream_t s) {
+    constexpr int NF = SW::NF, H = SW::kFilter ? 5 : 2;
     const unsigned gy = NF == 1 ? 5u : 1u;
+    const bool exact = ax.N == ax.P * K, nt = streams<SW>(ax, cm);
     if constexpr (AX == 0) {
         const int lpw = 64 / ax.P;
-        const size_t lds = sizeof(double) * lpw * ax.P * (K + 1);
-        dim3 block(64), grid((unsigned)((ax.nlines + lpw - 1) / lpw), gy);
-        hipLaunchKernelGGL((xtT_kernel<K, SW, ST>), grid, block, lds, s, ax, cm, sw, tabT, mu, an);
+        const size_t lds = sizeof(double) * (lpw * ax.P * (K + 1) + 64);
+        const dim3 grid((unsigned)((ax.nlines + lpw - 1) / lpw), gy);
+        const void* k = exact ? (nt ? (const void*)xtT_kernel<K, SW, true, true> : (const void*)xtT_kernel<K, SW, true, false>)
+                              : (nt ? (const void*)xtT_kernel<K, SW, false, true> : (const void*)xtT_kernel<K, SW, false, false>);
+        return launch(k, grid, dim3(64), lds, with_runs(ax, grid.x, true, 64), cm, sw, s);
     } else {
-        const int TL = ax.tl == 8 ? 8 : 16;
-        const size_t halo = (size_t)(ST == 0 ? NF : 1) * 2 * H * ax.P * TL;
-        const size_t carries = (size_t)2 * NF * ax.P * TL;
+        constexpr int TL = 16;
+        const size_t halo = (size_t)NF * 2 * H * ax.P * TL, carries = (size_t)2 * NF * ax.P * TL;
         const size_t lds = sizeof(double) * (halo > carries ? halo : carries);
-        dim3 block(TL * ax.P), grid((unsigned)((ax.nlines + TL - 1) / TL), gy);
-        const void* k = TL == 8 ? (const void*)directT_kernel<K, AX, 8, SW, ST>
-                                : (const void*)directT_kernel<K, AX, 16, SW, ST>;
-        if (lds > 65536) CS_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        if (TL == 8)
-            hipLaunchKernelGGL((directT_kernel<K, AX, 8, SW, ST>), grid, block, lds, s, ax, cm, sw, tabT, mu, an);
-        else
-            hipLaunchKernelGGL((directT_kernel<K, AX, 16, SW, ST>), grid, block, lds, s, ax, cm, sw, tabT, mu, an);
+        const dim3 grid((unsigned)((ax.nlines + TL - 1) / TL), gy);
+        const void* k = exact ? (nt ? (const void*)directT_kernel<K, AX, TL, SW, true, true>
+                                    : (const void*)directT_kernel<K, AX, TL, SW, true, false>)
+                              : (nt ? (const void*)directT_kernel<K, AX, TL, SW, false, true>
+                                    : (const void*)directT_kernel<K, AX, TL, SW, false, false>);
+        return launch(k, grid, dim3(TL * ax.P), lds, with_runs(ax, grid.x, true, (AX == 1 ? 128 : 1024) / TL), cm, sw,
+                      s);
     }
-    CS_HIP(hipGetLastError());
-    return CS_OK;
+}
+
+template <int AX, class SW>
+int launch_t(const AxisDesc& ax, const SweepCommon& cm, const SW& sw, hipStream_t s) {
+    if constexpr (AX != 0 && SW::kFilter)
+        if (ax.K == 16) return launch_k<16, AX>(ax, cm, sw, s);
+    return launch_k<8, AX>(ax, cm, sw, s);
 }
 
 EulerPhys euler_phys_of(const cs_solver* sv) {
@@ -651,26 +704,37 @@ long adj_face_buf(const cs_solver* sv) { return 5 * sv->g.lmx * 2; }
 long adj_tape(const cs_solver* sv) { return adj_face_buf(sv) + 2 * faces_size(sv->g); }
 long adj_doubles(const cs_solver* sv) { return adj_tape(sv) + 20 * sv->g.lmx + 4 * faces_size(sv->g); }
 
-int upload(const std::vector<double>& h, double** d) {
-    CS_HIP(hipMalloc(d, h.size() * sizeof(double)));
-    CS_HIP(hipMemcpy(*d, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice));
+// device table of the transposed operator `op` along the axis of t
+int upload(const cs_solver* sv, int op, const AxisDesc& t, int seam, double** d) {
+    std::vector<double> h, c;
+    int rc = build_adjoint_table(op, t.N, seam, seam, sv->cfg.alpha_f, sv->num->pb_host, t.K, h);
+    if (rc) return rc;
+    chunk_table(h, t.N, t.K, t.P, c);
+    CS_HIP(hipMalloc(d, c.size() * sizeof(double)));
+    CS_HIP(hipMemcpy(*d, c.data(), c.size() * sizeof(double), hipMemcpyHostToDevice));
     return CS_OK;
 }
 
+// the descriptors of the transposed sweeps and the scratch.  Derivative: 8-point
+// chunks, whose 5 x 16 values of a 16-point one spill beside the epilogue's
+// loads (128^3 y, z: 64, 63 us against 68, 69).  Filter along y and z: 16-point
+// chunks where they fit, one field a workgroup (42, 50 us against 54, 60).
 int adjoint_setup(cs_solver* sv) {
     if (sv->adj) return CS_OK;
     int rc;
     for (int a = 0; a < 3; a++) {
-        const AxisDesc& ax = sv->ax[a];
-        std::vector<double> h;
-        if ((rc = build_adjoint_table(OP_DERIV_T, ax.N, ax.seam, ax.seam, sv->cfg.alpha_f, sv->num->pb_host, 8, h)))
-            return rc;
-        if ((rc = upload(h, &sv->ttabs[a]))) return rc;
-        if (sv->cfg.filter && !ax.seam) {
-            if ((rc = build_adjoint_table(OP_FILTER_T, ax.N, 0, 0, sv->cfg.alpha_f, sv->num->pb_host, 8, h)))
-                return rc;
-            if ((rc = upload(h, &sv->fttabs[a]))) return rc;
+        AxisDesc t = sv->ax[a], f = t;
+        if (fits16(f, a)) {
+            f.K = 16;
+            f.P = (f.N + 15) / 16;
         }
+        if (!sv->ttabs[a] && (rc = upload(sv, OP_DERIV_T, t, t.seam, &sv->ttabs[a]))) return rc;
+        if (sv->cfg.filter && !f.seam && !sv->fttabs[a] && (rc = upload(sv, OP_FILTER_T, f, 0, &sv->fttabs[a])))
+            return rc;
+        t.tab = sv->ttabs[a];
+        f.ftab = sv->fttabs[a];
+        sv->tax[a] = t;
+        sv->ftax[a] = f;
     }
     CS_HIP(hipMalloc(&sv->adj, sizeof(double) * adj_doubles(sv)));
     return CS_OK;
@@ -681,19 +745,14 @@ template <int AX>
 int filter_t_axis(cs_solver* sv, double* lam, const SweepCommon& cm, hipStream_t s) {
     const AxisDesc& ax = sv->ax[AX];
     if (ax.seam) return filter_sweeps(sv, lam, s, AX);        // cyclic: its own transpose
-    const double* an = ax.ftab + 6 * ax.N + 8;
-    if (AX == 0) {
-        FT<5> f{lam, sv->g.lmx};
-        return launch_t<AX, 1>(ax, cm, f, sv->fttabs[AX], nullptr, an, s);
-    }
-    FT<1> f{lam, sv->g.lmx};
-    return launch_t<AX, 1>(ax, cm, f, sv->fttabs[AX], nullptr, an, s);
+    const FT<AX == 0 ? 5 : 1> f{lam, sv->g.lmx, ax.ftab + 6 * ax.P * ax.K + 8};
+    return launch_t<AX>(sv->ftax[AX], cm, f, s);
 }
 
 template <int AX, int MODE, bool CURV>
 int stage_sweep_t(cs_solver* sv, const SweepCommon& cm, const double* q, const double* t, const double* gin,
                   double* gout, double* lam, double* tout, double ck, const double* fb, hipStream_t s) {
-    const AxisDesc& ax = sv->ax[AX];
+    const AxisDesc& ax = sv->tax[AX];
     const long lmx = sv->g.lmx;
     AT<AX, MODE, CURV> a{};
     fields(q, lmx, a.q);
@@ -702,10 +761,9 @@ int stage_sweep_t(cs_solver* sv, const SweepCommon& cm, const double* q, const d
     fields(gout, lmx, a.gout);
     fields(lam, lmx, a.lam);
     fields(tout, lmx, a.tout);
-    const double* mu = nullptr;
     if (ax.gcbc) {
-        mu = fb + 2 * face_offset(sv->g, AX);
-        a.G = mu + 10 * ax.nlines;
+        a.mu = fb + 2 * face_offset(sv->g, AX);
+        a.G = a.mu + 10 * ax.nlines;
     }
     a.nface = ax.nlines;
     a.ck = ck;
@@ -713,7 +771,7 @@ int stage_sweep_t(cs_solver* sv, const SweepCommon& cm, const double* q, const d
     a.uf = uf_of(sv, AX);
     a.umf = sv->cfg.umf;
     if constexpr (CURV) a.mt = sv->met;
-    return launch_t<AX, 0>(ax, cm, a, sv->ttabs[AX], mu, nullptr, s);
+    return launch_t<AX>(ax, cm, a, s);
 }
 
 // ck = dt/div times the constant Jacobian; curvilinear solvers pass a seed
@@ -815,9 +873,11 @@ int step_recording(cs_solver* sv, double* qa, const double* sbcc, double dt, dou
 
 bool adjoint_fused(const cs_solver* sv) {
     if (sv->adj_mode != 1 || sv->cfg.viscous) return false;
-    for (int a = 0; a < 3; a++)
-        if (sv->ax[a].K != 8 || sv->ax[a].N != sv->ax[a].P * 8 || sv->ax[a].P > kMaxP) return false;
-    return !sv->cfg.filter || filter_fusable(sv);
+    for (int a = 0; a < 3; a++) {
+        const AxisDesc& ax = sv->ax[a];
+        if (ax.K != 8 || !chunks_fit(ax.N, ax.P, 8) || ax.P > (a == 0 ? 64 : kMaxP)) return false;
+    }
+    return true;
 }
 
 long tape_doubles(const cs_solver* sv) { return 20 * sv->g.lmx + 4 * faces_size(sv->g); }

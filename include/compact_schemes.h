@@ -360,7 +360,8 @@ int cs_solver_rk4_vjp_tape(cs_solver* sv, const double* tape, double* lam, doubl
                            cs_stream stream);
 /* adjoint implementation (no reference counterpart): 1 (default) = transposed
  * line sweeps fused with the pointwise Jacobian products, used when every
- * axis splits into 8-point chunks (N % 8 == 0, N <= 256); 0 = per-operator
+ * axis splits into 8-point chunks at most one row short (y and z lines up to
+ * 256 points, x lines up to 512); 0 = per-operator
  * transposed line solves (cs_deriv_adjoint, cs_filter_adjoint).  Results
  * agree to rounding. */
 int cs_solver_adjoint_mode(cs_solver* sv, int mode);
