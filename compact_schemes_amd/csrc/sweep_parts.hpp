@@ -80,6 +80,15 @@ __device__ __forceinline__ void dt_curv_point(const double (&M)[3][3], double J,
     m1 = fmax(m1, p.rhoi * ph.mu * rr1 * ssi * ssi);
 }
 
+// heat flux along an axis from the physical c^2 gradient and the axis's
+// stress row: the last lines of viscous_closure with constant metrics, the
+// same operations in the same order
+__device__ __forceinline__ double heat_flux(const Phys& ph, double c2g, double u, double v, double w, double t0,
+                                            double t1, double t2) {
+    const double b1 = kGamm1Prndtli * (ph.mu * ph.J);
+    return b1 * c2g + u * t0 + v * t1 + w * t2;
+}
+
 // byte offset of row 0 of line f of an axis (f runs over the face's points
 // with the first remaining index fastest)
 __device__ __forceinline__ uoff line_off(int axis, uoff f, uoff lxi, uoff plane) {
