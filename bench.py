@@ -187,7 +187,7 @@ def main():
         torch.cuda.synchronize()
         ms_k = e0.elapsed_time(e1) / nk
         bytes_per_launch = 16.0 * lmx          # read + write one FP64 field
-        kern = {"name": "cs::line_kernel<16,0,1> (y derivative)", "ms": ms_k, "bytes": bytes_per_launch}
+        kern = {"name": "cs::fused::direct_kernel, LineSweep<false> (y derivative)", "ms": ms_k, "bytes": bytes_per_launch}
     else:
         q.copy_(q_init)
         kern = solver.time_dominant_kernel(q, stream)
@@ -218,7 +218,7 @@ def main():
 
     if args.path == "fused":
         # the whole path against the same roof: credited bytes of one RHS
-        # (736 B/pt) and of one RK4 step (4 stages of 776 B/pt, three filter
+        # (704 B/pt) and of one RK4 step (4 stages of 744 B/pt, three filter
         # sweeps of 80) over their measured times
         rhs_gbs = RHS_BYTES_PER_PT * lmx / (ms_rhs * 1e-3) / 1e9
         step_gbs = STEP_BYTES_PER_PT * lmx / (ms_step * 1e-3) / 1e9
@@ -282,18 +282,19 @@ def other_workloads(timeout=300):
 
 
 PROFILE_TRAFFIC = os.path.join(ROOT, "profiles", "pmc_traffic_rk_stage_256.txt")
-RHS_BYTES_PER_PT = 736                     # six sweeps of one viscous RHS
+RHS_BYTES_PER_PT = 704                     # six sweeps of one viscous RHS
 # RK4 step: four stages and the filter along x, y, z; the time step's maxima
 # are reduced inside the first gradient sweep of the first stage (the y sweep
 # of the 256^3 workload: 16 lines x 32 chunks, whole waves), which reads q anyway
-STEP_BYTES_PER_PT = 4 * 776 + 3 * 80
+STEP_BYTES_PER_PT = 4 * 744 + 3 * 80
 PROFILE_FP64 = os.path.join(ROOT, "profiles", "pmc_fp64_rk_stage_256.txt")
 
 
-# credited bytes of one curvilinear RHS: the 736 of the constant-metric RHS plus
-# the closure's nine metrics and Jacobian (80), each flux sweep's metric row
-# (24) and the five stress and heat-flux components beyond its own row (40)
-CURV_RHS_BYTES_PER_PT = RHS_BYTES_PER_PT + 80 + 3 * (24 + 40)
+# credited bytes of one curvilinear RHS: the 704 of the constant-metric RHS plus
+# the closure's other two c^2 gradients and heat fluxes (32), its nine metrics
+# and Jacobian (80), each flux sweep's metric row (24) and the five stress and
+# heat-flux components beyond its own row (40)
+CURV_RHS_BYTES_PER_PT = RHS_BYTES_PER_PT + 32 + 80 + 3 * (24 + 40)
 
 
 def curvilinear_bench(args, n=256):
@@ -526,7 +527,7 @@ def precision_bench(args, dims=(512, 512, 256), nsteps=50):
     limit of the initial state).  Primary: the fused solver with FP64
     intermediates against the same solver with the viscous intermediates
     (gradients, stress, heat flux) stored in FP32 (cs_solver_set_precision
-    1: 588 instead of 736 HBM bytes per point and RHS).  Secondary: the
+    1: 572 instead of 704 HBM bytes per point and RHS).  Secondary: the
     reference-ordered operators with FP64 line solves against FP32 solves +
     one FP64-residual refinement sweep (cs_set_precision 1).  Errors per
     conserved variable relative to the state and to its change over the run;

@@ -749,17 +749,16 @@ struct NoBatch {
 // the loads to the stores.  So nothing but them is live: the loads run
 // kRowsAhead rows ahead of the evaluation (all rows at once spill 500-700 B a
 // lane), a field's window exists only while its right-hand side is formed, and
-// the epilogue's loads run kRowsOut rows ahead of the additions.  16 lines are
-// 128-byte rows.  Measured at 256^3 (start -> now, us; a copy of 2.1 GB runs at
+// the epilogue's loads run kRowsOut rows ahead of the additions.  Measured at 256^3 (start -> now, us; a copy of 2.1 GB runs at
 // 4.8 TB/s, the same row pattern without arithmetic at 5.3 along y and 4.7
-// along z): S1y 284 -> 216 (5.6 TB/s), S2y 550 -> 482 (5.3), S1z 309 -> 275
-// (4.4), S2z 514 -> 431 (4.4).
+// along z): S1y 284 -> 216 (5.6 TB/s), S2y 550 -> 482 (5.3), S1z 309 -> 250
+// (4.8), S2z 514 -> 408 (4.6).
 // ---------------------------------------------------------------------------
 constexpr int kRowsAhead = 2;   // rows whose loads are in flight while a row is evaluated
 constexpr int kRowsOut = 4;     // rows whose epilogue loads are in flight
 
 template <int K, int AX, int TL, class SW, bool GCBC, bool EX, bool NT, class BATCH = NoBatch>
-__global__ void __launch_bounds__(TL * kMaxP < 1024 ? TL * kMaxP : 1024)
+__global__ void __launch_bounds__(TL == 32 ? 512 : TL * kMaxP < 1024 ? TL * kMaxP : 1024)
 __attribute__((amdgpu_waves_per_eu(K == 16 ? SW::kWpe16 : SW::kWpe)))
 direct_kernel(AxisDesc ax, SweepCommon cm, SW sw, BATCH batch) {
     extern __shared__ double lds[];       // direct_lds
@@ -1391,15 +1390,40 @@ static const void* xt_symbol(bool exact, bool nt) {
     return nt ? (const void*)xt_kernel<K, SW, GCBC, false, true> : (const void*)xt_kernel<K, SW, GCBC, false, false>;
 }
 
+// Lines a workgroup of a y/z sweep takes where tl (8 or 16) asks for 16.
+// One field on lines of up to 16 chunks: 64, so that a wave is one chunk, its
+// table entries come by scalar loads and rows are 512 bytes (256^3 filter y 309 ->
+// 283, z 316 -> 292 us; 128^3 40 -> 34, 40 -> 36).  The five- and four-field
+// sweeps along z on up to 16 chunks of 16 points: 32, 256-byte rows of a plane
+// that is otherwise passed over in 128-byte pieces (256^3 S2z 442 -> 408, S1z
+// 277 -> 250 us, 128^3 S2z 45 -> 39, 48x40x32 12.0 -> 11.4); the same waves fit
+// a CU.  Along y, where 16 lines' rows lie next to the following workgroup's,
+// 32 lose (S2y 484 -> 546, S1y 218 -> 247 us).
+template <int K, int AX, class SW>
+static int block_lines(int P, int tl) {
+    if (tl == 8) return 8;
+    if (SW::NF == 1 && P <= 16) return 64;
+    return AX == 2 && K == 16 && SW::NF > 1 && !SW::kFilter && P <= 16 ? 32 : 16;
+}
+
+template <int K, int AX, int TL, class SW, bool GCBC>
+static const void* direct_at(bool exact, bool nt) {
+    if (exact) return nt ? (const void*)direct_kernel<K, AX, TL, SW, GCBC, true, true>
+                         : (const void*)direct_kernel<K, AX, TL, SW, GCBC, true, false>;
+    return nt ? (const void*)direct_kernel<K, AX, TL, SW, GCBC, false, true>
+              : (const void*)direct_kernel<K, AX, TL, SW, GCBC, false, false>;
+}
+
 // 8 lines a workgroup are 64-byte rows: never streamed
 template <int K, int AX, class SW, bool GCBC>
 static const void* direct_symbol(int TL, bool exact, bool nt) {
     if (TL == 8) return exact ? (const void*)direct_kernel<K, AX, 8, SW, GCBC, true, false>
                               : (const void*)direct_kernel<K, AX, 8, SW, GCBC, false, false>;
-    if (exact) return nt ? (const void*)direct_kernel<K, AX, 16, SW, GCBC, true, true>
-                         : (const void*)direct_kernel<K, AX, 16, SW, GCBC, true, false>;
-    return nt ? (const void*)direct_kernel<K, AX, 16, SW, GCBC, false, true>
-              : (const void*)direct_kernel<K, AX, 16, SW, GCBC, false, false>;
+    if constexpr (SW::NF == 1)
+        if (TL == 64) return direct_at<K, AX, 64, SW, GCBC>(exact, nt);
+    if constexpr (AX == 2 && K == 16 && SW::NF > 1 && !SW::kFilter)
+        if (TL == 32) return direct_at<K, AX, 32, SW, GCBC>(exact, nt);
+    return direct_at<K, AX, 16, SW, GCBC>(exact, nt);
 }
 
 template <class SW, class BATCH = NoBatch>
@@ -1462,7 +1486,7 @@ static int launch_sweep(const AxisDesc& ax, const SweepCommon& cm, const SW& sw,
         static_assert(K == 8, "x lines run 8-point chunks");
         return launch_x<K, SW, GCBC>(ax, cm, sw, 1u, s);
     } else {
-        const int TL = ax.tl == 8 ? 8 : 16;
+        const int TL = block_lines<K, AX, SW>(ax.P, ax.tl);
         return launch_yz<K, AX, SW, GCBC>(ax, cm, sw, TL, ax.xcd != 0, direct_lds<SW>(ax.P, TL, ax.seam), 1u, s);
     }
 }
@@ -1479,7 +1503,7 @@ static int launch_filter(const AxisDesc& ax, const SweepCommon& cm, const SW& sw
     if constexpr (AX == 0) {
         return launch_x<K, SW, false>(ax, cm, sw, gy, s);
     } else {
-        const int TL = ax.ftl == 8 ? 8 : 16;
+        const int TL = block_lines<K, AX, SW>(ax.P, ax.ftl);
         return launch_yz<K, AX, SW, false>(ax, cm, sw, TL, true, direct_lds<SW>(ax.P, TL, false), gy, s);
     }
 }

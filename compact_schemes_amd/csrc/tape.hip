@@ -466,10 +466,10 @@ xtT_kernel(AxisDesc ax, SweepCommon cm, SW sw) {
 // spent beside that were branches: one around each row's loads for the face
 // terms kept them from being in flight together, and the end chunks tested
 // every tap of the stencil (128^3: flux y 88 -> 64 us, z 70 -> 63, filter y
-// 84 -> 42, z 90 -> 50).
+// 84 -> 37, z 90 -> 44).
 // ---------------------------------------------------------------------------
 template <int K, int AX, int TL, class SW, bool EX, bool NT>
-__global__ void __launch_bounds__(TL * kMaxP)
+__global__ void __launch_bounds__(TL * kMaxP < 1024 ? TL * kMaxP : 1024)
 __attribute__((amdgpu_waves_per_eu(SW::kWpe)))
 directT_kernel(AxisDesc ax, SweepCommon cm, SW sw) {
     constexpr int NF = SW::NF;
@@ -481,7 +481,7 @@ directT_kernel(AxisDesc ax, SweepCommon cm, SW sw) {
     const int N = ax.N, P = ax.P, NP = P * K;
     const Chunks<K, EX> ch(N, P);
     const int lloc = threadIdx.x % TL;
-    const int c = threadIdx.x / TL;
+    const int c = TL == 64 ? __builtin_amdgcn_readfirstlane(threadIdx.x / TL) : threadIdx.x / TL;
     const long line = group_of(ax.xcd) * TL + lloc;
     const bool act = line < ax.nlines;
     const long ln = act ? line : ax.nlines - 1;
@@ -653,8 +653,16 @@ __global__ void __launch_bounds__(256) face_adjoint_kernel(const double* q, cons
     }
 }
 
+template <int K, int AX, int TL, class SW>
+const void* direct_t(bool exact, bool nt) {
+    if (exact) return nt ? (const void*)directT_kernel<K, AX, TL, SW, true, true>
+                         : (const void*)directT_kernel<K, AX, TL, SW, true, false>;
+    return nt ? (const void*)directT_kernel<K, AX, TL, SW, false, true>
+              : (const void*)directT_kernel<K, AX, TL, SW, false, false>;
+}
+
 // transposed sweep along AX on chunks of K points: x lines one wave a
-// workgroup, y/z lines 16 lines; FT<1> spreads the five fields over grid.y
+// workgroup, y/z lines 16 or 64 lines; FT<1> spreads the five fields over grid.y
 template <int K, int AX, class SW>
 int launch_k(const AxisDesc& ax, const SweepCommon& cm, const SW& sw, hipStream_t s) {
     constexpr int NF = SW::NF, H = SW::kFilter ? 5 : 2;
@@ -668,14 +676,14 @@ int launch_k(const AxisDesc& ax, const SweepCommon& cm, const SW& sw, hipStream_
                               : (nt ? (const void*)xtT_kernel<K, SW, false, true> : (const void*)xtT_kernel<K, SW, false, false>);
         return launch(k, grid, dim3(64), lds, with_runs(ax, grid.x, true, 64), cm, sw, s);
     } else {
-        constexpr int TL = 16;
+        const int TL = SW::NF == 1 && ax.P <= 16 ? 64 : 16;      // as block_lines
         const size_t halo = (size_t)NF * 2 * H * ax.P * TL, carries = (size_t)2 * NF * ax.P * TL;
         const size_t lds = sizeof(double) * (halo > carries ? halo : carries);
         const dim3 grid((unsigned)((ax.nlines + TL - 1) / TL), gy);
-        const void* k = exact ? (nt ? (const void*)directT_kernel<K, AX, TL, SW, true, true>
-                                    : (const void*)directT_kernel<K, AX, TL, SW, true, false>)
-                              : (nt ? (const void*)directT_kernel<K, AX, TL, SW, false, true>
-                                    : (const void*)directT_kernel<K, AX, TL, SW, false, false>);
+        const void* k = nullptr;
+        if constexpr (NF == 1)
+            if (TL == 64) k = direct_t<K, AX, 64, SW>(exact, nt);
+        if (!k) k = direct_t<K, AX, 16, SW>(exact, nt);
         return launch(k, grid, dim3(TL * ax.P), lds, with_runs(ax, grid.x, true, (AX == 1 ? 128 : 1024) / TL), cm, sw,
                       s);
     }

@@ -27,12 +27,12 @@ def sweep_names(order):
 
 
 SWEEP_NAMES = sweep_names(1)
-SWEEP_BYTES_VISC = [8 * (5 + 4), 8 * (5 + 4), 8 * (5 + 8 + 9), 8 * (5 + 4 + 5), 8 * (5 + 4 + 5 + 5),
+SWEEP_BYTES_VISC = [8 * (5 + 4), 8 * (5 + 4), 8 * (5 + 6 + 7), 8 * (5 + 4 + 5), 8 * (5 + 4 + 5 + 5),
                     8 * (5 + 4 + 5 + 5), 8 * (5 + 4 + 5 + 5 + 5), 3 * 8 * (5 + 5)] + [8 * (5 + 5)] * 3
 SWEEP_BYTES_EULER = [0, 0, 0, 8 * (5 + 5), 8 * (5 + 5 + 5), 8 * (5 + 5 + 5), 8 * (5 + 5 + 5 + 5),
                      3 * 8 * (5 + 5)] + [8 * (5 + 5)] * 3
 # viscous intermediates (4 gradients per gradient sweep, stress and heat flux) in FP32
-SWEEP_BYTES_VISC_F32 = [8 * 5 + 4 * 4, 8 * 5 + 4 * 4, 8 * 5 + 4 * 8 + 4 * 9, 8 * (5 + 5) + 4 * 4,
+SWEEP_BYTES_VISC_F32 = [8 * 5 + 4 * 4, 8 * 5 + 4 * 4, 8 * 5 + 4 * 6 + 4 * 7, 8 * (5 + 5) + 4 * 4,
                         8 * (5 + 5 + 5) + 4 * 4, 8 * (5 + 5 + 5) + 4 * 4, 8 * (5 + 5 + 5 + 5) + 4 * 4,
                         3 * 8 * (5 + 5)] + [8 * (5 + 5)] * 3
 # the filter sweeps (one per axis) that close an RK4 step
@@ -167,7 +167,7 @@ class FusedSolver:
         if which >= 8:
             per = 40
         elif which < 3:
-            per = 40 + ts * (17 if which == 2 else 4) + (80 if which == 2 and c else 0)
+            per = 40 + ts * ((17 if c else 13) if which == 2 else 4) + (80 if which == 2 and c else 0)
         else:
             per = 80 + (ts * (9 if c else 4) if self.viscous else 0) + (24 if c else 0) + {5: 40, 6: 80}.get(which, 0)
         return self.dims[0] % (2 if ax == 0 else 16) == 0 and per * self.lmx > 256 * 2 ** 20
@@ -186,7 +186,9 @@ class FusedSolver:
             if ax == 0:
                 return f"cs::fused::xt_kernel<8, {sf}, false, {b(self.dims[0] % 8 == 0)}, {b(nt)}, cs::fused::NoBatch>"
             ex = self.dims[ax] % chunk == 0
-            return f"cs::fused::direct_kernel<{chunk}, {ax}, {lines}, {sf}, false, {b(ex)}, {b(nt and lines == 16)}, cs::fused::NoBatch>"
+            if lines == 16 and fields == 1 and -(-self.dims[ax] // chunk) <= 16:
+                lines = 64
+            return f"cs::fused::direct_kernel<{chunk}, {ax}, {lines}, {sf}, false, {b(ex)}, {b(nt and lines >= 16)}, cs::fused::NoBatch>"
         ax = S1_AXES[self.order][which] if which < 3 else S2_AXES[self.order][min(which, 5) - 3]
         n = self.dims[ax]
         variant, lines, _ = self.get_tune(ax)[0]
@@ -204,7 +206,9 @@ class FusedSolver:
         nt = self._streams(which, ax)
         if ax == 0:
             return f"cs::fused::xt_kernel<{K}, {sw}, {gc}, {b(n % K == 0)}, {b(nt)}, cs::fused::NoBatch>"
-        return f"cs::fused::direct_kernel<{K}, {ax}, {lines}, {sw}, {gc}, {b(n % K == 0)}, {b(nt and lines == 16)}, "\
+        if lines == 16 and ax == 2 and K == 16 and -(-n // K) <= 16:
+            lines = 32
+        return f"cs::fused::direct_kernel<{K}, {ax}, {lines}, {sw}, {gc}, {b(n % K == 0)}, {b(nt and lines >= 16)}, "\
                "cs::fused::NoBatch>"
 
     def time_step(self, q, stream=None):

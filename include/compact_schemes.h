@@ -264,7 +264,8 @@ int cs_solver_sweep(cs_solver* sv, int which, const double* qa, double* de, cons
  * with coalesced loads, 2 = variant 0 on 16-point chunks (y/z lines of 32 to
  * 256 points, a multiple of 16; the default along y and z, there also on
  * lines that 16-point chunks one row short can cut); lines = 8 or 16 lines
- * per workgroup (y/z lines of variants 0 and 2, all lines of variant 1);
+ * per workgroup (y/z lines of variants 0 and 2, all lines of variant 1; 16 is
+ * 32 along z on up to 16 chunks of 16 points);
  * xcd = 1 keeps neighbouring line groups on one XCD.  Results agree to
  * rounding whatever the choice. */
 int cs_solver_tune(cs_solver* sv, int axis, int variant, int lines, int xcd);
@@ -272,7 +273,7 @@ int cs_solver_tune(cs_solver* sv, int axis, int variant, int lines, int xcd);
  * fields = 1 filters one conserved variable per workgroup (the five variables
  * spread over the grid; default along y and z), 5 all five per workgroup
  * (default along x); lines = 8 or 16 lines per workgroup of the y/z sweeps
- * (default 16); chunk = 8 or 16 points per chunk thread (16: y/z lines of 32
+ * (default 16, which is 64 for one variable on lines of up to 16 chunks); chunk = 8 or 16 points per chunk thread (16: y/z lines of 32
  * to 256 points, a multiple of 16; the default there).  Results agree to
  * rounding whatever the choice. */
 int cs_solver_tune_filter(cs_solver* sv, int axis, int fields, int lines, int chunk);
@@ -294,8 +295,8 @@ int cs_solver_autotune(cs_solver* sv, const double* qa, const double* sbcc, int 
 /* storage precision of the viscous intermediates between the sweeps (no
  * reference counterpart; the reference templates everything on one Type):
  * 0 = FP64 (default); 1 = the velocity and c^2 gradients of the first two
- * gradient sweeps, the stress tensor and the heat flux stored in FP32 (588
- * instead of 736 HBM bytes per point and RHS).  The conserved variables, the
+ * gradient sweeps, the stress tensor and the heat flux stored in FP32 (572
+ * instead of 704 HBM bytes per point and RHS).  The conserved variables, the
  * partial RHS, closure and seam rows, characteristic BCs and the RK
  * accumulation stay FP64, and every sweep computes in FP64.  No effect on
  * inviscid solvers. */
