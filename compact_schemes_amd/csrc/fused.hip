@@ -8,9 +8,10 @@
 // Here each sweep reads its inputs once, differentiates several fields along
 // one axis and writes only what the next sweep needs:
 //   S1x, S1y: q -> (u, v, w, c^2) -> d/dx, d/dy                      (4 fields out)
-//   S1z:      q, x/y gradients -> d/dz -> stress (6) + heat flux (3)
-//   S2x:      q, stress row x, heat x -> F^x (5) -> dF/dx            (partial RHS)
-//   S2y, S2z: ... + previous partial RHS; S2z adds the RK stage update
+//   S1z:      q, x/y gradients of u, v, w -> d/dz -> stress (6) + heat flux along z
+//   S2x:      q, stress row x, c^2 gradient along x -> F^x (5) -> dF/dx  (partial RHS)
+//   S2y, S2z: ... + previous partial RHS; S2z takes the heat flux and adds the RK stage update
+// (cs_solver_set_order 0; the default order closes along x: gradients y, z, x, fluxes z, y, x)
 // and every S2 sweep applies the non-reflective characteristic update of its
 // two faces from the boundary values of its own solve (the reference's drva).
 //

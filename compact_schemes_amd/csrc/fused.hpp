@@ -31,8 +31,8 @@ struct AxisDesc {
     int seam;            // both faces seam (periodic wrap on one subdomain)
     int gcbc;            // both faces non-reflective characteristic BCs
     // kernel variant (chosen per axis, see cs_solver_tune):
-    int variant;         // 0: direct (ragged when N != P*K); 1: LDS row-block tiles; 2: direct, 16-point chunks
-    int tl;              // lines per workgroup (y/z lines of variant 0, all of variant 1): 8 or 16
+    int variant;         // 0: direct; 1: LDS row-block tiles; 2: direct, 16-point chunks
+    int tl;              // lines per workgroup (y/z lines of variant 0, all of variant 1): 8 or 16 (block_lines)
     int xcd;             // 1: neighbouring line groups go to workgroups on the same XCD
     // filter sweep along this axis: 1 = one field per workgroup (grid.y over
     // the five fields), 5 = all five fields per workgroup; lines per workgroup

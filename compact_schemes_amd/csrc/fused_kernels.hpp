@@ -988,7 +988,8 @@ direct_kernel(AxisDesc ax, SweepCommon cm, SW sw, BATCH batch) {
 //
 // Two waves a SIMD, each with its 8 points' loads in flight; at 256^3 the
 // sweeps run at the rate of a plain stream of the same fields (5.6 TB/s): S1x
-// 556 -> 520 us, filter 392 -> 240 us, S2x 606 -> 548 us in a step.  What held
+// 556 -> 520 us (430 with its 144 bytes a point), filter 392 -> 240 us, S2x 606
+// -> 548 us in a step.  What held
 // them back were instructions, not bytes (the filter: 4150 a wave, 2000 now):
 // branches around every point, closure rows tested row by row, seam rows read
 // again from memory, scans over the whole line.
