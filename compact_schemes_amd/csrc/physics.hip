@@ -14,6 +14,23 @@ namespace cs {
 
 constexpr int kBlock = 256;
 
+// with the streaming hint where NT
+template <bool NT>
+__device__ __forceinline__ double ld(const double* p) {
+    if constexpr (NT) return __builtin_nontemporal_load(p);
+    else return *p;
+}
+template <bool NT>
+__device__ __forceinline__ void st(double* p, double v) {
+    if constexpr (NT) __builtin_nontemporal_store(v, p);
+    else *p = v;
+}
+// The hint pays where a kernel passes over more than the last-level cache
+// holds (160x128x96, 42 fields: fluxes_pre 120 -> 108 us, visc 108 -> 91);
+// below, the next kernel finds there what this one wrote (96x80x64: the
+// step 798 us without the hint there, 808 with it).
+static bool streams(int nfields, long lmx) { return 8.0 * nfields * (double)lmx > 256.0 * (1 << 20); }
+
 static dim3 grid_for(long n) { return dim3((unsigned)((n + kBlock - 1) / kBlock)); }
 
 // primitive variables (absent upstream): de0 = 1/rho, de1..3 = u, v, w,
@@ -35,7 +52,7 @@ __global__ void __launch_bounds__(kBlock) primitives_kernel(const double* qa, do
 // calc_fluxes_pre_compute_kernel, src/cuda/kernels/physics.hpp:42-193
 // (D21 intended: stress/heat are not read when Visc is false; the E + p it
 // leaves in de is overwritten by the flux divergence and not written here).
-template <bool Visc>
+template <bool Visc, bool NT>
 __global__ void __launch_bounds__(kBlock) fluxes_pre_kernel(double* buffer, const double* qa, const double* pr,
                                                             const double* de, const double* xim, const double* etm,
                                                             const double* zem, const double* stress,
@@ -43,30 +60,33 @@ __global__ void __launch_bounds__(kBlock) fluxes_pre_kernel(double* buffer, cons
     long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= lmx) return;
     double q[5], u[3], mt[3][3], tau[6] = {0, 0, 0, 0, 0, 0}, hf[3] = {0, 0, 0};
-    load_q(qa, t, lmx, q);
-    u[0] = de[t + lmx]; u[1] = de[t + 2 * lmx]; u[2] = de[t + 3 * lmx];
+    for (int v = 0; v < 5; v++) q[v] = ld<NT>(qa + t + v * lmx);
+    for (int d = 0; d < 3; d++) u[d] = ld<NT>(de + t + (d + 1) * lmx);
     for (int d = 0; d < 3; d++) {
-        mt[0][d] = xim[t + d * lmx]; mt[1][d] = etm[t + d * lmx]; mt[2][d] = zem[t + d * lmx];
+        mt[0][d] = ld<NT>(xim + t + d * lmx);
+        mt[1][d] = ld<NT>(etm + t + d * lmx);
+        mt[2][d] = ld<NT>(zem + t + d * lmx);
     }
     if (Visc) {
-        for (int k = 0; k < 6; k++) tau[k] = stress[t + k * lmx];
-        for (int k = 0; k < 3; k++) hf[k] = heat[t + k * lmx];
+        for (int k = 0; k < 6; k++) tau[k] = ld<NT>(stress + t + k * lmx);
+        for (int k = 0; k < 3; k++) hf[k] = ld<NT>(heat + t + k * lmx);
     }
     double F[5][3];
-    flux_all<Visc>(q, pr[t], u, mt, tau, hf, umf, F);
+    flux_all<Visc>(q, ld<NT>(pr + t), u, mt, tau, hf, umf, F);
     for (int m = 0; m < 5; m++)
-        for (int j = 0; j < 3; j++) buffer[t + (long)j * lmx + (long)m * 3 * lmx] = F[m][j];
+        for (int j = 0; j < 3; j++) st<NT>(buffer + t + (long)(3 * m + j) * lmx, F[m][j]);
 }
 
 // calc_fluxes_post_compute_kernel<m>, src/cuda/kernels/physics.hpp:195-209,
 // for all five variables
+template <bool NT>
 __global__ void __launch_bounds__(kBlock) fluxes_post_kernel(double* de, const double* bd, long lmx) {
     long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= lmx) return;
     double d[kNV][3];
     for (int m = 0; m < kNV; m++)
-        for (int j = 0; j < 3; j++) d[m][j] = bd[t + (long)(3 * m + j) * lmx];
-    for (int m = 0; m < kNV; m++) de[t + (long)m * lmx] = d[m][0] + d[m][1] + d[m][2];
+        for (int j = 0; j < 3; j++) d[m][j] = ld<NT>(bd + t + (long)(3 * m + j) * lmx);
+    for (int m = 0; m < kNV; m++) st<NT>(de + t + (long)m * lmx, d[m][0] + d[m][1] + d[m][2]);
 }
 
 // calc_viscous_shear_stress_post_compute_kernel<m> (m = 1..4) and
@@ -76,7 +96,8 @@ __global__ void __launch_bounds__(kBlock) fluxes_post_kernel(double* de, const d
 // flux.  The reference passes the twelve gradients through the stress and
 // heat arrays (five kernels, 84 fields read or written); in registers the
 // 26 reads and 11 writes are left, and they are the bound (160x128x96: five
-// kernels 229 us, this one 108 = 5.4 TB/s).
+// kernels 229 us, this one 91 = 6.4 TB/s).
+template <bool NT>
 __global__ void __launch_bounds__(kBlock) visc_kernel(double* de, const double* ssk, const double* yaco,
                                                       const double* bd, const double* xim, const double* etm,
                                                       const double* zem, double* stress, double* heat, long lmx) {
@@ -84,21 +105,23 @@ __global__ void __launch_bounds__(kBlock) visc_kernel(double* de, const double* 
     if (t >= lmx) return;
     double mt[3][3], f[4][3], u[3];
     for (int d = 0; d < 3; d++) {
-        mt[0][d] = xim[t + d * lmx]; mt[1][d] = etm[t + d * lmx]; mt[2][d] = zem[t + d * lmx];
-        u[d] = de[t + (d + 1) * lmx];
+        mt[0][d] = ld<NT>(xim + t + d * lmx);
+        mt[1][d] = ld<NT>(etm + t + d * lmx);
+        mt[2][d] = ld<NT>(zem + t + d * lmx);
+        u[d] = ld<NT>(de + t + (d + 1) * lmx);
     }
     for (int m = 0; m < 4; m++)
-        for (int j = 0; j < 3; j++) f[m][j] = bd[t + (long)(3 * (m + 1) + j) * lmx];
-    const double mu = ssk[t], J = yaco[t];
+        for (int j = 0; j < 3; j++) f[m][j] = ld<NT>(bd + t + (long)(3 * (m + 1) + j) * lmx);
+    const double mu = ld<NT>(ssk + t), J = ld<NT>(yaco + t);
     double g[12];   // (u_x, u_y, u_z, v_x, v_y, v_z, w_x, w_y, w_z, c2_x, c2_y, c2_z)
     for (int m = 0; m < 4; m++)
         for (int d = 0; d < 3; d++) g[3 * m + d] = mt[0][d] * f[m][0] + mt[1][d] * f[m][1] + mt[2][d] * f[m][2];
     double tau[6], hf[3], d4;
     viscous_closure(mu, J, g, g + 9, u, tau, hf, &d4);
-    de[t] = mu;
-    de[t + 4 * lmx] = d4;
-    for (int k = 0; k < 6; k++) stress[t + k * lmx] = tau[k];
-    for (int k = 0; k < 3; k++) heat[t + k * lmx] = hf[k];
+    st<NT>(de + t, mu);
+    st<NT>(de + t + 4 * lmx, d4);
+    for (int k = 0; k < 6; k++) st<NT>(stress + t + k * lmx, tau[k]);
+    for (int k = 0; k < 3; k++) st<NT>(heat + t + k * lmx, hf[k]);
 }
 
 // calc_time_step_kernel, src/cuda/kernels/physics.hpp:335-427 (D9 intended:
@@ -227,25 +250,25 @@ int launch_primitives(const double* qa, double* de, double* p, long lmx, hipStre
 int launch_fluxes_pre(bool visc, double* buffer, const double* qa, const double* p, const double* de,
                       const double* xim, const double* etm, const double* zem, const double* stress,
                       const double* heat, cs_point umf, long lmx, hipStream_t s) {
-    if (visc)
-        hipLaunchKernelGGL(fluxes_pre_kernel<true>, grid_for(lmx), dim3(kBlock), 0, s, buffer, qa, p, de, xim, etm,
-                           zem, stress, heat, umf, lmx);
-    else
-        hipLaunchKernelGGL(fluxes_pre_kernel<false>, grid_for(lmx), dim3(kBlock), 0, s, buffer, qa, p, de, xim,
-                           etm, zem, stress, heat, umf, lmx);
+    const bool nt = streams(visc ? 42 : 33, lmx);
+    auto k = visc ? (nt ? fluxes_pre_kernel<true, true> : fluxes_pre_kernel<true, false>)
+                  : (nt ? fluxes_pre_kernel<false, true> : fluxes_pre_kernel<false, false>);
+    hipLaunchKernelGGL(k, grid_for(lmx), dim3(kBlock), 0, s, buffer, qa, p, de, xim, etm, zem, stress, heat, umf, lmx);
     CS_HIP(hipGetLastError());
     return CS_OK;
 }
 
 int launch_fluxes_post(double* de, const double* bd, long lmx, hipStream_t s) {
-    hipLaunchKernelGGL(fluxes_post_kernel, grid_for(lmx), dim3(kBlock), 0, s, de, bd, lmx);
+    auto k = streams(20, lmx) ? fluxes_post_kernel<true> : fluxes_post_kernel<false>;
+    hipLaunchKernelGGL(k, grid_for(lmx), dim3(kBlock), 0, s, de, bd, lmx);
     CS_HIP(hipGetLastError());
     return CS_OK;
 }
 
 int launch_visc(double* de, const double* ssk, const double* yaco, const double* bd, const double* xim,
                 const double* etm, const double* zem, double* stress, double* heat, long lmx, hipStream_t s) {
-    hipLaunchKernelGGL(visc_kernel, grid_for(lmx), dim3(kBlock), 0, s, de, ssk, yaco, bd, xim, etm, zem, stress, heat,
+    auto k = streams(37, lmx) ? visc_kernel<true> : visc_kernel<false>;
+    hipLaunchKernelGGL(k, grid_for(lmx), dim3(kBlock), 0, s, de, ssk, yaco, bd, xim, etm, zem, stress, heat,
                        lmx);
     CS_HIP(hipGetLastError());
     return CS_OK;
