@@ -13,8 +13,10 @@ constexpr int kMaxP = 32;     // chunks per line
 
 // First row of chunk c (N for c = P) of a line of N rows in P = ceil(N/K)
 // chunks: K rows a chunk, K-1 in the D = P*K - N chunks after the first; lines
-// too short for that (chunks_fit) are balanced, at least 4 rows a chunk.
-__host__ __device__ inline bool chunks_fit(int N, int P, int K) { return P * K - N <= (P > 2 ? P - 2 : 0); }
+// too short for that (chunks_fit) are balanced, at least 4 rows a chunk.  The
+// first and the last chunk are two: a sweep kernel's chunk forms the rows of
+// one line end only, so a line that is one chunk runs the general kernels.
+__host__ __device__ inline bool chunks_fit(int N, int P, int K) { return P > 1 && P * K - N <= P - 2; }
 __host__ __device__ inline int chunk_start(int N, int P, int K, int c) {
     if (!chunks_fit(N, P, K)) return (int)(((long)c * N) / P);
     const int D = P * K - N, d = c < 1 ? 0 : c - 1;
