@@ -901,7 +901,7 @@ direct_kernel(AxisDesc ax, SweepCommon cm, SW sw, BATCH batch) {
             sw.dtpart[2 * blockIdx.x + 1] = a1;
         }
     }
-    fold_forward<NF, K, SW::kFilter>(lds, tab, NP, P, TL, c, lloc, G);
+    fold_forward<NF, K>(lds, tab, NP, P, TL, c, lloc, G);
     apply_carry<K, NF>(tab, 3 * NP, s, r, G);
     if constexpr (!EX) zero_padding<K, NF>(r, whole);
     backward_local<K, NF>(tab, NP, s, r, carry);
@@ -909,7 +909,7 @@ direct_kernel(AxisDesc ax, SweepCommon cm, SW sw, BATCH batch) {
 #pragma unroll
     for (int f = 0; f < NF; f++) xb[(f * P + c) * TL + lloc] = carry[f];
     __syncthreads();
-    fold_backward<NF, K, SW::kFilter>(xb, tab, NP, P, TL, c, lloc, X);
+    fold_backward<NF, K>(xb, tab, NP, P, TL, c, lloc, X);
     apply_carry<K, NF>(tab, 4 * NP, s, r, X);
     if (cyc) {
         // rows 0 and N-1 of the modified system through LDS (after the folds' reads)
@@ -1117,14 +1117,13 @@ xt_kernel(AxisDesc ax, SweepCommon cm, SW sw, BATCH batch) {
         }
     }
 
-    constexpr int kReach = SW::kFilter ? 64 : 64 / K;    // chunks (kCarryRows, rounded up to a power of two)
     double carry[NF], G[NF], X[NF];
     forward_local<K, NF>(tab, NP, s, r, carry);
-    scan_forward<NF>(tab[3 * NP + s + K - 1], carry, c, P, kReach, G);
+    scan_forward<NF>(tab[3 * NP + s + K - 1], carry, c, P, G);
     apply_carry<K, NF>(tab, 3 * NP, s, r, G);
     if constexpr (!EX) zero_padding<K, NF>(r, whole);
     backward_local<K, NF>(tab, NP, s, r, carry);
-    scan_backward<NF>(tab[4 * NP + s], carry, c, P, kReach, X);
+    scan_backward<NF>(tab[4 * NP + s], carry, c, P, X);
     apply_carry<K, NF>(tab, 4 * NP, s, r, X);
     if (cyc) {
         double y0[NF], yN1[NF];
@@ -1283,7 +1282,7 @@ __global__ void __launch_bounds__(TL * kMaxP) tile_kernel(AxisDesc ax, SweepComm
 #pragma unroll
     for (int f = 0; f < NF; f++) lds[(f * P + c) * TL + lloc] = carry[f];
     __syncthreads();
-    fold_forward<NF, K, false>(lds, tab, NP, P, TL, c, lloc, G);
+    fold_forward<NF, K>(lds, tab, NP, P, TL, c, lloc, G);
     apply_carry<K, NF>(tab, 3 * NP, c * K, r, G);
 #pragma unroll
     for (int t = 1; t < K; t++)
@@ -1294,7 +1293,7 @@ __global__ void __launch_bounds__(TL * kMaxP) tile_kernel(AxisDesc ax, SweepComm
 #pragma unroll
     for (int f = 0; f < NF; f++) xb[(f * P + c) * TL + lloc] = carry[f];
     __syncthreads();
-    fold_backward<NF, K, false>(xb, tab, NP, P, TL, c, lloc, X);
+    fold_backward<NF, K>(xb, tab, NP, P, TL, c, lloc, X);
     apply_carry<K, NF>(tab, 4 * NP, c * K, r, X);
 
     if constexpr (GCBC) {

@@ -144,34 +144,33 @@ __device__ __forceinline__ void apply_carry(const double* tab, int off, int s, d
     }
 }
 
-// How many chunks away a carry of the derivative's solve still counts: the
-// interior LU factors of alpha = 1/3 shrink it by (3 - sqrt 5)/2 = 0.382 a row,
-// so after 48 rows it is below 1e-20 of its size, under the last bit of any
-// row it is added to.  The filter's factors (0.82 a row at alpha_f = 0.49)
-// reach across the whole line.
-constexpr int kCarryRows = 48;
-template <int K, bool FILTER>
-__device__ __forceinline__ int carry_reach(int P) { return FILTER ? P : kCarryRows / K; }
+// Every chunk of a line counts in a carry: a row reaches every other of its
+// line, by a factor of (3 - sqrt 5)/2 = 0.382 a row along a derivative, 0.82
+// along a filter at alpha_f = 0.49, and a NaN or an infinity whole.  Folding a
+// derivative's carries over the nearest 48 rows alone loses that for 1.6 % of
+// a step at 256^3 (10.27 against 10.11 ms) and 2.9 % at 150x133x97 (1.72
+// against 1.67).  kCarryRows is the longest line of the sweep kernels.
+constexpr int kCarryRows = 1024;
 
 // carries across the chunks of a line through LDS: buf = [NF][P][TL]
-template <int NF, int K, bool FILTER>
+template <int NF, int K>
 __device__ __forceinline__ void fold_forward(const double* buf, const double* tab, int NP, int P, int TL, int c,
                                              int lloc, double (&G)[NF]) {
 #pragma unroll
     for (int f = 0; f < NF; f++) G[f] = 0.0;
-    for (int cc = max(0, c - carry_reach<K, FILTER>(P)); cc < c; cc++) {
+    for (int cc = 0; cc < c; cc++) {
         const double M = tab[3 * NP + cc * K + K - 1];
 #pragma unroll
         for (int f = 0; f < NF; f++) G[f] = __builtin_fma(M, G[f], buf[(f * P + cc) * TL + lloc]);
     }
 }
 
-template <int NF, int K, bool FILTER>
+template <int NF, int K>
 __device__ __forceinline__ void fold_backward(const double* buf, const double* tab, int NP, int P, int TL, int c,
                                               int lloc, double (&X)[NF]) {
 #pragma unroll
     for (int f = 0; f < NF; f++) X[f] = 0.0;
-    for (int cc = min(P - 1, c + carry_reach<K, FILTER>(P)); cc > c; cc--) {
+    for (int cc = P - 1; cc > c; cc--) {
         const double R = tab[4 * NP + cc * K];
 #pragma unroll
         for (int f = 0; f < NF; f++) X[f] = __builtin_fma(R, X[f], buf[(f * P + cc) * TL + lloc]);
@@ -180,14 +179,13 @@ __device__ __forceinline__ void fold_backward(const double* buf, const double* t
 
 // carries across the chunks of a line held by P consecutive lanes of a wave
 // (c = lane's chunk): segmented Kogge-Stone scans of the affine maps
-// x -> A*x + B over the `reach` nearest chunks (a power of two, or >= P)
+// x -> A*x + B
 template <int NF>
-__device__ __forceinline__ void scan_forward(double A, const double (&carry)[NF], int c, int P, int reach,
-                                             double (&G)[NF]) {
+__device__ __forceinline__ void scan_forward(double A, const double (&carry)[NF], int c, int P, double (&G)[NF]) {
     double B[NF];
 #pragma unroll
     for (int f = 0; f < NF; f++) B[f] = carry[f];
-    for (int d = 1; d < min(P, reach); d <<= 1) {
+    for (int d = 1; d < P; d <<= 1) {
         const double Au = __shfl_up(A, d);
         double Bu[NF];
 #pragma unroll
@@ -206,12 +204,11 @@ __device__ __forceinline__ void scan_forward(double A, const double (&carry)[NF]
 }
 
 template <int NF>
-__device__ __forceinline__ void scan_backward(double A, const double (&carry)[NF], int c, int P, int reach,
-                                              double (&X)[NF]) {
+__device__ __forceinline__ void scan_backward(double A, const double (&carry)[NF], int c, int P, double (&X)[NF]) {
     double B[NF];
 #pragma unroll
     for (int f = 0; f < NF; f++) B[f] = carry[f];
-    for (int d = 1; d < min(P, reach); d <<= 1) {
+    for (int d = 1; d < P; d <<= 1) {
         const double Ad = __shfl_down(A, d);
         double Bd[NF];
 #pragma unroll

@@ -384,14 +384,13 @@ xtT_kernel(AxisDesc ax, SweepCommon cm, SW sw) {
         }
     }
 
-    constexpr int kReach = SW::kFilter ? 64 : 8;        // chunks (kCarryRows, rounded up to a power of two)
     double carry[NF], G[NF], X[NF];
     forward_local<K, NF>(tab, NP, s, r, carry);
-    scan_forward<NF>(tab[3 * NP + s + K - 1], carry, c, P, kReach, G);
+    scan_forward<NF>(tab[3 * NP + s + K - 1], carry, c, P, G);
     apply_carry<K, NF>(tab, 3 * NP, s, r, G);
     if constexpr (!EX) zero_padding<K, NF>(r, whole);
     backward_local<K, NF>(tab, NP, s, r, carry);
-    scan_backward<NF>(tab[4 * NP + s], carry, c, P, kReach, X);
+    scan_backward<NF>(tab[4 * NP + s], carry, c, P, X);
     apply_carry<K, NF>(tab, 4 * NP, s, r, X);
 
     const bool wrap = !SW::kFilter && ax.seam;
@@ -519,7 +518,7 @@ directT_kernel(AxisDesc ax, SweepCommon cm, SW sw) {
 #pragma unroll
     for (int f = 0; f < NF; f++) lds[(f * P + c) * TL + lloc] = carry[f];
     __syncthreads();
-    fold_forward<NF, K, SW::kFilter>(lds, tab, NP, P, TL, c, lloc, G);
+    fold_forward<NF, K>(lds, tab, NP, P, TL, c, lloc, G);
     apply_carry<K, NF>(tab, 3 * NP, s, r, G);
     if constexpr (!EX) zero_padding<K, NF>(r, whole);
     backward_local<K, NF>(tab, NP, s, r, carry);
@@ -527,7 +526,7 @@ directT_kernel(AxisDesc ax, SweepCommon cm, SW sw) {
 #pragma unroll
     for (int f = 0; f < NF; f++) xb[(f * P + c) * TL + lloc] = carry[f];
     __syncthreads();
-    fold_backward<NF, K, SW::kFilter>(xb, tab, NP, P, TL, c, lloc, X);
+    fold_backward<NF, K>(xb, tab, NP, P, TL, c, lloc, X);
     apply_carry<K, NF>(tab, 4 * NP, s, r, X);
 
     // halo rows hb[(f*2H + k)*P + c][TL]: k < H the first H rows of chunk c,
