@@ -179,7 +179,7 @@ int one_sweep(cs_solver* sv, int which, const double* q, const double* sbcc, dou
     if (which < 0 || which > 10) return fail(CS_ERR_ARG, "sweep index out of 0..10");
     if (which >= 7) {
         for (int a = 0; a < 3; a++)
-            if ((which == 7 || which - 8 == a) && !filter_axis_tunable(sv, a))
+            if ((which == 7 || which - 8 == a) && !filter_axis_equal(sv, a))
                 return fail(CS_ERR_UNSUPPORTED, "this axis does not split into equal chunks");
         if (out != q) CS_HIP(hipMemcpyAsync(out, q, sizeof(double) * 5 * sv->g.lmx, hipMemcpyDeviceToDevice, s));
         return filter_sweeps(sv, out, s, which == 7 ? -1 : which - 8);
@@ -191,7 +191,7 @@ int one_sweep(cs_solver* sv, int which, const double* q, const double* sbcc, dou
 
 bool filter_axis_fused(const cs_solver* sv, int a) { return sv->fax[a].ftab != nullptr; }
 
-bool filter_axis_tunable(const cs_solver* sv, int a) {
+bool filter_axis_equal(const cs_solver* sv, int a) {
     return filter_axis_fused(sv, a) && sv->ax[a].N == sv->ax[a].P * sv->ax[a].K;
 }
 

@@ -139,8 +139,8 @@ int one_sweep(cs_solver* sv, int which, const double* q, const double* sbcc, dou
 void chunk_table(const std::vector<double>& h, int n, int K, int P, std::vector<double>& out);
 // the filter along axis a runs a fused sweep (fax), else the line solver
 bool filter_axis_fused(const cs_solver* sv, int a);
-// that sweep runs equal chunks and takes the shapes of cs_solver_tune_filter
-bool filter_axis_tunable(const cs_solver* sv, int a);
+// that sweep runs equal chunks (the single filter sweeps of cs_solver_sweep)
+bool filter_axis_equal(const cs_solver* sv, int a);
 int filter_sweeps(cs_solver* sv, double* q, hipStream_t s, int axis = -1);
 int step_filter(cs_solver* sv, double* qa, hipStream_t s);
 // adjoint (vjp.hip: per-operator products; tape.hip: fused transposed sweeps)

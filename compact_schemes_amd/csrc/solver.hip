@@ -130,17 +130,14 @@ int cs_solver_destroy(cs_solver* sv) {
     return CS_OK;
 }
 
-// the shapes cs_solver_tune offers on 16-point chunks: equal ones
-static int check_chunks16(const AxisDesc& ax, int axis) {
-    if (axis == 0 || ax.K != 8 || ax.N % 16 != 0 || ax.N < 32)
-        return fail(CS_ERR_UNSUPPORTED, "16-point chunks: y or z lines of 32..256 points, a multiple of 16");
-    return CS_OK;
-}
+static const char* const kNoChunks16 = "16-point chunks: y or z lines of 32..256 points that they cut at most one row short";
 
-// the right-hand-side sweeps of `axis` on 16-point chunks
+// the right-hand-side sweeps of `axis` on 16-point chunks, where they cut its
+// lines (fits16: what cs_solver_create makes the default, and what
+// cs_solver_tune, the autotuner and the cache may choose)
 static int use_chunks16(cs_solver* sv, int axis, int lines, int xcd) {
     const AxisDesc& ax = sv->ax[axis];
-    if (!fits16(ax, axis)) return fail(CS_ERR_UNSUPPORTED, "16-point chunks do not cut this line");
+    if (!fits16(ax, axis)) return fail(CS_ERR_UNSUPPORTED, kNoChunks16);
     if (!sv->tabs16[axis]) {
         const int rc = upload_table(OP_DERIV, ax.N, ax.seam, sv->cfg.alpha_f, 16, (ax.N + 15) / 16,
                                     &sv->tabs16[axis]);
@@ -157,8 +154,8 @@ static int use_chunks16(cs_solver* sv, int axis, int lines, int xcd) {
     return CS_OK;
 }
 
-// the filter sweep of `axis` (y or z) on 16-point chunks (lines of 32..256
-// points, a multiple of 16) or back on the 8-point chunks of ax
+// the filter sweep of `axis` (y or z) on 16-point chunks, where they cut its
+// lines, or back on the 8-point chunks of ax
 static int filter_chunks(cs_solver* sv, int axis, int chunk) {
     const AxisDesc& ax = sv->ax[axis];
     AxisDesc f = ax;
@@ -167,7 +164,7 @@ static int filter_chunks(cs_solver* sv, int axis, int chunk) {
     if (chunk != ax.K && (ax.K != 8 || axis == 0))
         return fail(CS_ERR_UNSUPPORTED, "this axis's filter sweep runs " + std::to_string(ax.K) + "-point chunks");
     if (chunk == 16 && ax.K == 8) {
-        if (!ax.ftab || !fits16(ax, axis)) return fail(CS_ERR_UNSUPPORTED, "16-point chunks do not cut this line");
+        if (!ax.ftab || !fits16(ax, axis)) return fail(CS_ERR_UNSUPPORTED, kNoChunks16);
         if (!sv->ftabs16[axis]) {
             const int rc = upload_table(OP_FILTER, ax.N, ax.seam, sv->cfg.alpha_f, 16, (ax.N + 15) / 16,
                                         &sv->ftabs16[axis]);
@@ -322,7 +319,7 @@ static int sweep_shape(cs_solver* sv, int axis, int variant, int lines, int xcd)
 static int filter_shape(cs_solver* sv, int axis, int fields, int lines, int chunk) {
     if ((fields != 1 && fields != 5) || (lines != 8 && lines != 16) || (chunk != 8 && chunk != 16))
         return fail(CS_ERR_ARG, "fields 1/5, lines 8/16, chunk 8/16");
-    if (!filter_axis_tunable(sv, axis)) return fail(CS_ERR_UNSUPPORTED, "this axis does not split into equal chunks");
+    if (!filter_axis_fused(sv, axis)) return fail(CS_ERR_UNSUPPORTED, "the filter of this axis has no fused sweep");
     int rc = filter_chunks(sv, axis, chunk);
     if (rc) return rc;
     sv->ax[axis].ffields = sv->fax[axis].ffields = fields;
@@ -344,19 +341,15 @@ static void apply_tuned(cs_solver* sv, bool filters) {
         ax.xcd = d[5];
         int v[3];
         if (!tuned_sweep(a, ax.N, ax.seam, sv->cfg.viscous ? sv->prec : 0, sv->curv, v) ||
-            (v[0] == 2 && check_chunks16(ax, a)) || sweep_shape(sv, a, v[0], v[1], v[2]))
+            sweep_shape(sv, a, v[0], v[1], v[2]))
             (void)sweep_shape(sv, a, d[0], d[1], d[2]);
-        if (filters && filter_axis_tunable(sv, a) && tuned_filter(a, ax.N, ax.seam, v))
+        if (filters && filter_axis_fused(sv, a) && tuned_filter(a, ax.N, ax.seam, v))
             (void)filter_shape(sv, a, v[0], v[1], v[2]);
     }
 }
 
 int cs_solver_tune(cs_solver* sv, int axis, int variant, int lines, int xcd) {
     if (!sv || axis < 0 || axis > 2) return fail(CS_ERR_ARG, "bad solver or axis");
-    if (variant == 2 && (lines == 8 || lines == 16)) {
-        const int rc = check_chunks16(sv->ax[axis], axis);
-        if (rc) return rc;
-    }
     return sweep_shape(sv, axis, variant, lines, xcd);
 }
 
@@ -418,8 +411,7 @@ int cs_solver_autotune(cs_solver* sv, const double* qa, const double* sbcc, int 
                     // grouping, the tiled one takes lines only
                     if (a == 0 && (x == 1 || (v == 0 && l == 8))) continue;
                     if (v == best[0] && l == best[1] && x == best[2]) continue;
-                    if ((v == 2 && check_chunks16(sv->ax[a], a)) || sweep_shape(sv, a, v, l, x))
-                        continue;   // not admissible on this axis
+                    if (sweep_shape(sv, a, v, l, x)) continue;   // not admissible on this axis
                     float t;
                     if ((rc = time_calls(sweeps, reps, s, ev, &t))) return rc;
                     if (t < kGain * tbest) {
@@ -434,7 +426,7 @@ int cs_solver_autotune(cs_solver* sv, const double* qa, const double* sbcc, int 
     if (!sv->cfg.filter) return CS_OK;
     CS_HIP(hipMemcpyAsync(out, qa, sizeof(double) * 5 * sv->g.lmx, hipMemcpyDeviceToDevice, s));
     for (int a = 0; a < 3; a++) {
-        if (!filter_axis_tunable(sv, a)) continue;
+        if (!filter_axis_fused(sv, a)) continue;
         auto filt = [&]() { return filter_sweeps(sv, out, s, a); };
         const AxisDesc cur = sv->fax[a];
         int best[3] = {cur.ffields, cur.ftl, cur.K};

@@ -102,7 +102,7 @@ class FusedSolver:
         # axis splits into chunks at most one row short, else a line-solver launch
         self.filter_axes = [bool(filt) and self._chunks_fit(n, 8 if (a == 0 or n <= 256) else 16)
                             for a, n in enumerate(self.dims)]
-        # the single-sweep calls (sweep 7..10, tune_filter) take equal chunks
+        # the single-sweep calls (sweep 7..10) take equal chunks
         self.filter_fused = all(f and n % (8 if (a == 0 or n <= 256) else 16) == 0
                                 for a, (f, n) in enumerate(zip(self.filter_axes, self.dims)))
 

@@ -262,8 +262,8 @@ int cs_solver_sweep(cs_solver* sv, int which, const double* qa, double* de, cons
  * src/numerics_rtc.hpp:120-126): variant 0 = each chunk thread evaluates its
  * own rows (halo rows exchanged between chunks), 1 = LDS row-block tiles
  * with coalesced loads, 2 = variant 0 on 16-point chunks (y/z lines of 32 to
- * 256 points, a multiple of 16; the default along y and z, there also on
- * lines that 16-point chunks one row short can cut); lines = 8 or 16 lines
+ * 256 points that 16-point chunks at most one row short cut; the default
+ * there); lines = 8 or 16 lines
  * per workgroup (y/z lines of variants 0 and 2, all lines of variant 1; 16 is
  * 32 along z on up to 16 chunks of 16 points);
  * xcd = 1 keeps neighbouring line groups on one XCD.  Results agree to
@@ -273,14 +273,16 @@ int cs_solver_tune(cs_solver* sv, int axis, int variant, int lines, int xcd);
  * fields = 1 filters one conserved variable per workgroup (the five variables
  * spread over the grid; default along y and z), 5 all five per workgroup
  * (default along x); lines = 8 or 16 lines per workgroup of the y/z sweeps
- * (default 16, which is 64 for one variable on lines of up to 16 chunks); chunk = 8 or 16 points per chunk thread (16: y/z lines of 32
- * to 256 points, a multiple of 16; the default there).  Results agree to
- * rounding whatever the choice. */
+ * (default 16, which is 64 for one variable on lines of up to 16 chunks);
+ * chunk = 8 or 16 points per chunk thread (16: as variant 2 of
+ * cs_solver_tune; the default there).  Results agree to rounding whatever the
+ * choice. */
 int cs_solver_tune_filter(cs_solver* sv, int axis, int fields, int lines, int chunk);
 /* launch shapes in use along axis (no reference counterpart): shape6 =
  * {variant, lines, xcd} of the right-hand-side sweeps, then {fields, lines,
  * chunk} of the fused filter sweep ({0, 0, 0} when that filter runs the line
- * solver). */
+ * solver).  cs_solver_tune and cs_solver_tune_filter take back what this
+ * reports. */
 int cs_solver_get_tune(const cs_solver* sv, int axis, int* shape6);
 /* autotuner of the fused sweeps (no reference counterpart; the reference
  * fixes its block shapes per build, src/numerics_rtc.hpp:120-126): times
