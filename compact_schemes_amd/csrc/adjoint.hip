@@ -244,20 +244,21 @@ static int adjoint_apply(cs_numerics* num, int op, int axis, const double* in, d
     LineArgs a{};
     a.in = in;
     a.out = y;
-    a.tab = t->dev;
+    const auto& g = t->gen[line_kind(axis)];
+    a.tab = g.tab;
     a.pb = num->pb;
     a.N = t->n;
     a.nlines = (int)num->g.face_size(axis);
     a.lxi = num->g.lxi;
     a.plane = (long)num->g.lxi * num->g.let;
     a.st = num->g.stride(axis);
-    a.P = t->P;
-    a.tab32 = t->dev32;
-    if ((rc = launch_line(OP_SOLVE, axis, t->K, a, s))) return rc;
+    a.P = g.P;
+    a.tab32 = g.tab32;
+    if ((rc = launch_line(OP_SOLVE, axis, g.K, a, s))) return rc;
     // out = B^T y
     double an5[6] = {};
     if (op == OP_FILTER_T) filter_coefficients(5, num->alpha_f, an5);
-    const double* T = t->dev + 9 * (size_t)t->n + 44;
+    const double* T = g.tab + 9 * (size_t)t->n + 44;
     const long lmx = num->g.lmx;
     const dim3 grid((unsigned)((lmx + 255) / 256)), block(256);
     const int lxi = num->g.lxi, let = num->g.let;

@@ -421,8 +421,9 @@ struct EventPair {
     }
 };
 
-// Times every admissible chunk length for each (operator, line length) the
-// batch holds, on one of its subdomains, and records the fastest; then
+// Times every admissible chunk length for each (operator, line length, x or
+// y/z lines) the batch holds, on one of its subdomains, and records the
+// fastest; then
 // rebuilds the batch with the choices.  The choices apply to every operator
 // table built afterwards in this process (cs_deriv / cs_filter on a new
 // context included), so batched and single-subdomain results stay identical.
@@ -433,7 +434,8 @@ int cs_batch_autotune(cs_batch* b, int reps, cs_stream stream) {
     if (!b || !b->bound) return fail(CS_ERR_STATE, "batch has no bound fields");
     if (reps < 1) reps = 3;
     hipStream_t s = (hipStream_t)stream;
-    // one case per (operator, line length, start/end rows, precision)
+    // one case per (operator, line length, start/end rows, precision) and kind
+    // of line: x lines and y/z lines run kernels of their own
     struct Case { int op, n, start, end, prec, s, axis; };
     std::vector<Case> cases;
     for (int sd = 0; sd < b->count; sd++)
@@ -443,7 +445,8 @@ int cs_batch_autotune(cs_batch* b, int reps, cs_stream stream) {
                 const Case c{op, num->g.n(axis), num->ndf[0][axis], num->ndf[1][axis], num->precision, sd, axis};
                 bool seen = false;
                 for (auto& o : cases)
-                    seen |= (o.op == c.op && o.n == c.n && o.start == c.start && o.end == c.end && o.prec == c.prec);
+                    seen |= (o.op == c.op && o.n == c.n && o.start == c.start && o.end == c.end && o.prec == c.prec &&
+                             line_kind(o.axis) == line_kind(c.axis));
                 if (!seen) cases.push_back(c);
             }
     int rc = CS_OK;
@@ -478,7 +481,7 @@ int cs_batch_autotune(cs_batch* b, int reps, cs_stream stream) {
             if (ms < best) { best = ms; bestK = K; }
         }
         if (rc) break;
-        set_tuned_chunk(c.op, c.n, c.start, c.end, c.prec, bestK);
+        set_tuned_chunk(c.op, c.n, c.start, c.end, c.prec, line_kind(c.axis), bestK);
     }
     }
     if (rc) return rc;

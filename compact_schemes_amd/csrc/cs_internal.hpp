@@ -102,21 +102,25 @@ struct LineOpKey {
     }
 };
 
+// x lines (0) and y or z lines (1) run kernels of their own, so each kind of
+// line has its own chunk lengths
+inline int line_kind(int axis) { return axis == 0 ? 0 : 1; }
+
 struct LineOpTable {
-    int n = 0, K = 0, P = 0;
-    double* dev = nullptr;     // FP64 table (build_line_table); owns the memory of the others
-    float* dev32 = nullptr;    // FP32 factorisation for the mixed-precision solve
-    // the operator on the sweep kernels (line_sweeps.hip), y/z lines and x
-    // lines: chunk length and count, chunk_table (null: general kernels)
+    int n = 0;
+    double* dev = nullptr;     // one allocation: everything below points into it
+    // per line_kind: the operator on the general kernels (line_solver.hip) --
+    // chunk length and count, FP64 table (build_line_table), FP32
+    // factorisation for the mixed-precision solve
+    struct { int K = 0, P = 0; double* tab = nullptr; float* tab32 = nullptr; } gen[2];
+    // and on the sweep kernels (line_sweeps.hip): chunk length and count,
+    // chunk_table (null: general kernels)
     struct { int K = 0, P = 0; double* chunks = nullptr; } sweep[2];
-    size_t count = 0;
 };
 
 inline void free_line_op(LineOpTable& t) {
     if (t.dev) (void)hipFree(t.dev);
-    t.sweep[0].chunks = t.sweep[1].chunks = nullptr;
-    t.dev32 = nullptr;
-    t.dev = nullptr;
+    t = LineOpTable();
 }
 
 int choose_chunk(int n, int* K, int* P);
@@ -185,8 +189,8 @@ int launch_batch_lines(int op, int K, int axis, int P, const LineArgs* args, con
 // fused right-hand-side sweep shapes per (axis, line length, seam axis,
 // precision of the intermediates, constant 0 / per-point 1 metrics), fused
 // filter shapes per (axis, line length, seam axis)
-int tuned_chunk(int op, int n, int start, int end, int prec);
-void set_tuned_chunk(int op, int n, int start, int end, int prec, int K);
+int tuned_chunk(int op, int n, int start, int end, int prec, int kind);
+void set_tuned_chunk(int op, int n, int start, int end, int prec, int kind, int K);
 bool tuned_sweep(int axis, int n, int seam, int prec, int metrics, int* variant_lines_xcd);
 void set_tuned_sweep(int axis, int n, int seam, int prec, int metrics, const int* variant_lines_xcd);
 bool tuned_filter(int axis, int n, int seam, int* fields_lines_chunk);

@@ -740,13 +740,13 @@ int launch_batch_lines(int op, int K, int axis, int P, const LineArgs* args, con
 // of 8; 256^3 derivative along y 53 against 68 us).  x lines: the length that
 // leaves fewer of a wave's 64 lanes idle (292 points: 37 of 64 with 8-point
 // chunks, 57 with 16), 8 when equal.
-static int sweep_chunk(int n, int x) {
+static int sweep_chunk(int n, int kind) {
     int best = 0, lanes = 0;
     for (int K : {8, 16}) {
         const int P = (n + K - 1) / K;
         if (n < 16 || (K == 16 && n < 32) || !fused::chunks_fit(n, P, K)) continue;
-        if (x && P <= 64 && 64 / P * P > lanes) { best = K; lanes = 64 / P * P; }
-        if (!x && P <= fused::kMaxP) best = K;
+        if (kind == 0 && P <= 64 && 64 / P * P > lanes) { best = K; lanes = 64 / P * P; }
+        if (kind == 1 && P <= fused::kMaxP) best = K;
     }
     return best;
 }
@@ -758,52 +758,71 @@ int make_line_op(const cs_numerics* num, int op, int n, int start, int end, int 
     if (n < minlen) return fail(CS_ERR_SHAPE, "line length " + std::to_string(n) + " below the stencil size");
     t->n = n;
     const bool plain = (op == OP_DERIV || op == OP_FILTER);
-    if (K == 0 && plain) K = tuned_chunk(op, n, start, end, num->precision);
-    const int tuned = K;
-    if (K != 0) {
-        if (K != 8 && K != 16 && K != 32) return fail(CS_ERR_ARG, "chunk length must be 8, 16 or 32");
-        t->K = K;
-        t->P = (n + K - 1) / K;
-        if (t->P > max_chunks(K)) return fail(CS_ERR_SHAPE, "chunk length too short for this line");
-    } else {
-        int rc = choose_chunk(n, &t->K, &t->P);
+    // one upload: the tables of the general kernels (one where both kinds of
+    // line take one chunk length), the same operator in the layout of the
+    // sweep kernels, and FP32 copies of the factorisations (nu, mu, rho, Mf,
+    // Rb, z, 1/den, kappa) for the mixed-precision solve
+    std::vector<double> h[2], hc, all;
+    size_t tab_at[2], chunks_at[2] = {0, 0}, at32[2];
+    int tuned[2];
+    for (int kind = 0; kind < 2; kind++) {
+        auto& g = t->gen[kind];
+        tuned[kind] = K == 0 && plain ? tuned_chunk(op, n, start, end, num->precision, kind) : K;
+        g.K = tuned[kind];
+        if (g.K != 0) {
+            if (g.K != 8 && g.K != 16 && g.K != 32) return fail(CS_ERR_ARG, "chunk length must be 8, 16 or 32");
+            g.P = (n + g.K - 1) / g.K;
+            if (g.P > max_chunks(g.K)) return fail(CS_ERR_SHAPE, "chunk length too short for this line");
+        } else {
+            const int rc = choose_chunk(n, &g.K, &g.P);
+            if (rc) return rc;
+        }
+        if (kind == 1 && g.K == t->gen[0].K) {
+            tab_at[1] = tab_at[0];
+            continue;
+        }
+        tab_at[kind] = all.size();
+        const int rc = plain ? build_line_table(op, n, start, end, num->alpha_f, g.K, h[kind])
+                             : build_adjoint_table(op, n, start, end, num->alpha_f, num->pb_host, g.K, h[kind]);
         if (rc) return rc;
+        all.insert(all.end(), h[kind].begin(), h[kind].end());
     }
-    std::vector<double> h;
-    int rc = (op == OP_DERIV_T || op == OP_FILTER_T)
-                 ? build_adjoint_table(op, n, start, end, num->alpha_f, num->pb_host, t->K, h)
-                 : build_line_table(op, n, start, end, num->alpha_f, t->K, h);
-    if (rc) return rc;
-    // one upload: the table, the same operator in the layout of the sweep
-    // kernels, and an FP32 copy of the factorisation (nu, mu, rho, Mf, Rb, z,
-    // 1/den, kappa) for the mixed-precision solve
-    std::vector<double> hc, all = h;
-    size_t at[2] = {0, 0};
-    for (int x = 0; x < 2 && plain && start == end; x++) {
-        auto& w = t->sweep[x];
-        w.K = tuned ? (tuned <= 16 ? tuned : 0) : sweep_chunk(n, x);
+    for (int kind = 0; kind < 2 && plain && start == end; kind++) {
+        auto& w = t->sweep[kind];
+        w.K = tuned[kind] ? (tuned[kind] <= 16 ? tuned[kind] : 0) : sweep_chunk(n, kind);
         w.P = w.K ? (n + w.K - 1) / w.K : 0;
         if (n < 16 || !w.K || !fused::chunks_fit(n, w.P, w.K)) w.K = 0;
         if (!w.K) continue;
-        at[x] = at[0];
-        if (x && w.K == t->sweep[0].K) continue;
-        at[x] = all.size();
-        fused::chunk_table(h, n, w.K, w.P, hc);
+        if (kind == 1 && w.K == t->sweep[0].K) {
+            chunks_at[1] = chunks_at[0];
+            continue;
+        }
+        chunks_at[kind] = all.size();
+        fused::chunk_table(h[0], n, w.K, w.P, hc);
         all.insert(all.end(), hc.begin(), hc.end());
     }
-    const size_t n32 = 6 * (size_t)n + 2, at32 = all.size();
-    all.resize(at32 + (n32 + 1) / 2);
-    float* h32 = reinterpret_cast<float*>(&all[at32]);
-    for (size_t i = 0; i < n32; i++) h32[i] = (float)h[i];
+    const size_t n32 = 6 * (size_t)n + 2;
+    for (int kind = 0; kind < 2; kind++) {
+        if (h[kind].empty()) {
+            at32[kind] = at32[0];
+            continue;
+        }
+        at32[kind] = all.size();
+        all.resize(at32[kind] + (n32 + 1) / 2);
+        float* h32 = reinterpret_cast<float*>(&all[at32[kind]]);
+        for (size_t i = 0; i < n32; i++) h32[i] = (float)h[kind][i];
+    }
     hipError_t e = hipMalloc(&t->dev, all.size() * sizeof(double));
     if (e == hipSuccess) e = hipMemcpy(t->dev, all.data(), all.size() * sizeof(double), hipMemcpyHostToDevice);
     if (e != hipSuccess) {
         free_line_op(*t);      // the caller keeps nothing of a failed table
         return fail(CS_ERR_HIP, std::string("operator table upload failed: ") + hipGetErrorString(e));
     }
-    for (int x = 0; x < 2; x++) t->sweep[x].chunks = at[x] ? t->dev + at[x] : nullptr;
-    t->dev32 = reinterpret_cast<float*>(t->dev + at32);
-    t->count = h.size();
+    for (int kind = 0; kind < 2; kind++) {
+        t->gen[kind].tab = t->dev + tab_at[kind];
+        t->gen[kind].tab32 = reinterpret_cast<float*>(t->dev + at32[kind]);
+        t->sweep[kind].chunks = chunks_at[kind] ? t->dev + chunks_at[kind] : nullptr;
+    }
     return CS_OK;
 }
 
@@ -821,16 +840,17 @@ int get_line_op(cs_numerics* num, int op, int axis, int start, int end, LineOpTa
 }
 
 void choose_kernel(const LineOpTable& t, int op, int axis, LineArgs* a, int* K) {
-    const auto& w = t.sweep[axis == 0 ? 1 : 0];
-    a->tab = t.dev;
-    a->tab32 = t.dev32;
+    const auto& w = t.sweep[line_kind(axis)];
+    const auto& g = t.gen[line_kind(axis)];
+    a->tab = g.tab;
+    a->tab32 = g.tab32;
     a->chunks = w.chunks;
     a->P = w.P;
     *K = w.K;
     if (line_sweep_ok(op, axis, w.K, *a)) return;
     a->chunks = nullptr;
-    a->P = t.P;
-    *K = t.K;
+    a->P = g.P;
+    *K = g.K;
 }
 
 int line_apply(cs_numerics* num, int op, int axis, const double* in, double* out, int start, int end,

@@ -6,8 +6,9 @@
 // LXI_LOCAL), i.e. per line length, boundary pair and block shape.  The
 // choices here are data: three kinds of entries, each keyed by what the
 // kernels' speed depends on.
-//   line:   (operator, line length, start/end rows, precision) -> chunk length
-//           of the per-operator and batched line kernels;
+//   line:   (operator, line length, start/end rows, precision, kind: 0 x lines,
+//           1 y and z lines) -> chunk length of the per-operator and batched
+//           line kernels;
 //   sweep:  (axis, line length, seam axis, precision of the intermediates,
 //           metrics: 0 constant per axis, 1 per point) -> kernel variant, lines
 //           per workgroup, XCD grouping of the fused right-hand-side sweeps;
@@ -16,10 +17,11 @@
 // Entries are written by the autotuners (cs_batch_autotune,
 // cs_solver_autotune) or by hand, and read when operator tables and solvers
 // are built.  File format, one entry per line ('#' starts a comment):
-//   line <op> <length> <start> <end> <precision> <K>
+//   line <op> <length> <start> <end> <precision> <K> [kind]
 //   sweep <axis> <length> <seam> <precision> <metrics> <variant> <lines> <xcd>
 //   filter <axis> <length> <seam> <fields> <lines> <chunk>
-// A line of three integers "<op> <length> <K>" (the earlier format) is a line
+// A line entry without its kind is one for both kinds; a line of three
+// integers "<op> <length> <K>" (the earlier format) is a line
 // entry for FP64 and both closure and seam ends; a sweep entry of seven
 // integers (no metrics field) is one for constant metrics.
 #include "cs_internal.hpp"
@@ -32,7 +34,7 @@ namespace cs {
 namespace {
 
 std::mutex g_lock;
-std::map<std::array<int, 5>, int> g_line;                   // op, n, start, end, prec -> K
+std::map<std::array<int, 6>, int> g_line;                   // op, n, start, end, prec, kind -> K
 std::map<std::array<int, 5>, std::array<int, 3>> g_sweep;   // axis, n, seam, prec, metrics -> variant, lines, xcd
 std::map<std::array<int, 3>, std::array<int, 3>> g_filter;  // axis, n, seam -> fields, lines, chunk
 
@@ -62,16 +64,16 @@ int check_filter(int axis, int n, int seam, int fields, int lines, int chunk) {
 
 }  // namespace
 
-int tuned_chunk(int op, int n, int start, int end, int prec) {
+int tuned_chunk(int op, int n, int start, int end, int prec, int kind) {
     std::lock_guard<std::mutex> g(g_lock);
-    auto it = g_line.find({op, n, start, end, prec});
+    auto it = g_line.find({op, n, start, end, prec, kind});
     return it == g_line.end() ? 0 : it->second;
 }
 
-void set_tuned_chunk(int op, int n, int start, int end, int prec, int K) {
+void set_tuned_chunk(int op, int n, int start, int end, int prec, int kind, int K) {
     std::lock_guard<std::mutex> g(g_lock);
-    if (K == 0) g_line.erase({op, n, start, end, prec});
-    else g_line[{op, n, start, end, prec}] = K;
+    if (K == 0) g_line.erase({op, n, start, end, prec, kind});
+    else g_line[{op, n, start, end, prec, kind}] = K;
 }
 
 bool tuned_sweep(int axis, int n, int seam, int prec, int metrics, int* v3) {
@@ -109,13 +111,14 @@ extern "C" {
 int cs_tune_set(int op, int n, int start, int end, int precision, int K) {
     const int rc = check_line(op, n, start, end, precision, K);
     if (rc) return rc;
-    set_tuned_chunk(op, n, start, end, precision, K);
+    for (int kind = 0; kind < 2; kind++) set_tuned_chunk(op, n, start, end, precision, kind, K);
     return CS_OK;
 }
 
 int cs_tune_get(int op, int n, int start, int end, int precision, int* K) {
     if (!K) return fail(CS_ERR_ARG, "null argument");
-    *K = tuned_chunk(op, n, start, end, precision);
+    *K = tuned_chunk(op, n, start, end, precision, 0);
+    if (*K == 0) *K = tuned_chunk(op, n, start, end, precision, 1);
     return CS_OK;
 }
 
@@ -160,14 +163,22 @@ int cs_tune_save(const char* path) {
     FILE* fp = std::fopen(path, "w");
     if (!fp) return fail(CS_ERR_ARG, std::string("cannot write ") + path);
     std::fprintf(fp, "# compact_schemes_amd launch-shape choices\n");
-    std::fprintf(fp, "# line <op> <length> <start> <end> <precision> <K>\n");
+    std::fprintf(fp, "# line <op> <length> <start> <end> <precision> <K> [kind]\n");
     std::fprintf(fp, "# sweep <axis> <length> <seam> <precision> <metrics> <variant> <lines> <xcd>\n");
     std::fprintf(fp, "# filter <axis> <length> <seam> <fields> <lines> <chunk>\n");
     {
         std::lock_guard<std::mutex> g(g_lock);
-        for (auto& e : g_line)
-            std::fprintf(fp, "line %d %d %d %d %d %d\n", e.first[0], e.first[1], e.first[2], e.first[3], e.first[4],
+        for (auto& e : g_line) {
+            // one entry without a kind where both kinds have the same
+            auto key = e.first;
+            key[5] = 1 - key[5];
+            const auto other = g_line.find(key);
+            const bool both = other != g_line.end() && other->second == e.second;
+            if (both && e.first[5] == 1) continue;
+            std::fprintf(fp, "line %d %d %d %d %d %d", e.first[0], e.first[1], e.first[2], e.first[3], e.first[4],
                          e.second);
+            std::fprintf(fp, both ? "\n" : " %d\n", e.first[5]);
+        }
         for (auto& e : g_sweep)
             std::fprintf(fp, "sweep %d %d %d %d %d %d %d %d\n", e.first[0], e.first[1], e.first[2], e.first[3],
                          e.first[4], e.second[0], e.second[1], e.second[2]);
@@ -195,19 +206,23 @@ int cs_tune_load(const char* path) {
         if (std::sscanf(buf, "%15s", kind) != 1) continue;      // blank line
         if (!std::strcmp(kind, "line") || !std::strcmp(kind, "sweep") || !std::strcmp(kind, "filter")) {
             const char* rest = std::strstr(buf, kind) + std::strlen(kind);
-            const bool sweep = kind[0] == 's';
+            const bool sweep = kind[0] == 's', line = kind[0] == 'l';
             k = std::sscanf(rest, "%d %d %d %d %d %d %d %d %d", &v[0], &v[1], &v[2], &v[3], &v[4], &v[5], &v[6], &v[7],
                             &v[8]);
-            if (sweep ? (k != 7 && k != 8) : k != 6) {
+            if (sweep ? (k != 7 && k != 8) : line ? (k != 6 && k != 7) : k != 6) {
                 rc = fail(CS_ERR_ARG, std::string(path) + ":" + std::to_string(lineno) + ": expected " +
-                                          (sweep ? "7 or 8" : "6") + " integers after '" + kind + "'");
+                                          (sweep ? "7 or 8" : line ? "6 or 7" : "6") + " integers after '" + kind + "'");
                 break;
             }
             if (sweep && k == 7) {   // no metrics field: constant metrics
                 for (int i = 7; i > 4; i--) v[i] = v[i - 1];
                 v[4] = 0;
             }
-            if (kind[0] == 'l') rc = cs_tune_set(v[0], v[1], v[2], v[3], v[4], v[5]);
+            if (line && k == 7) {
+                if (!(rc = check_line(v[0], v[1], v[2], v[3], v[4], v[5])) && (v[6] < 0 || v[6] > 1))
+                    rc = fail(CS_ERR_ARG, "line entry: kind 0 (x lines) or 1 (y and z lines)");
+                if (!rc) set_tuned_chunk(v[0], v[1], v[2], v[3], v[4], v[6], v[5]);
+            } else if (line) rc = cs_tune_set(v[0], v[1], v[2], v[3], v[4], v[5]);
             else if (sweep) rc = cs_tune_set_sweep(v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]);
             else rc = cs_tune_set_filter_sweep(v[0], v[1], v[2], v[3], v[4], v[5]);
         } else if (std::sscanf(buf, "%d %d %d %d", &v[0], &v[1], &v[2], &v[3]) == 3) {

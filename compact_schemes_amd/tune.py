@@ -1,8 +1,8 @@
 """The process-wide cache of launch shapes (csrc/tune.hip).
 
 Three kinds of entries, each keyed by what the kernels' speed depends on:
-line kernels (operator, line length, start/end rows, precision) -> chunk
-length; fused right-hand-side sweeps (axis, line length, seam, precision,
+line kernels (operator, line length, start/end rows, precision; x lines and
+y/z lines each) -> chunk length; fused right-hand-side sweeps (axis, line length, seam, precision,
 metrics: 0 constant, 1 per point) -> (variant, lines, xcd); fused filter
 sweeps (axis, line length, seam) -> (fields, lines, chunk).  The autotuners
 (Batch.autotune, FusedSolver.autotune) fill it; operator tables and solvers built afterwards
@@ -17,11 +17,12 @@ DERIV, FILTER = 0, 1
 
 def set_line(op, n, K, start=0, end=0, precision=0):
     """K = 8, 16 or 32 points per chunk (0 clears); start/end: 0 = closure
-    rows, 1 = seam halo rows at that end of the line."""
+    rows, 1 = seam halo rows at that end of the line.  For x and for y/z lines."""
     check(lib().cs_tune_set(int(op), int(n), int(start), int(end), int(precision), int(K)))
 
 
 def get_line(op, n, start=0, end=0, precision=0):
+    """The entry of x lines, or of y/z lines where x lines have none; 0 = none."""
     k = ctypes.c_int()
     check(lib().cs_tune_get(int(op), int(n), int(start), int(end), int(precision), ctypes.byref(k)))
     return k.value

@@ -406,8 +406,8 @@ int cs_batch_replay(cs_batch* b, cs_stream stream);
 /* work items and kernel launches of the four phases (deriv, filter x, y, z) */
 int cs_batch_info(const cs_batch* b, int* items4, int* launches4);
 /* autotuner: times the admissible chunk lengths (8, 16, 32 points) of every
- * (operator, line length, start/end rows, precision) of the batch, records
- * the fastest (cs_tune_set), rebuilds the
+ * (operator, line length, start/end rows, precision, x or y/z lines) of the
+ * batch, records the fastest in the cache of cs_tune_set, rebuilds the
  * batch and picks the fastest grid mode (cs_batch_set_persistent).  The
  * choices hold for every operator table built afterwards in
  * the process (the numerics contexts created later included), so batched and
@@ -420,7 +420,10 @@ int cs_batch_autotune(cs_batch* b, int reps, cs_stream stream);
  * batched line kernels for op (0 = derivative, 1 = filter), line length n,
  * start/end = the first/last rows of the line (0 = closure rows, 1 = seam
  * halo rows) and precision (cs_set_precision's mode); operator tables built
- * afterwards use it. */
+ * afterwards use it.  x lines and y/z lines, which run kernels of their own,
+ * have an entry each: cs_tune_set sets (or clears) both, cs_batch_autotune the
+ * one that it timed; cs_tune_get gives that of x lines, or of y/z lines where x
+ * lines have none. */
 int cs_tune_set(int op, int n, int start, int end, int precision, int K);
 int cs_tune_get(int op, int n, int start, int end, int precision, int* K);   /* K = 0: none */
 /* fused right-hand-side sweeps: shape of cs_solver_tune for (axis, line
@@ -436,11 +439,11 @@ int cs_tune_set_filter_sweep(int axis, int n, int seam, int fields, int lines, i
 int cs_tune_get_filter_sweep(int axis, int n, int seam, int* found, int* shape3);
 int cs_tune_clear(void);   /* all three kinds */
 /* persisted as text, one entry per line ('#' starts a comment):
- *   line <op> <n> <start> <end> <precision> <K>
+ *   line <op> <n> <start> <end> <precision> <K> [kind: 0 x, 1 y and z lines]
  *   sweep <axis> <n> <seam> <precision> <metrics> <variant> <lines> <xcd>
  *   filter <axis> <n> <seam> <fields> <lines> <chunk>
- * cs_tune_load adds the entries of a file to the cache; a line of three
- * integers "<op> <n> <K>" sets K for FP64 lines with closure rows at both ends
+ * cs_tune_load adds the entries of a file to the cache; a line entry without
+ * its kind is one for both kinds, a line of three integers "<op> <n> <K>" sets K for FP64 lines with closure rows at both ends
  * and with seam rows at both ends, a sweep line without the metrics field is
  * an entry for constant metrics.  A malformed or inadmissible entry stops
  * the load with CS_ERR_ARG (or CS_ERR_SHAPE) and a message naming file:line;
