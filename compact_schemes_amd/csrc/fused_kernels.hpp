@@ -66,7 +66,7 @@ struct S1T {
     static constexpr int NF = 4;
     static constexpr bool kGcbc = false;   // gradients only; BC updates act on the flux sweeps
     static constexpr bool kBlocks = false;
-    // bytes per point the sweep passes over (streaming rule of the launch)
+    // memory the sweep takes per point (streaming rule of the launch)
     static constexpr int kBytes = 40 + (int)sizeof(TS) * (CLOSE ? (CURV ? 17 : 13) : 4) + (CURV && CLOSE ? 80 : 0);
     // the transposing x kernel keeps u, v, w of its points in LDS for the
     // closure (store_pv) instead of reading q again
@@ -467,7 +467,7 @@ template <int AX>
 struct SF1 {
     static constexpr int NF = 1;
     static constexpr bool kBlocks = false;
-    static constexpr int kBytes = 40;
+    static constexpr int kBytes = 8;
     static constexpr bool kGcbc = false;
     static constexpr int kStash = 0;
     static constexpr int kH = 5;
@@ -1378,10 +1378,15 @@ inline AxisDesc with_runs(const AxisDesc& ax, long groups, bool on, int most) {
 // the 128-byte grid a line is shared by two workgroups (201x160x176: S2y 323
 // against 366 us, S1x 214 against 243).  x lines are one run of memory, of
 // which only the ends are shared; rows of 16 bytes already pay there.
+// kBytes is the memory a point of the sweep takes, a field read and written
+// once, times the fields over grid.y (five-field derivatives of the
+// per-operator right-hand side at 192^3: 1932 -> 1897 us a right-hand side
+// against counting one of them; counting the transposed filter's fields
+// twice: 160^3 adjoint 2393 -> 2414).
 template <class SW>
-static bool streams(const AxisDesc& ax, const SweepCommon& cm) {
+static bool streams(const AxisDesc& ax, const SweepCommon& cm, unsigned gy) {
     const int align = ax.st == 1 ? 2 : 16;
-    return cm.lxi % align == 0 && (double)SW::kBytes * (double)ax.N * (double)ax.nlines > 256.0 * (1 << 20);
+    return cm.lxi % align == 0 && (double)SW::kBytes * gy * (double)ax.N * (double)ax.nlines > 256.0 * (1 << 20);
 }
 
 template <int K, class SW, bool GCBC>
@@ -1452,7 +1457,7 @@ static int launch_x(const AxisDesc& ax, const SweepCommon& cm, const SW& sw, uns
     const int lpw = 64 / ax.P;
     const size_t lds = xt_lds<K, SW>(ax.P);
     const dim3 grid((unsigned)((ax.nlines + lpw - 1) / lpw), gy);
-    return launch(xt_symbol<K, SW, GCBC>(ax.N == ax.P * K, streams<SW>(ax, cm)), grid, dim3(64), lds,
+    return launch(xt_symbol<K, SW, GCBC>(ax.N == ax.P * K, streams<SW>(ax, cm, gy)), grid, dim3(64), lds,
                   with_runs(ax, grid.x, true, 64), cm, sw, s);
 }
 
@@ -1463,7 +1468,7 @@ template <int K, int AX, class SW, bool GCBC>
 static int launch_yz(const AxisDesc& ax, const SweepCommon& cm, const SW& sw, int TL, bool runs, size_t lds,
                      unsigned gy, hipStream_t s) {
     const dim3 grid((unsigned)((ax.nlines + TL - 1) / TL), gy);
-    return launch(direct_symbol<K, AX, SW, GCBC>(TL, ax.N == ax.P * K, streams<SW>(ax, cm)), grid, dim3(TL * ax.P),
+    return launch(direct_symbol<K, AX, SW, GCBC>(TL, ax.N == ax.P * K, streams<SW>(ax, cm, gy)), grid, dim3(TL * ax.P),
                   lds, with_runs(ax, grid.x, runs, (AX == 1 ? 128 : 1024) / TL), cm, sw, s);
 }
 

@@ -90,7 +90,7 @@ static int launch_one(const LineArgs& a, hipStream_t s) {
         return launch_x<K, SW, false>(ax, cm, sw, gy, s);
     } else {
         const int TL = sweep_lines(AX, ax.P);
-        const bool exact = ax.N == ax.P * K, nt = streams<SW>(ax, cm);
+        const bool exact = ax.N == ax.P * K, nt = streams<SW>(ax, cm, gy);
         const void* k = TL == 64 ? (exact ? (nt ? (const void*)direct_kernel<K, AX, 64, SW, false, true, true>
                                                 : (const void*)direct_kernel<K, AX, 64, SW, false, true, false>)
                                           : (nt ? (const void*)direct_kernel<K, AX, 64, SW, false, false, true>

@@ -80,8 +80,10 @@ struct AT {
     static constexpr int NF = 5;
     static constexpr bool kFilter = false;
     static constexpr int kWpe = 3;        // waves per SIMD of the y/z kernels (168 VGPRs)
-    // bytes a point: seed, q, result; the accumulator; lam (and the next seed)
-    static constexpr int kBytes = 120 + (MODE > 0 ? 40 : 0) + (MODE == 2 ? 80 : MODE == 3 ? 40 : 0) + (CURV ? 24 : 0);
+    // streaming rule: seed, q and the result or accumulator; lam and the next
+    // seed.  MODE 1 adds in place, so its accumulator counts once (128^3 adjoint
+    // 1216 -> 1166 us); MODE 3 counts as MODE 2 (40 less: 112^3 888 -> 896)
+    static constexpr int kBytes = 120 + (MODE > 1 ? 80 : 0) + (CURV ? 24 : 0);
     const double* q[5];       // the stage state the RHS was evaluated at
     const double* t[5];       // seed
     const double* gin[5];
@@ -168,7 +170,7 @@ struct FT {
     static constexpr int NF = NFV;
     static constexpr bool kFilter = true;
     static constexpr int kWpe = 4;
-    static constexpr int kBytes = 16 * NFV;
+    static constexpr int kBytes = 8 * NFV;      // in place
     double* q;
     long lmx;
     const double* an;         // the filter's coefficient sets (filter_bt)
@@ -666,7 +668,7 @@ template <int K, int AX, class SW>
 int launch_k(const AxisDesc& ax, const SweepCommon& cm, const SW& sw, hipStream_t s) {
     constexpr int NF = SW::NF, H = SW::kFilter ? 5 : 2;
     const unsigned gy = NF == 1 ? 5u : 1u;
-    const bool exact = ax.N == ax.P * K, nt = streams<SW>(ax, cm);
+    const bool exact = ax.N == ax.P * K, nt = streams<SW>(ax, cm, gy);
     if constexpr (AX == 0) {
         const int lpw = 64 / ax.P;
         const size_t lds = sizeof(double) * (lpw * ax.P * (K + 1) + 64);
