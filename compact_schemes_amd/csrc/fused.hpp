@@ -8,7 +8,6 @@
 namespace cs {
 namespace fused {
 
-constexpr int kYLines = 16;   // lines per workgroup of a y/z sweep
 constexpr int kMaxP = 32;     // chunks per line
 
 // First row of chunk c (N for c = P) of a line of N rows in P = ceil(N/K)

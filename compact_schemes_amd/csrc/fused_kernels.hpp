@@ -47,8 +47,6 @@ __device__ __forceinline__ void add_out(const SW& sw, uoff bo, double* d) {
     }
 }
 
-
-
 // ---------------------------------------------------------------------------
 // sweep functors
 // ---------------------------------------------------------------------------
@@ -745,14 +743,14 @@ struct NoBatch {
 // chunks through LDS.
 //
 // Bound by memory latency at the occupancy its registers allow (K = 16: 256
-// VGPRs, two 4-wave workgroups a CU): the K x NF values stay in registers from
-// the loads to the stores.  So nothing but them is live: the loads run
-// kRowsAhead rows ahead of the evaluation (all rows at once spill 500-700 B a
-// lane), a field's window exists only while its right-hand side is formed, and
-// the epilogue's loads run kRowsOut rows ahead of the additions.  Measured at 256^3 (start -> now, us; a copy of 2.1 GB runs at
-// 4.8 TB/s, the same row pattern without arithmetic at 5.3 along y and 4.7
-// along z): S1y 284 -> 216 (5.6 TB/s), S2y 550 -> 482 (5.3), S1z 309 -> 250
-// (4.8), S2z 514 -> 408 (4.6).
+// VGPRs, 8 waves a CU): the K x NF values stay in registers from the loads to
+// the stores.  So nothing but them is live: the loads run kRowsAhead rows ahead
+// of the evaluation (all rows at once spill 500-700 B a lane), a field's window
+// exists only while its right-hand side is formed, and the epilogue's loads run
+// kRowsOut rows ahead of the additions.  Measured at 256^3 (us, before -> now;
+// a copy of 2.1 GB runs at 4.8 TB/s, the same row pattern without arithmetic
+// at 5.3 along y and 4.7 along z): S1y 284 -> 220 (5.5 TB/s), S2y 550 -> 482
+// (5.3), S1z 309 -> 259 (4.7), S2z 514 -> 400 (4.7).
 // ---------------------------------------------------------------------------
 constexpr int kRowsAhead = 2;   // rows whose loads are in flight while a row is evaluated
 constexpr int kRowsOut = 4;     // rows whose epilogue loads are in flight
@@ -988,11 +986,10 @@ direct_kernel(AxisDesc ax, SweepCommon cm, SW sw, BATCH batch) {
 //
 // Two waves a SIMD, each with its 8 points' loads in flight; at 256^3 the
 // sweeps run at the rate of a plain stream of the same fields (5.6 TB/s): S1x
-// 556 -> 520 us (430 with its 144 bytes a point), filter 392 -> 240 us, S2x 606
-// -> 548 us in a step.  What held
-// them back were instructions, not bytes (the filter: 4150 a wave, 2000 now):
-// branches around every point, closure rows tested row by row, seam rows read
-// again from memory, scans over the whole line.
+// 556 -> 418 us (144 bytes a point instead of 176), filter 392 -> 237, S2x 606
+// -> 528 in a step.  What held them back were instructions, not bytes (the
+// filter: 4150 a wave, 2000 now): branches around every point, closure rows
+// tested row by row, seam rows read again from memory.
 // ---------------------------------------------------------------------------
 template <int K, class SW, bool GCBC, bool EX, bool NT, class BATCH = NoBatch>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
@@ -1400,10 +1397,12 @@ static const void* xt_symbol(bool exact, bool nt) {
 // table entries come by scalar loads and rows are 512 bytes (256^3 filter y 309 ->
 // 283, z 316 -> 292 us; 128^3 40 -> 34, 40 -> 36).  The five- and four-field
 // sweeps along z on up to 16 chunks of 16 points: 32, 256-byte rows of a plane
-// that is otherwise passed over in 128-byte pieces (256^3 S2z 442 -> 408, S1z
-// 277 -> 250 us, 128^3 S2z 45 -> 39, 48x40x32 12.0 -> 11.4); the same waves fit
-// a CU.  Along y, where 16 lines' rows lie next to the following workgroup's,
-// 32 lose (S2y 484 -> 546, S1y 218 -> 247 us).
+// that is otherwise passed over in 128-byte pieces (256^3 S2z 442 -> 415, S1z
+// 271 -> 269 us, with FP32 storage 412 -> 351, 299 -> 208; 128^3 S2z 47 -> 43,
+// S1z 28 -> 25; over lengths of 48 to 256 a right-hand side gains 1 % on
+// average, 8 % at most, and loses 1 to 3 % at 9, 10, 13 and 15 chunks, which
+// leave waves of a CU empty).  Along y, where 16 lines' rows lie next to the
+// following workgroup's, 32 lose (S2y 484 -> 546, S1y 218 -> 247 us).
 template <int K, int AX, class SW>
 static int block_lines(int P, int tl) {
     if (tl == 8) return 8;

@@ -52,9 +52,9 @@ static int upload_table(int op, int n, int seam, double af, int K, int P, double
     return CS_OK;
 }
 
-// the filter that closes an RK4 step (cfg.filter): one five-variable sweep
-// per axis when every axis splits into 8-point chunks, else the line solver
-// with the five variables in one launch per axis
+// the filter that closes an RK4 step (cfg.filter): along each axis one fused
+// sweep of the five variables where chunks at most one row short cut its lines,
+// else one launch of the line solver's kernels
 int step_filter(cs_solver* sv, double* qa, hipStream_t s) {
     if (!sv->cfg.filter) return CS_OK;
     for (int a = 0; a < 3; a++) {
@@ -241,9 +241,9 @@ int cs_solver_create(const cs_solver_config* cfg, cs_solver** out) {
     }
     for (int a = 0; a < 3; a++) sv->rax[a] = sv->fax[a] = sv->ax[a];
     // y and z lines that 16-point chunks can cut run on them: half the chunk
-    // carries and halo rows, two 4-wave workgroups a CU (256^3, 8- against
-    // 16-point chunks: S1y 262 -> 216, S2y 498 -> 482, S1z 290 -> 275, S2z 471 ->
-    // 431, filter y 376 -> 344, filter z 420 -> 371 us)
+    // carries and halo rows, 8 waves a CU (256^3, 8- against 16-point chunks:
+    // S1y 271 -> 215, S2y 487 -> 477, S1z 308 -> 268, S2z 490 -> 394, filter y
+    // 376 -> 344, filter z 420 -> 371 us)
     for (int a = 1; a < 3; a++) {
         rc = CS_OK;
         if (fits16(sv->ax[a], a)) {

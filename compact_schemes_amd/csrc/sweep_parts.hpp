@@ -82,7 +82,8 @@ __device__ __forceinline__ void dt_curv_point(const double (&M)[3][3], double J,
 
 // heat flux along an axis from the physical c^2 gradient and the axis's
 // stress row: the last lines of viscous_closure with constant metrics, the
-// same operations in the same order
+// same operations in the same order (with FP32 storage of the intermediates on
+// the stored gradient and stress; the heat flux itself is then not rounded)
 __device__ __forceinline__ double heat_flux(const Phys& ph, double c2g, double u, double v, double w, double t0,
                                             double t1, double t2) {
     const double b1 = kGamm1Prndtli * (ph.mu * ph.J);
@@ -97,10 +98,11 @@ __device__ __forceinline__ uoff line_off(int axis, uoff f, uoff lxi, uoff plane)
     return f * 8u;
 }
 
-// recurrences of the solve on the K rows of a chunk.  tab rows are chunk
-// rows: [5][P*K], rows past the line's end hold zeros (build_axis_table,
-// pad_line_table), so every chunk runs K rows; NP = P*K.  The products that
-// are fused are named, so that every kernel rounds alike.
+// recurrences of the solve on the K rows of a chunk.  tab is a chunk_table:
+// [6][P*K] rows nu, mu, rho, Mf, Rb, z by chunk row and 44 scalars; a padding
+// row has nu = 0 and mu = rho = 1, which hands the carries on, so every chunk
+// runs K rows; NP = P*K.  The products that are fused are named, so that every
+// kernel rounds alike.
 template <int K, int NF>
 __device__ __forceinline__ void forward_local(const double* tab, int NP, int s, double (&r)[NF][K],
                                               double (&carry)[NF]) {

@@ -309,8 +309,9 @@ constexpr int kPointsT = 3;     // points of a lane in the x kernel
 // (a contiguous run); coalesced loads and stores, LDS transposes field by
 // field, carries by wave scans.
 //
-// Bound by the 15 fields it reads and 10 it writes: 128^3 MODE 2 116 -> 103 us
-// (4.9 TB/s), MODE 3 95 -> 89.
+// Bound by the 20 fields it reads and 10 it writes: 128^3 MODE 2 116 -> 88 us
+// (5.7 TB/s), MODE 3 95 -> 73; what the y sweep left in the last-level cache
+// helps.
 // ---------------------------------------------------------------------------
 template <int K, class SW, bool EX, bool NT>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
@@ -466,8 +467,8 @@ xtT_kernel(AxisDesc ax, SweepCommon cm, SW sw) {
 // Bound by latency at three waves a SIMD, as the forward sweeps are.  What it
 // spent beside that were branches: one around each row's loads for the face
 // terms kept them from being in flight together, and the end chunks tested
-// every tap of the stencil (128^3: flux y 88 -> 64 us, z 70 -> 63, filter y
-// 84 -> 37, z 90 -> 44).
+// every tap of the stencil (128^3: flux y 88 -> 72 us, z 70 -> 66, filter y
+// 84 -> 32, z 90 -> 37).
 // ---------------------------------------------------------------------------
 template <int K, int AX, int TL, class SW, bool EX, bool NT>
 __global__ void __launch_bounds__(TL * kMaxP < 1024 ? TL * kMaxP : 1024)
@@ -725,9 +726,10 @@ int upload(const cs_solver* sv, int op, const AxisDesc& t, int seam, double** d)
 }
 
 // the descriptors of the transposed sweeps and the scratch.  Derivative: 8-point
-// chunks, whose 5 x 16 values of a 16-point one spill beside the epilogue's
-// loads (128^3 y, z: 64, 63 us against 68, 69).  Filter along y and z: 16-point
-// chunks where they fit, one field a workgroup (42, 50 us against 54, 60).
+// chunks: the 5 x 16 values of a 16-point one spill beside the epilogue's
+// loads (128^3 y, z, carries over 48 rows: 64, 63 us against 68, 69).  Filter
+// along y and z: 16-point chunks where they fit, one field a workgroup (128^3
+// y, z: 32, 37 us; on 8-point chunks 54, 60 with 16 lines a workgroup).
 int adjoint_setup(cs_solver* sv) {
     if (sv->adj) return CS_OK;
     int rc;
